@@ -43,14 +43,16 @@ enum SnbDoubleSlot
 #define SNB_NLC_MAXA 256
 // neighbour cells per cell of a triclinic grid (MAX_GRID_NEIGHBORS, neighbor_list.cpp:3)
 #define SNB_NL_MAX_NBR 192
-#define SNB_FFT_MAX_STAGES 16
 #define SNB_FFT_MAX_N 1024
 
+// A line transform: pass p (in order) takes the stage radices
+// (code >> 8 p) & 255 = 16 * first + second (second 1: a single stage);
+// every 2-3-5-7-smooth length up to SNB_FFT_MAX_N takes at most 5 passes.
 struct SnbFftPlan
 {
     int n;
-    int nstages;
-    int radix[SNB_FFT_MAX_STAGES];
+    int npass;
+    uint64_t code;
 };
 
 struct SnbNl

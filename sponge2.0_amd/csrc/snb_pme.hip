@@ -31,18 +31,28 @@
 int snb_fft_make_plan(int n, SnbFftPlan* plan)
 {
     if (n < 1 || n > SNB_FFT_MAX_N) return SNB_ERR_UNSUPPORTED;
-    plan->n = n;
-    plan->nstages = 0;
-    int m = n;
+    int radix[16], nstages = 0, m = n;
     const int order[5] = {4, 2, 3, 5, 7};
     for (int k = 0; k < 5; k++)
         while (m % order[k] == 0)
         {
-            if (plan->nstages >= SNB_FFT_MAX_STAGES) return SNB_ERR_UNSUPPORTED;
-            plan->radix[plan->nstages++] = order[k];
+            radix[nstages++] = order[k];
             m /= order[k];
         }
     if (m != 1) return SNB_ERR_UNSUPPORTED;
+    if (nstages == 0) radix[nstages++] = 1;
+    // neighbouring stages whose product is at most 16 share a pass (a radix-7
+    // stage stands alone: with another one it needs too many registers)
+    plan->n = n;
+    plan->npass = 0;
+    plan->code = 0;
+    for (int k = 0; k < nstages;)
+    {
+        const int a = radix[k], b = k + 1 < nstages ? radix[k + 1] : 7;
+        const bool two = b != 7 && a * b <= 16;
+        plan->code |= (uint64_t)(16 * a + (two ? b : 1)) << (8 * plan->npass++);
+        k += two ? 2 : 1;
+    }
     return SNB_OK;
 }
 
@@ -112,94 +122,247 @@ __device__ __forceinline__ void small_dft<5>(float2* v, float s)
 template <>
 __device__ __forceinline__ void small_dft<7>(float2* v, float s)
 {
-    const float C[7] = {1.0f, 0.62348980185873353f, -0.22252093395631440f,
-                        -0.90096886790241913f, -0.90096886790241913f,
-                        -0.22252093395631440f, 0.62348980185873353f};
-    const float S[7] = {0.0f, 0.78183148246802981f, 0.97492791218182361f,
-                        0.43388373911755812f, -0.43388373911755812f,
-                        -0.97492791218182361f, -0.78183148246802981f};
+    const float C[3] = {0.62348980185873353f, -0.22252093395631440f, -0.90096886790241913f};
+    const float S[3] = {0.78183148246802981f, 0.97492791218182361f, 0.43388373911755812f};
     float2 out[7];
-    for (int m = 0; m < 7; m++)
+#pragma unroll
+    for (int m = 0; m < 7; m++) out[m] = v[0];
+    // input by input: its products with the three cosines and sines once
+#pragma unroll
+    for (int r = 1; r < 7; r++)
     {
-        float2 acc = v[0];
-        for (int r = 1; r < 7; r++)
+        const float2 a = v[r];
+        float xc[3], yc[3], xs[3], ys[3];
+#pragma unroll
+        for (int h = 0; h < 3; h++)
         {
-            int q = (r * m) % 7;
-            float2 w = make_float2(C[q], s * S[q]);
-            acc = cadd(acc, cmul(v[r], w));
+            xc[h] = a.x * C[h];
+            yc[h] = a.y * C[h];
+            xs[h] = a.x * (s * S[h]);
+            ys[h] = a.y * (s * S[h]);
         }
-        out[m] = acc;
+        out[0] = cadd(out[0], a);
+#pragma unroll
+        for (int m = 1; m < 7; m++)
+        {
+            const int q = (r * m) % 7, h = q <= 3 ? q - 1 : 6 - q;
+            out[m] = cadd(out[m], q <= 3 ? make_float2(xc[h] - ys[h], xs[h] + yc[h])
+                                         : make_float2(xc[h] + ys[h], yc[h] - xs[h]));
+        }
+        // keeps the products of the next input from being formed early (registers)
+        __builtin_amdgcn_sched_barrier(0);
     }
+#pragma unroll
     for (int m = 0; m < 7; m++) v[m] = out[m];
 }
 
-// One Stockham stage for `lines` lines of length n stored contiguously
-// (stride n) in src, result in dst.  tw = e^{-2 pi i k/n} table in LDS.
-template <int R>
-__device__ void stockham_stage(const float2* src, float2* dst, int n, int lines, int ns,
-                               const float2* tw, float s)
+template <>
+__device__ __forceinline__ void small_dft<1>(float2*, float)
 {
-    const int nr = n / R;
-    const int total = lines * nr;
+}
+
+// a value that is the same in the whole wavefront, in a scalar register
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// element e of an array, the byte offset in 32 bits (scalar base + vector offset)
+template <class T>
+__device__ __forceinline__ T& at32(T* base, unsigned e)
+{
+    return *(T*)((const char*)base + e * (unsigned)sizeof(T));
+}
+
+// t / d for 0 <= t < 2^20, from rcp = v_rcp_f32(d): (t + 1/2) / d lies at
+// least 1/(2 d) from an integer, and the rounding of the reciprocal and of
+// the product moves it by less than 2.4e-7 (t + 1/2) / d.
+__device__ __forceinline__ float quick_rcp(int d) { return __builtin_amdgcn_rcpf((float)d); }
+__device__ __forceinline__ int quick_div(int t, float rcp)
+{
+    return (int)(((float)t + 0.5f) * rcp);
+}
+
+// One pass of the Stockham transforms of `lines` lines of length n: stage
+// RA (sub-transform length ns before it) and, with RB > 1, the stage RB after
+// it, RA * RB points of a line in one thread's registers.  Thread item u
+// covers the RB butterflies u + q n/(RA RB) of the first stage; their outputs
+// r are the inputs q of the second stage's butterfly with the same r, so the
+// two stages need no exchange between threads.  ld(line, i) gives element i
+// of the pass's input, st(line, i, v) takes element i of its output.  FIRST:
+// ns = 1, the first stage has no twiddles and those of the second are the
+// same for every thread (tw then points to global memory: scalar loads);
+// otherwise tw is the table e^{-2 pi i k/n} in LDS.  LF: consecutive threads
+// take consecutive lines, else consecutive items of a line.
+// Every butterfly keeps the operations of single stages in their order, so the
+// result does not depend on how stages are paired.  The line kernels are bound
+// by latency (a few workgroups a CU, each a chain of passes): pairing halves
+// the barriers and LDS round trips, and divisions by reciprocal replace the
+// integer divisions that made up most of the instructions of a single-stage
+// loop.  At 96^3, one kernel alone: z 10.0 -> 6.2 us, y 11.4 -> 6.2, x with
+// the convolution 18.2 -> 10.7, inverse plane 20.3 -> 10.6; at 216^3: z 70 ->
+// 36, y 88 -> 47, x 148 -> 57, inverse z 148 -> 90; at 28^3: 6.6 -> 5.8, 5.3
+// -> 4.1, 8.2 -> 6.2, 7.6 -> 6.2.
+template <int RA, int RB, int SIGN, bool FIRST, bool LF, class LD, class ST>
+__device__ __forceinline__ void fft_pass(int n, int lines, int ns, const float2* tw, const LD& ld,
+                                         const ST& st)
+{
+    const int nu = n / (RA * RB);
+    const int total = lines * nu;
+    const int m = FIRST ? n : n / ns;            // RA RB times the rest of the plan
+    const int step_a = m / RA, step_b = m / (RA * RB);
+    const float rl = quick_rcp(LF ? lines : nu), rn = quick_rcp(ns);
+    const float sg = (float)SIGN;
     for (int t = threadIdx.x; t < total; t += blockDim.x)
     {
-        int line = t / nr, j = t - line * nr;
-        const float2* in = src + line * n;
-        float2* out = dst + line * n;
-        int k = j % ns;
-        float2 v[R];
-#pragma unroll
-        for (int r = 0; r < R; r++) v[r] = in[j + r * nr];
-        if (ns > 1)
+        int line, u;
+        if (LF)
         {
-            int step = n / (ns * R);  // twiddle w^{r k}, w = e^{s 2 pi i/(ns R)}
+            u = quick_div(t, rl);
+            line = t - u * lines;
+        }
+        else
+        {
+            line = quick_div(t, rl);
+            u = t - line * nu;
+        }
+        const int b = FIRST ? u : quick_div(u, rn);
+        const int k = FIRST ? 0 : u - b * ns;
+        float2 v[RB][RA];
 #pragma unroll
-            for (int r = 1; r < R; r++)
+        for (int q = 0; q < RB; q++)
+#pragma unroll
+            for (int r = 0; r < RA; r++) v[q][r] = ld(line, u, (q + r * RB) * nu);
+        if (!FIRST)
+        {
+#pragma unroll
+            for (int r = 1; r < RA; r++)
             {
-                float2 w = tw[(r * k * step) % n];
-                w.y *= -s;  // table holds e^{-i..}; s = -1 keeps it, s = +1 conjugates
-                v[r] = cmul(v[r], w);
+                float2 w = tw[r * k * step_a];
+                w.y = SIGN < 0 ? w.y : -w.y;  // the table holds e^{-i..}
+#pragma unroll
+                for (int q = 0; q < RB; q++) v[q][r] = cmul(v[q][r], w);
             }
         }
-        small_dft<R>(v, s);
-        int idx = (j / ns) * ns * R + k;
 #pragma unroll
-        for (int r = 0; r < R; r++) out[idx + r * ns] = v[r];
+        for (int q = 0; q < RB; q++) small_dft<RA>(v[q], sg);
+        const int o = b * ns * (RA * RB) + k;
+#pragma unroll
+        for (int r = 0; r < RA; r++)
+        {
+            float2 z[RB];
+            z[0] = v[0][r];
+#pragma unroll
+            for (int q = 1; q < RB; q++)
+            {
+                z[q] = v[q][r];
+                if (FIRST && r == 0) continue;
+                float2 w = tw[q * (k + r * ns) * step_b];
+                w.y = SIGN < 0 ? w.y : -w.y;
+                z[q] = cmul(z[q], w);
+            }
+            small_dft<RB>(z, sg);
+#pragma unroll
+            for (int q = 0; q < RB; q++) st(line, o, (r + q * RA) * ns, z[q]);
+        }
     }
 }
 
-// Transforms `lines` contiguous lines in a (ping-pong with b); returns the
-// buffer holding the result.
-__device__ float2* fft_lines(float2* a, float2* b, const SnbFftPlan& plan, int lines,
-                             const float2* tw, float s)
+template <int SIGN, bool FIRST, bool LF, class LD, class ST>
+__device__ __forceinline__ void fft_pass_any(int radices, int n, int lines, int ns,
+                                             const float2* tw, const LD& ld, const ST& st)
 {
-    int ns = 1;
+#define SNB_FFT_PASS(A, B)                                          \
+    case (A) * 16 + (B):                                            \
+        fft_pass<A, B, SIGN, FIRST, LF>(n, lines, ns, tw, ld, st); \
+        break
+    switch (radices)
+    {
+        SNB_FFT_PASS(4, 4);
+        SNB_FFT_PASS(4, 2);
+        SNB_FFT_PASS(4, 3);
+        SNB_FFT_PASS(4, 1);
+        SNB_FFT_PASS(2, 3);
+        SNB_FFT_PASS(2, 5);
+        SNB_FFT_PASS(2, 1);
+        SNB_FFT_PASS(3, 3);
+        SNB_FFT_PASS(3, 5);
+        SNB_FFT_PASS(3, 1);
+        SNB_FFT_PASS(5, 1);
+        SNB_FFT_PASS(1, 1);
+        default: fft_pass<7, 1, SIGN, FIRST, LF>(n, lines, ns, tw, ld, st); break;
+    }
+#undef SNB_FFT_PASS
+}
+
+// The buffer that the last pass of a plan reads (the other one is free for
+// its output); a pass over LDS writes the buffer that it does not read.
+__device__ __forceinline__ float2* fft_last_src(const SnbFftPlan& plan, float2* a, float2* b)
+{
+    return plan.npass >= 2 && (plan.npass & 1) ? b : a;
+}
+
+// Transforms `lines` lines: the first pass reads through ld, the last writes
+// through st; between them the lines are in LDS, `ls` elements apart (odd, so
+// that the same element of neighbouring lines falls on different banks).  a
+// (and b for plans of three or more passes) are free on entry.  twg: twiddles
+// in global memory, tw: the same in LDS (written by this workgroup before the
+// call, no barrier needed in between).  Ends without a barrier.
+template <int SIGN, bool LF, class LD, class ST>
+__device__ __forceinline__ void fft_run(const SnbFftPlan& plan, int lines, int ls, float2* a,
+                                        float2* b, const float2* __restrict__ twg,
+                                        const float2* tw, const LD& ld, const ST& st)
+{
+    // (one value per workgroup; a batched launch loads it per context)
+    const int n = uni(plan.n), np = uni(plan.npass);
+    const uint64_t code =
+        (uint32_t)uni((int)plan.code) | (uint64_t)(uint32_t)uni((int)(plan.code >> 32)) << 32;
+    auto radices = [=](int p) { return (int)(code >> (8 * p)) & 255; };
     float2* src = a;
     float2* dst = b;
-    for (int st = 0; st < plan.nstages; st++)
+    fft_pass_any<SIGN, true, LF>(radices(0), n, lines, 1, twg, ld,
+                                 [=](int l, int i, int d, float2 v) { a[l * ls + i + d] = v; });
+    __syncthreads();
+    int ns = (radices(0) >> 4) * (radices(0) & 15);
+    for (int p = 1; p + 1 < np; p++)
     {
-        int R = plan.radix[st];
-        switch (R)
-        {
-            case 4: stockham_stage<4>(src, dst, plan.n, lines, ns, tw, s); break;
-            case 2: stockham_stage<2>(src, dst, plan.n, lines, ns, tw, s); break;
-            case 3: stockham_stage<3>(src, dst, plan.n, lines, ns, tw, s); break;
-            case 5: stockham_stage<5>(src, dst, plan.n, lines, ns, tw, s); break;
-            default: stockham_stage<7>(src, dst, plan.n, lines, ns, tw, s); break;
-        }
+        fft_pass_any<SIGN, false, LF>(
+            radices(p), n, lines, ns, tw,
+            [=](int l, int i, int d) { return src[l * ls + i + d]; },
+            [=](int l, int i, int d, float2 v) { dst[l * ls + i + d] = v; });
         __syncthreads();
-        ns *= R;
+        ns *= (radices(p) >> 4) * (radices(p) & 15);
         float2* t = src;
         src = dst;
         dst = t;
     }
-    return src;
+    if (np > 1)
+        fft_pass_any<SIGN, false, LF>(radices(np - 1), n, lines, ns, tw,
+                                      [=](int l, int i, int d) { return src[l * ls + i + d]; }, st);
+    else
+    {
+        const float rl = quick_rcp(LF ? lines : n);
+        for (int t = threadIdx.x; t < lines * n; t += blockDim.x)
+        {
+            const int q = quick_div(t, rl);
+            const int l = LF ? t - q * lines : q, i = LF ? q : t - q * n;
+            st(l, i, 0, a[l * ls + i]);
+        }
+    }
 }
 
-__device__ void load_twiddles(float2* dst, const float2* src, int n)
+__device__ __forceinline__ void load_twiddles(float2* dst, const float2* __restrict__ src, int n)
 {
     for (int k = threadIdx.x; k < n; k += blockDim.x) dst[k] = src[k];
 }
+
+// Threads of a line-pass workgroup: a pass of a two-pass plan has 100 to 300
+// items (13 or 21 lines of 96 points: 78 or 126, then 208 or 336), and small
+// workgroups find room beside the direct-space kernel; plans of three passes
+// hold two buffers (4 workgroups a CU at 216 points) and have 200 to 650
+// items a pass: twice the threads keep more wavefronts in flight there.
+#define SNB_FFT_MAX_THREADS 256
+#define SNB_FFT_WAVES 5  // per SIMD: at most 96 registers
+static inline unsigned fft_threads(const SnbFftPlan& plan) { return plan.npass > 2 ? 256 : 128; }
+// LDS line stride
+__host__ __device__ static inline int fft_ls(int n) { return n | 1; }
 
 static int lines_per_block(int n)
 {
@@ -219,25 +382,24 @@ __device__ __forceinline__ void k_fft_z_r2c_body(const float* __restrict__ real,
     unsigned bid, unsigned nbid)
 {
     extern __shared__ float2 smem[];
-    int n = plan.n;
+    const int n = plan.n, ls = fft_ls(n);
     float2* tw = smem;
     float2* a = smem + n;
-    float2* b = a + L * n;
+    float2* b = a + L * ls;
     load_twiddles(tw, twg, n);
-    int row0 = bid * L;
-    int lines = min(L, nrow - row0);
-    for (int t = threadIdx.x; t < lines * n; t += blockDim.x)
-        a[t] = make_float2(real[(size_t)row0 * n + t], 0.0f);
-    __syncthreads();
-    float2* res = fft_lines(a, b, plan, lines, tw, -1.0f);
-    for (int t = threadIdx.x; t < lines * fc; t += blockDim.x)
-    {
-        int l = t / fc, k = t - l * fc;
-        spec[(size_t)(row0 + l) * fc + k] = res[l * n + k];
-    }
+    const int row0 = uni(bid * L);
+    const int lines = uni(min(L, nrow - row0));
+    const float* in = real + (size_t)row0 * n;
+    float2* out = spec + (size_t)row0 * fc;
+    fft_run<-1, false>(
+        plan, lines, ls, a, b, twg, tw,
+        [=](int l, int i, int d) { return make_float2(at32(in + d, l * n + i), 0.0f); },
+        [=](int l, int i, int d, float2 v) {
+            if (i + d < fc) at32(out + d, l * fc + i) = v;
+        });
 }
 
-__global__ void __launch_bounds__(256) k_fft_z_r2c(const float* __restrict__ real,
+__global__ void __launch_bounds__(SNB_FFT_MAX_THREADS, SNB_FFT_WAVES) k_fft_z_r2c(const float* __restrict__ real,
                                                    float2* __restrict__ spec, int nrow,
                                                    SnbFftPlan plan, int fc,
                                                    const float2* __restrict__ twg, int L)
@@ -256,7 +418,7 @@ struct FftZr2cArgs
     int L;
 };
 
-__global__ void __launch_bounds__(256) k_fft_z_r2c_batch(SnbSegTab t)
+__global__ void __launch_bounds__(SNB_FFT_MAX_THREADS, SNB_FFT_WAVES) k_fft_z_r2c_batch(SnbSegTab t)
 {
     unsigned bid, nbid;
     const FftZr2cArgs& a = snb_seg<FftZr2cArgs>(t, bid, nbid);
@@ -271,33 +433,27 @@ __device__ __forceinline__ void k_fft_z_c2r_body(const float2* __restrict__ spec
     unsigned bid, unsigned nbid)
 {
     extern __shared__ float2 smem[];
-    int n = plan.n;
+    const int n = plan.n, ls = fft_ls(n);
     float2* tw = smem;
     float2* a = smem + n;
-    float2* b = a + L * n;
+    float2* b = a + L * ls;
     load_twiddles(tw, twg, n);
-    int row0 = bid * L;
-    int lines = min(L, nrow - row0);
-    for (int t = threadIdx.x; t < lines * n; t += blockDim.x)
-    {
-        int l = t / n, k = t - l * n;
-        float2 v;
-        if (k < fc)
-            v = spec[(size_t)(row0 + l) * fc + k];
-        else
-        {
-            v = spec[(size_t)(row0 + l) * fc + (n - k)];
-            v.y = -v.y;
-        }
-        a[t] = v;
-    }
-    __syncthreads();
-    float2* res = fft_lines(a, b, plan, lines, tw, 1.0f);
-    for (int t = threadIdx.x; t < lines * n; t += blockDim.x)
-        real[(size_t)row0 * n + t] = res[t].x;
+    const int row0 = uni(bid * L);
+    const int lines = uni(min(L, nrow - row0));
+    const float2* in = spec + (size_t)row0 * fc;
+    float* out = real + (size_t)row0 * n;
+    fft_run<1, false>(
+        plan, lines, ls, a, b, twg, tw,
+        [=](int l, int i, int d) {
+            i += d;
+            float2 v = in[l * fc + (i < fc ? i : n - i)];
+            if (i >= fc) v.y = -v.y;
+            return v;
+        },
+        [=](int l, int i, int d, float2 v) { at32(out + d, l * n + i) = v.x; });
 }
 
-__global__ void __launch_bounds__(256) k_fft_z_c2r(const float2* __restrict__ spec,
+__global__ void __launch_bounds__(SNB_FFT_MAX_THREADS, SNB_FFT_WAVES) k_fft_z_c2r(const float2* __restrict__ spec,
                                                    float* __restrict__ real, int nrow,
                                                    SnbFftPlan plan, int fc,
                                                    const float2* __restrict__ twg, int L)
@@ -316,7 +472,7 @@ struct FftZc2rArgs
     int L;
 };
 
-__global__ void __launch_bounds__(256) k_fft_z_c2r_batch(SnbSegTab t)
+__global__ void __launch_bounds__(SNB_FFT_MAX_THREADS, SNB_FFT_WAVES) k_fft_z_c2r_batch(SnbSegTab t)
 {
     unsigned bid, nbid;
     const FftZc2rArgs& a = snb_seg<FftZc2rArgs>(t, bid, nbid);
@@ -324,40 +480,34 @@ __global__ void __launch_bounds__(256) k_fft_z_c2r_batch(SnbSegTab t)
 }
 
 // y pass over spec[fx][fy][fc]: block = (x, chunk of W consecutive kz).
-__device__ __forceinline__ void k_fft_y_body(float2* __restrict__ spec, int fx, int fy,
-                                               int fc, SnbFftPlan plan,
-                                               const float2* __restrict__ twg, int W, float s,
-    unsigned bid, unsigned nbid)
+template <int SIGN>
+__device__ __forceinline__ void k_fft_y_body(float2* __restrict__ spec, int fx, int fy, int fc,
+                                             SnbFftPlan plan, const float2* __restrict__ twg,
+                                             int W, unsigned bid, unsigned nbid)
 {
     extern __shared__ float2 smem[];
-    int n = plan.n;  // == fy
+    const int n = plan.n, ls = fft_ls(n);
     float2* tw = smem;
     float2* a = smem + n;
-    float2* b = a + W * n;
+    float2* b = a + W * ls;
     load_twiddles(tw, twg, n);
-    int nchunk = (fc + W - 1) / W;
-    int x = bid / nchunk;
-    int k0 = (bid - x * nchunk) * W;
-    int w = min(W, fc - k0);
-    for (int t = threadIdx.x; t < n * w; t += blockDim.x)
-    {
-        int y = t / w, l = t - y * w;
-        a[l * n + y] = spec[((size_t)x * fy + y) * fc + k0 + l];
-    }
-    __syncthreads();
-    float2* res = fft_lines(a, b, plan, w, tw, s);
-    for (int t = threadIdx.x; t < n * w; t += blockDim.x)
-    {
-        int y = t / w, l = t - y * w;
-        spec[((size_t)x * fy + y) * fc + k0 + l] = res[l * n + y];
-    }
+    const int nchunk = (fc + W - 1) / W;
+    const int x = uni(bid / nchunk);
+    const int k0 = uni((bid - x * nchunk) * W);
+    const int w = uni(min(W, fc - k0));
+    float2* io = spec + (size_t)x * fy * fc + k0;
+    fft_run<SIGN, true>(
+        plan, w, ls, a, b, twg, tw,
+        [=](int l, int i, int d) { return at32(io + d * fc, i * fc + l); },
+        [=](int l, int i, int d, float2 v) { at32(io + d * fc, i * fc + l) = v; });
 }
 
-__global__ void __launch_bounds__(256) k_fft_y(float2* __restrict__ spec, int fx, int fy,
-                                               int fc, SnbFftPlan plan,
-                                               const float2* __restrict__ twg, int W, float s)
+template <int SIGN>
+__global__ void __launch_bounds__(SNB_FFT_MAX_THREADS, SNB_FFT_WAVES) k_fft_y(float2* __restrict__ spec, int fx,
+                                                          int fy, int fc, SnbFftPlan plan,
+                                                          const float2* __restrict__ twg, int W)
 {
-    k_fft_y_body(spec, fx, fy, fc, plan, twg, W, s, blockIdx.x, gridDim.x);
+    k_fft_y_body<SIGN>(spec, fx, fy, fc, plan, twg, W, blockIdx.x, gridDim.x);
 }
 
 struct FftYArgs
@@ -369,14 +519,14 @@ struct FftYArgs
     SnbFftPlan plan;
     const float2* twg;
     int W;
-    float s;
 };
 
-__global__ void __launch_bounds__(256) k_fft_y_batch(SnbSegTab t)
+template <int SIGN>
+__global__ void __launch_bounds__(SNB_FFT_MAX_THREADS, SNB_FFT_WAVES) k_fft_y_batch(SnbSegTab t)
 {
     unsigned bid, nbid;
     const FftYArgs& a = snb_seg<FftYArgs>(t, bid, nbid);
-    k_fft_y_body(a.spec, a.fx, a.fy, a.fc, a.plan, a.twg, a.W, a.s, bid, nbid);
+    k_fft_y_body<SIGN>(a.spec, a.fx, a.fy, a.fc, a.plan, a.twg, a.W, bid, nbid);
 }
 
 // x pass with the convolution: block = (y, chunk of W consecutive kz).
@@ -395,60 +545,58 @@ __device__ __forceinline__ void k_fft_x_conv_body(
     unsigned bid, unsigned nbid)
 {
     extern __shared__ float2 smem[];
-    int n = plan.n;  // == fx
+    const int n = plan.n, ls = fft_ls(n);
     float2* tw = smem;
     float2* a = smem + n;
-    float2* b = a + W * n;
+    float2* b = a + W * ls;
     load_twiddles(tw, twg, n);
-    int nchunk = (fc + W - 1) / W;
-    int y = bid / nchunk;
-    int k0 = (bid - y * nchunk) * W;
-    int w = min(W, fc - k0);
-    for (int t = threadIdx.x; t < n * w; t += blockDim.x)
-    {
-        int x = t / w, l = t - x * w;
-        a[l * n + x] = spec[((size_t)x * fy + y) * fc + k0 + l];
-    }
-    __syncthreads();
-    float2* res = fft_lines(a, b, plan, w, tw, -1.0f);
+    const int nchunk = (fc + W - 1) / W;
+    const int y = uni(bid / nchunk);
+    const int k0 = uni((bid - y * nchunk) * W);
+    const int w = uni(min(W, fc - k0));
+    // 32-bit offsets from a scalar base: a pass's own part i of an index is below
+    // half the length, and d * plane is scalar
+    const size_t plane = (size_t)fy * fc;
+    float2* io = spec + (size_t)y * fc + k0;
+    const float* bcl = bc + (size_t)y * fc + k0;
     double e = 0, v0 = 0, v1 = 0, v2 = 0, v3 = 0, v4 = 0, v5 = 0;
-    for (int t = threadIdx.x; t < n * w; t += blockDim.x)
-    {
-        int l = t / n, kx = t - l * n;
-        int kz = k0 + l;
-        float bcv = bc[((size_t)kx * fy + y) * fc + kz];
-        float2 f = res[t];
-        if (NEED_EV && bcv != 0.0f)
-        {
-            double a2 = (double)f.x * f.x + (double)f.y * f.y;
-            double wfull = (kz == 0 || (2 * kz == fz)) ? 1.0 : 2.0;
-            e += 0.5 * wfull * (double)bcv * a2;
-            double wref = (kz == 0 || kz == fc - 1) ? 0.5 : 1.0;
-            double kxr = kx > fx / 2 ? kx - fx : kx;
-            double kyr = y > fy / 2 ? y - fy : y;
-            double mx = kxr * r11;
-            double my = kxr * r21 + kyr * r22;
-            double mz = kxr * r31 + kyr * r32 + kz * r33;
-            double msq = mx * mx + my * my + mz * mz;
-            double cf = 2.0 / msq * (1.0 + mpre * msq);
-            double hb = wref * 0.5 * (double)bcv * a2;
-            v0 -= hb * (1.0 - cf * mx * mx);
-            v1 -= hb * (0.0 - cf * my * mx);
-            v2 -= hb * (1.0 - cf * my * my);
-            v3 -= hb * (0.0 - cf * mz * mx);
-            v4 -= hb * (0.0 - cf * mz * my);
-            v5 -= hb * (1.0 - cf * mz * mz);
-        }
-        res[t] = make_float2(f.x * bcv, f.y * bcv);
-    }
+    float2* mid = fft_last_src(plan, a, b);
+    float2* conv = mid == a ? b : a;
+    fft_run<-1, true>(
+        plan, w, ls, a, b, twg, tw,
+        [=](int l, int i, int d) { return at32(io + d * plane, (unsigned)i * plane + l); },
+        [=, &e, &v0, &v1, &v2, &v3, &v4, &v5](int l, int i, int d, float2 f) {
+            const int kz = k0 + l, kx = i + d;
+            const float bcv = at32(bcl + d * plane, (unsigned)i * plane + l);
+            if (NEED_EV && bcv != 0.0f)
+            {
+                double a2 = (double)f.x * f.x + (double)f.y * f.y;
+                double wfull = (kz == 0 || (2 * kz == fz)) ? 1.0 : 2.0;
+                e += 0.5 * wfull * (double)bcv * a2;
+                double wref = (kz == 0 || kz == fc - 1) ? 0.5 : 1.0;
+                double kxr = kx > fx / 2 ? kx - fx : kx;
+                double kyr = y > fy / 2 ? y - fy : y;
+                double mx = kxr * r11;
+                double my = kxr * r21 + kyr * r22;
+                double mz = kxr * r31 + kyr * r32 + kz * r33;
+                double msq = mx * mx + my * my + mz * mz;
+                double cf = 2.0 / msq * (1.0 + mpre * msq);
+                double hb = wref * 0.5 * (double)bcv * a2;
+                v0 -= hb * (1.0 - cf * mx * mx);
+                v1 -= hb * (0.0 - cf * my * mx);
+                v2 -= hb * (1.0 - cf * my * my);
+                v3 -= hb * (0.0 - cf * mz * mx);
+                v4 -= hb * (0.0 - cf * mz * my);
+                v5 -= hb * (1.0 - cf * mz * mz);
+            }
+            conv[l * ls + kx] = make_float2(f.x * bcv, f.y * bcv);
+        });
     __syncthreads();
-    float2* other = (res == a) ? b : a;
-    float2* res2 = fft_lines(res, other, plan, w, tw, 1.0f);
-    for (int t = threadIdx.x; t < n * w; t += blockDim.x)
-    {
-        int x = t / w, l = t - x * w;
-        spec[((size_t)x * fy + y) * fc + k0 + l] = res2[l * n + x];
-    }
+    fft_run<1, true>(
+        plan, w, ls, mid, conv, twg, tw, [=](int l, int i, int d) { return conv[l * ls + i + d]; },
+        [=](int l, int i, int d, float2 v) {
+            at32(io + d * plane, (unsigned)i * plane + l) = v;
+        });
     if (NEED_EV)
     {
         __shared__ double red[8][4];
@@ -471,7 +619,7 @@ __device__ __forceinline__ void k_fft_x_conv_body(
 }
 
 template <bool NEED_EV>
-__global__ void __launch_bounds__(256) k_fft_x_conv(
+__global__ void __launch_bounds__(SNB_FFT_MAX_THREADS, NEED_EV ? 2 : SNB_FFT_WAVES) k_fft_x_conv(
     float2* __restrict__ spec, const float* __restrict__ bc, int fx, int fy, int fz, int fc,
     SnbFftPlan plan, const float2* __restrict__ twg, int W, double r11, double r21,
     double r22, double r31, double r32, double r33, double mpre, double* __restrict__ partials)
@@ -503,7 +651,7 @@ struct FftXConvArgs
 };
 
 template <bool NEED_EV>
-__global__ void __launch_bounds__(256) k_fft_x_conv_batch(SnbSegTab t)
+__global__ void __launch_bounds__(SNB_FFT_MAX_THREADS, NEED_EV ? 2 : SNB_FFT_WAVES) k_fft_x_conv_batch(SnbSegTab t)
 {
     unsigned bid, nbid;
     const FftXConvArgs& a = snb_seg<FftXConvArgs>(t, bid, nbid);
@@ -516,11 +664,12 @@ __global__ void __launch_bounds__(256) k_fft_x_conv_batch(SnbSegTab t)
 // Fused inverse plane pass: one workgroup per x-plane does the y and z
 // transforms in LDS.  Two real z-rows travel as one complex row (row 2p as the
 // real part, row 2p+1 as the imaginary part), which halves the z work.
-// LDS: tw_z[fz] | tw_y[fy] | A[cap] | B[cap], cap = max(ceil(fy/2)*fz, fc*fy).
+// LDS: tw_z[fz] | tw_y[fy] | A[cap] | B[cap], cap = max(ceil(fy/2)*lsz, fc*lsy).
 // ---------------------------------------------------------------------------
+#define SNB_PLANE_THREADS 512
 __host__ __device__ static size_t plane_cap(int fy, int fz, int fc)
 {
-    size_t a = (size_t)((fy + 1) / 2) * fz, b = (size_t)fc * fy;
+    size_t a = (size_t)((fy + 1) / 2) * fft_ls(fz), b = (size_t)fc * fft_ls(fy);
     return a > b ? a : b;
 }
 
@@ -546,52 +695,46 @@ __device__ __forceinline__ void k_fft_plane_inv_body(const float2* __restrict__ 
     float2* B = A + cap;
     load_twiddles(twz, twzg, fz);
     load_twiddles(twy, twyg, fy);
-    const int x = bid;
-    const int np = (fy + 1) / 2;
+    const int x = uni(bid), np = (fy + 1) / 2, lsy = fft_ls(fy), lsz = fft_ls(fz);
     const float2* in = spec + (size_t)x * fy * fc;
-    for (int t = threadIdx.x; t < fy * fc; t += blockDim.x)
-    {
-        int y = t / fc, k = t - y * fc;
-        A[k * fy + y] = in[t];
-    }
+    float* plane = real + (size_t)x * fy * fz;
+    float2* mid = fft_last_src(plan_y, A, B);
+    float2* res = mid == A ? B : A;
+    fft_run<1, true>(
+        plan_y, fc, lsy, A, B, twyg, twy,
+        [=](int l, int i, int d) { return at32(in + d * fc, i * fc + l); },
+        [=](int l, int i, int d, float2 v) { res[l * lsy + i + d] = v; });
     __syncthreads();
-    float2* res = fft_lines(A, B, plan_y, fc, twy, 1.0f);
-    float2* O = (res == A) ? B : A;
     // Hermitian extension of rows 2p and 2p+1 along z, packed as Ya + i Yb.
     // The imaginary parts at kz = 0 and at the Nyquist plane are dropped,
     // which is what taking the real part of a C2R output does.
     const bool nyq = (fz % 2) == 0;
-    for (int t = threadIdx.x; t < np * fz; t += blockDim.x)
-    {
-        int p = t / fz, k = t - p * fz;
-        int kk = k < fc ? k : fz - k;
-        float2 a = res[kk * fy + 2 * p];
-        float2 b = (2 * p + 1 < fy) ? res[kk * fy + 2 * p + 1] : make_float2(0.0f, 0.0f);
-        if (k >= fc)
-        {
-            a.y = -a.y;
-            b.y = -b.y;
-        }
-        if (k == 0 || (nyq && 2 * k == fz))
-        {
-            a.y = 0.0f;
-            b.y = 0.0f;
-        }
-        O[t] = make_float2(a.x - b.y, a.y + b.x);
-    }
-    __syncthreads();
-    float2* res2 = fft_lines(O, res, plan_z, np, twz, 1.0f);
-    float* plane = real + (size_t)x * fy * fz;
-    for (int t = threadIdx.x; t < np * fz; t += blockDim.x)
-    {
-        int p = t / fz, z = t - p * fz;
-        float2 v = res2[t];
-        plane[(size_t)(2 * p) * fz + z] = v.x;
-        if (2 * p + 1 < fy) plane[(size_t)(2 * p + 1) * fz + z] = v.y;
-    }
+    fft_run<1, false>(
+        plan_z, np, lsz, mid, res, twzg, twz,
+        [=](int p, int k, int d) {
+            k += d;
+            const int kk = k < fc ? k : fz - k;
+            float2 a = res[kk * lsy + 2 * p];
+            float2 b = (2 * p + 1 < fy) ? res[kk * lsy + 2 * p + 1] : make_float2(0.0f, 0.0f);
+            if (k >= fc)
+            {
+                a.y = -a.y;
+                b.y = -b.y;
+            }
+            if (k == 0 || (nyq && 2 * k == fz))
+            {
+                a.y = 0.0f;
+                b.y = 0.0f;
+            }
+            return make_float2(a.x - b.y, a.y + b.x);
+        },
+        [=](int p, int z, int d, float2 v) {
+            at32(plane + d, 2 * p * fz + z) = v.x;
+            if (2 * p + 1 < fy) at32(plane + fz + d, 2 * p * fz + z) = v.y;
+        });
 }
 
-__global__ void __launch_bounds__(1024) k_fft_plane_inv(const float2* __restrict__ spec,
+__global__ void __launch_bounds__(SNB_PLANE_THREADS) k_fft_plane_inv(const float2* __restrict__ spec,
                                                         float* __restrict__ real, int fy,
                                                         int fz, int fc, SnbFftPlan plan_z,
                                                         SnbFftPlan plan_y,
@@ -614,7 +757,7 @@ struct PlaneInvArgs
     const float2* twyg;
 };
 
-__global__ void __launch_bounds__(1024) k_fft_plane_inv_batch(SnbSegTab t)
+__global__ void __launch_bounds__(SNB_PLANE_THREADS) k_fft_plane_inv_batch(SnbSegTab t)
 {
     unsigned bid, nbid;
     const PlaneInvArgs& a = snb_seg<PlaneInvArgs>(t, bid, nbid);
@@ -1169,12 +1312,14 @@ static int upload_twiddles(int n, float2** dst)
     return SNB_OK;
 }
 
-// lines per workgroup for the y and x passes (a chunk of consecutive kz)
+// lines per workgroup for the y and x passes (a chunk of consecutive kz): at
+// most 16, the same number in every chunk up to one
 static int fft_w(int fc, int n)
 {
     int w = lines_per_block(n);
     if (w > 16) w = 16;
-    return fc < w ? fc : w;
+    const int nchunk = (fc + w - 1) / w;
+    return (fc + nchunk - 1) / nchunk;
 }
 
 // Influence function BC[kx][ky][kz] over the half spectrum (PM_force.cpp:544-612,
@@ -1271,7 +1416,13 @@ int snb_pme_setup_tables(snb_context* ctx, const SnbBox& box)
     return snb_pme_compute_bc(ctx, box);
 }
 
-static size_t lds_lines(int n, int L) { return sizeof(float2) * ((size_t)n + 2 * (size_t)L * n); }
+// twiddles and one or two buffers of L lines: two between three passes, and
+// for the convolution between two transforms
+static size_t lds_lines(const SnbFftPlan& plan, int L, bool conv)
+{
+    const size_t nbuf = conv || plan.npass > 2 ? 2 : 1;
+    return sizeof(float2) * ((size_t)plan.n + nbuf * (size_t)L * fft_ls(plan.n));
+}
 
 // Whether one x-plane of the grid fits the fused plane kernels' LDS; grants
 // the dynamic LDS on first use.
@@ -1299,7 +1450,8 @@ static int fft_yz_inverse(snb_context* ctx, float2* cplx, float* real)
     if (rc) return rc;
     if (ok)
     {
-        SNB_LAUNCH_B(k_fft_plane_inv, k_fft_plane_inv_batch, PlaneInvArgs, dim3(P.fx), dim3(1024),
+        SNB_LAUNCH_B(k_fft_plane_inv, k_fft_plane_inv_batch, PlaneInvArgs, dim3(P.fx),
+                     dim3(SNB_PLANE_THREADS),
                      plane_lds(P.fy, P.fz, P.fc), s, cplx, real, P.fy, P.fz, P.fc, P.plan_z,
                      P.plan_y, P.tw_z, P.tw_y);
         SNB_CHECK(hipGetLastError());
@@ -1307,12 +1459,14 @@ static int fft_yz_inverse(snb_context* ctx, float2* cplx, float* real)
     }
     int W = fft_w(P.fc, P.fy);
     int nchunk = (P.fc + W - 1) / W;
-    SNB_LAUNCH_B(k_fft_y, k_fft_y_batch, FftYArgs, dim3(P.fx * nchunk), dim3(256),
-                 lds_lines(P.fy, W), s, cplx, P.fx, P.fy, P.fc, P.plan_y, P.tw_y, W, 1.0f);
+    SNB_LAUNCH_B(k_fft_y<1>, k_fft_y_batch<1>, FftYArgs, dim3(P.fx * nchunk),
+                 dim3(fft_threads(P.plan_y)), lds_lines(P.plan_y, W, false), s, cplx, P.fx, P.fy, P.fc,
+                 P.plan_y, P.tw_y, W);
     int nrow = P.fx * P.fy;
     int Lz = lines_per_block(P.fz);
     SNB_LAUNCH_B(k_fft_z_c2r, k_fft_z_c2r_batch, FftZc2rArgs, dim3((nrow + Lz - 1) / Lz),
-                 dim3(256), lds_lines(P.fz, Lz), s, cplx, real, nrow, P.plan_z, P.fc, P.tw_z, Lz);
+                 dim3(fft_threads(P.plan_z)), lds_lines(P.plan_z, Lz, false), s, cplx, real, nrow,
+                 P.plan_z, P.fc, P.tw_z, Lz);
     SNB_CHECK(hipGetLastError());
     return SNB_OK;
 }
@@ -1325,52 +1479,56 @@ int snb_launch_fft_r2c(snb_context* ctx, const float* real, float2* cplx)
     // the LDS: line passes with small LDS share compute units with it
     int nrow = P.fx * P.fy;
     int Lz = lines_per_block(P.fz);
-    SNB_LAUNCH_B(k_fft_z_r2c, k_fft_z_r2c_batch, FftZr2cArgs, dim3((nrow + Lz - 1) / Lz), dim3(256),
-                 lds_lines(P.fz, Lz), s, real, cplx, nrow, P.plan_z, P.fc, P.tw_z, Lz);
+    SNB_LAUNCH_B(k_fft_z_r2c, k_fft_z_r2c_batch, FftZr2cArgs, dim3((nrow + Lz - 1) / Lz),
+                 dim3(fft_threads(P.plan_z)), lds_lines(P.plan_z, Lz, false), s, real, cplx, nrow,
+                 P.plan_z, P.fc, P.tw_z, Lz);
     int W = fft_w(P.fc, P.fy);
     int nchunk = (P.fc + W - 1) / W;
-    SNB_LAUNCH_B(k_fft_y, k_fft_y_batch, FftYArgs, dim3(P.fx * nchunk), dim3(256),
-                 lds_lines(P.fy, W), s, cplx, P.fx, P.fy, P.fc, P.plan_y, P.tw_y, W, -1.0f);
+    SNB_LAUNCH_B(k_fft_y<-1>, k_fft_y_batch<-1>, FftYArgs, dim3(P.fx * nchunk),
+                 dim3(fft_threads(P.plan_y)), lds_lines(P.plan_y, W, false), s, cplx, P.fx, P.fy, P.fc,
+                 P.plan_y, P.tw_y, W);
     SNB_CHECK(hipGetLastError());
     return SNB_OK;
 }
 
 // x-direction plain transform (no convolution), used by the FFT wrappers.
-__global__ void __launch_bounds__(256) k_fft_x(float2* __restrict__ spec, int fx, int fy, int fc,
-                                               SnbFftPlan plan, const float2* __restrict__ twg,
-                                               int W, float s)
+template <int SIGN>
+__global__ void __launch_bounds__(SNB_FFT_MAX_THREADS, SNB_FFT_WAVES) k_fft_x(float2* __restrict__ spec, int fx,
+                                                          int fy, int fc, SnbFftPlan plan,
+                                                          const float2* __restrict__ twg, int W)
 {
     extern __shared__ float2 smem[];
-    int n = plan.n;
+    const int n = plan.n, ls = fft_ls(n);
     float2* tw = smem;
     float2* a = smem + n;
-    float2* b = a + W * n;
+    float2* b = a + W * ls;
     load_twiddles(tw, twg, n);
-    int nchunk = (fc + W - 1) / W;
-    int y = blockIdx.x / nchunk;
-    int k0 = (blockIdx.x - y * nchunk) * W;
-    int w = min(W, fc - k0);
-    for (int t = threadIdx.x; t < n * w; t += blockDim.x)
-    {
-        int x = t / w, l = t - x * w;
-        a[l * n + x] = spec[((size_t)x * fy + y) * fc + k0 + l];
-    }
-    __syncthreads();
-    float2* res = fft_lines(a, b, plan, w, tw, s);
-    for (int t = threadIdx.x; t < n * w; t += blockDim.x)
-    {
-        int x = t / w, l = t - x * w;
-        spec[((size_t)x * fy + y) * fc + k0 + l] = res[l * n + x];
-    }
+    const int nchunk = (fc + W - 1) / W;
+    const int y = uni(blockIdx.x / nchunk);
+    const int k0 = uni((blockIdx.x - y * nchunk) * W);
+    const int w = uni(min(W, fc - k0));
+    const size_t plane = (size_t)fy * fc;
+    float2* io = spec + (size_t)y * fc + k0;
+    fft_run<SIGN, true>(
+        plan, w, ls, a, b, twg, tw,
+        [=](int l, int i, int d) { return at32(io + d * plane, (unsigned)i * plane + l); },
+        [=](int l, int i, int d, float2 v) {
+            at32(io + d * plane, (unsigned)i * plane + l) = v;
+        });
 }
 
-static int fft_x_plain(snb_context* ctx, float2* cplx, float sign)
+static int fft_x_plain(snb_context* ctx, float2* cplx, bool inverse)
 {
     SnbPme& P = ctx->pme;
     int W = fft_w(P.fc, P.fx);
     int nchunk = (P.fc + W - 1) / W;
-    SNB_LAUNCH(k_fft_x, dim3(P.fy * nchunk), dim3(256), lds_lines(P.fx, W),
-               ctx->stream, cplx, P.fx, P.fy, P.fc, P.plan_x, P.tw_x, W, sign);
+    const size_t lds = lds_lines(P.plan_x, W, false);
+    if (inverse)
+        SNB_LAUNCH(k_fft_x<1>, dim3(P.fy * nchunk), dim3(fft_threads(P.plan_x)), lds, ctx->stream,
+                   cplx, P.fx, P.fy, P.fc, P.plan_x, P.tw_x, W);
+    else
+        SNB_LAUNCH(k_fft_x<-1>, dim3(P.fy * nchunk), dim3(fft_threads(P.plan_x)), lds, ctx->stream,
+                   cplx, P.fx, P.fy, P.fc, P.plan_x, P.tw_x, W);
     SNB_CHECK(hipGetLastError());
     return SNB_OK;
 }
@@ -1381,7 +1539,7 @@ int snb_launch_fft_c2r(snb_context* ctx, const float2* cplx_in, float* real)
     hipStream_t s = ctx->stream;
     size_t nfft = (size_t)P.fx * P.fy * P.fc;
     SNB_CHECK(hipMemcpyAsync(P.spec, cplx_in, sizeof(float2) * nfft, hipMemcpyDeviceToDevice, s));
-    int rc = fft_x_plain(ctx, P.spec, 1.0f);
+    int rc = fft_x_plain(ctx, P.spec, true);
     if (rc) return rc;
     return fft_yz_inverse(ctx, P.spec, real);
 }
@@ -1390,7 +1548,7 @@ int snb_fft_forward_full(snb_context* ctx, const float* real, float2* cplx)
 {
     int rc = snb_launch_fft_r2c(ctx, real, cplx);
     if (rc) return rc;
-    return fft_x_plain(ctx, cplx, -1.0f);
+    return fft_x_plain(ctx, cplx, false);
 }
 
 int snb_launch_pme_recip(snb_context* ctx, const snb_vector* crd, const float* charge,
@@ -1438,13 +1596,15 @@ int snb_launch_pme_recip(snb_context* ctx, const snb_vector* crd, const float* c
     bool ev = need_energy || need_virial;
     if (ev)
         SNB_LAUNCH_B((k_fft_x_conv<true>), (k_fft_x_conv_batch<true>), FftXConvArgs,
-                     dim3(P.fy * nchunk), dim3(256), lds_lines(P.fx, W), s, P.spec, P.bc, P.fx,
+                     dim3(P.fy * nchunk), dim3(fft_threads(P.plan_x)), lds_lines(P.plan_x, W, true), s,
+                     P.spec, P.bc, P.fx,
                      P.fy, P.fz, P.fc, P.plan_x, P.tw_x, W, (double)box.rc[0], (double)box.rc[1],
                      (double)box.rc[2], (double)box.rc[3], (double)box.rc[4], (double)box.rc[5],
                      mpre, P.partials);
     else
         SNB_LAUNCH_B((k_fft_x_conv<false>), (k_fft_x_conv_batch<false>), FftXConvArgs,
-                     dim3(P.fy * nchunk), dim3(256), lds_lines(P.fx, W), s, P.spec, P.bc, P.fx,
+                     dim3(P.fy * nchunk), dim3(fft_threads(P.plan_x)), lds_lines(P.plan_x, W, true), s,
+                     P.spec, P.bc, P.fx,
                      P.fy, P.fz, P.fc, P.plan_x, P.tw_x, W, (double)box.rc[0], (double)box.rc[1],
                      (double)box.rc[2], (double)box.rc[3], (double)box.rc[4], (double)box.rc[5],
                      mpre, P.partials);
