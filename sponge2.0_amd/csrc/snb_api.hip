@@ -112,7 +112,8 @@ void free_nl(SnbNl& L)
 
 void free_window(SnbNl& L)
 {
-    dfree(L.nl16);
+    dfree(L.nl16_mem);
+    L.nl16 = nullptr;
     dfree(L.row_count);
     dfree(L.row_split);
     dfree(L.win_size);
@@ -123,6 +124,11 @@ void free_window(SnbNl& L)
     dfree(L.pub_count);
     dfree(L.ex_rng);
     dfree(L.block_work);
+    dfree(L.wslots);
+    dfree(L.units);
+    dfree(L.unit_run);
+    dfree(L.unit_count);
+    dfree(L.unit_base);
     dfree(L.block_perm);
     L.windowed = false;
 }
@@ -549,6 +555,7 @@ int snb_context_destroy(snb_context* c)
     dfree(c->lj.a);
     dfree(c->lj.b);
     dfree(c->lj.ab2);
+    dfree(c->lj.nolj);
     dfree(c->lj.coul);
     delete c;
     return SNB_OK;
@@ -635,7 +642,7 @@ int snb_set_exclusions(snb_context* c, const int* h_start, const int* h_list, co
 // ----------------------------------------------------------------- neighbor list
 static bool window_list_fits(const snb_context* c)
 {
-    return (double)c->n * c->nl.max_nb * sizeof(uint16_t) < 4294967296.0;
+    return ((double)c->n * c->nl.max_nb + 2 * SNB_NL16_PAD) * sizeof(uint16_t) < 4294967296.0;
 }
 
 // Allocates the windowed path's buffers for the shape in c->nl.win.
@@ -647,7 +654,8 @@ static int setup_window(snb_context* c)
     int rc = SNB_OK;
     L.invmax = window_cover(W.wu, W.a, W.nx) * window_cover(W.wv, W.b, W.ny) *
                window_cover(W.wz, W.s, W.nz);
-    if (!rc) rc = dalloc(&L.nl16, (size_t)n * L.max_nb);
+    if (!rc) rc = dalloc(&L.nl16_mem, (size_t)n * L.max_nb + 2 * SNB_NL16_PAD);
+    if (!rc) L.nl16 = L.nl16_mem + SNB_NL16_PAD;
     if (!rc) rc = dalloc(&L.row_count, n);
     if (!rc) rc = dalloc(&L.row_split, n);
     if (!rc) rc = dalloc(&L.win_size, W.nblock + 1);
@@ -659,6 +667,12 @@ static int setup_window(snb_context* c)
     if (!rc) rc = dalloc(&L.pub_count, n);
     if (!rc) rc = dalloc(&L.ex_rng, n);
     if (!rc) rc = dalloc(&L.block_work, W.nblock);
+    L.units_per_row = L.max_nb / 128 + 2;
+    if (!rc) rc = dalloc(&L.wslots, (size_t)n * L.invmax);
+    if (!rc) rc = dalloc(&L.units, (size_t)n * L.units_per_row);
+    if (!rc) rc = dalloc(&L.unit_run, (size_t)W.nblock * SNB_UNIT_RUNS);
+    if (!rc) rc = dalloc(&L.unit_count, W.nblock);
+    if (!rc) rc = dalloc(&L.unit_base, W.nblock + 1);
     if (!rc) rc = dalloc(&L.block_perm, W.nblock);
     if (rc)
     {
@@ -946,7 +960,7 @@ int snb_lj_set_row_stream(snb_context* c, int mode)
 {
     if (!c) return SNB_ERR_ARGUMENT;
     if (mode < -1 || mode > 1) return SNB_ERR_ARGUMENT;
-    c->lj.row_stream = mode;
+    // one loop, pipelined across row ends, serves every mode
     return SNB_OK;
 }
 
@@ -1006,10 +1020,12 @@ int snb_lj_initial(snb_context* c, int ntypes, const float* h_a, const float* h_
     dfree(J.a);
     dfree(J.b);
     dfree(J.ab2);
+    dfree(J.nolj);
     size_t npair = (size_t)ntypes * (ntypes + 1) / 2;
     int rc = dalloc(&J.a, npair);
     if (!rc) rc = dalloc(&J.b, npair);
     if (!rc) rc = dalloc(&J.ab2, (size_t)ntypes * ntypes);
+    if (!rc) rc = dalloc(&J.nolj, ntypes);
     if (!rc && !J.coul) rc = dalloc(&J.coul, SNB_COUL_N);
     if (rc) return rc;
     SNB_CHECK(hipMemcpy(J.a, h_a, sizeof(float) * npair, hipMemcpyHostToDevice));
@@ -1017,13 +1033,16 @@ int snb_lj_initial(snb_context* c, int ntypes, const float* h_a, const float* h_
     // square table for the windowed kernel, both parameters times 2^32 (an
     // exact power-of-two scaling)
     std::vector<float2> ab2((size_t)ntypes * ntypes);
+    std::vector<int> nolj(ntypes, 1);
     for (int a = 0; a < ntypes; a++)
         for (int b = 0; b < ntypes; b++)
         {
             int p = snb_lj_pair_index(a, b);
             ab2[(size_t)a * ntypes + b] =
                 make_float2(h_a[p] * 4294967296.0f, h_b[p] * 4294967296.0f);
+            if (h_a[p] != 0.0f || h_b[p] != 0.0f) nolj[a] = 0;
         }
+    SNB_CHECK(hipMemcpy(J.nolj, nolj.data(), sizeof(int) * ntypes, hipMemcpyHostToDevice));
     SNB_CHECK(hipMemcpy(J.ab2, ab2.data(), sizeof(float2) * ab2.size(), hipMemcpyHostToDevice));
     J.coul_beta = -1.0f;
     if (c->n > 0) SNB_CHECK(hipMemcpy(c->type, h_type, sizeof(int) * c->n, hipMemcpyHostToDevice));

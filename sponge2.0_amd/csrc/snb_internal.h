@@ -55,6 +55,10 @@ struct SnbFftPlan
     uint64_t code;
 };
 
+// spare list entries on either side of the windowed list: the pair kernel reads
+// whole 128-entry units of a row and ignores what lies beyond its ends
+#define SNB_NL16_PAD 128
+
 struct SnbNl
 {
     bool init = false;
@@ -85,6 +89,7 @@ struct SnbNl
     bool windowed = false;
     int export_mode = 1;  // reference-layout list at rebuild: 0 no, 1 yes, 2 yes with sorted rows
     SnbWin win;
+    uint16_t* nl16_mem = nullptr;  // the allocation: SNB_NL16_PAD entries on either side
     uint16_t* nl16 = nullptr;    // n * max_nb window slots, rows by sorted position
     int* row_count = nullptr;    // n: entries of each row
     int* row_split = nullptr;    // n: near pairs of each row (front part, snb_row_entry)
@@ -97,7 +102,13 @@ struct SnbNl
     int invmax = 0;
     int* pub_count = nullptr;    // n (export scratch)
     int2* ex_rng = nullptr;      // n: first/last exclusion partner per atom id
-    int* block_work = nullptr;   // nblock: list entries owned by each block
+    int* block_work = nullptr;   // nblock: cost of each block's units
+    int* wslots = nullptr;       // n * invmax: sorted index of each stage slot
+    int4* units = nullptr;       // the blocks' units (snb_window.h), n * units_per_row
+    int* unit_run = nullptr;     // nblock * SNB_UNIT_RUNS
+    int* unit_count = nullptr;   // nblock: units of each block
+    int* unit_base = nullptr;    // nblock + 1 (exclusive scan of unit_count)
+    int units_per_row = 0;       // most units of one row
     int* block_perm = nullptr;   // nblock: launch order, heaviest block first
     size_t win_lds_set = 0;      // dynamic LDS granted to the pair kernel
 };
@@ -111,6 +122,7 @@ struct SnbLj
     float* b = nullptr;
     // (A, B) of type pair (ti, tj) at ti * ntypes + tj, scaled by 2^32
     float2* ab2 = nullptr;
+    int* nolj = nullptr;  // per type: 1 if A and B are zero with every type
     // Coulomb force shape table (SNB_COUL_N pieces) for coul_beta and the cutoff
     float4* coul = nullptr;
     float coul_scale = 0.0f, coul_beta = -1.0f, coul_cutoff = -1.0f;
@@ -121,9 +133,6 @@ struct SnbLj
     // per-atom energy/virial of a pair: false = the lower atom id (the
     // reference's row atom), true = the windowed list's row owner (cheaper)
     bool owner_attribution = false;
-    // force-only pair loop: -1 by size, 0 pipelined within each row, 1
-    // pipelined across row ends
-    int row_stream = -1;
     // window forces of force-only steps: -1 by size, 0 through the stage and
     // its per-atom gather, 1 by atomic adds at the end of each block
     int j_direct = -1;

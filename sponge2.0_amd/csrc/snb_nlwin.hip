@@ -412,28 +412,103 @@ __global__ void __launch_bounds__(512) k_nl_build_cell_batch(SnbSegTab t)
         a.max_nb, a.near2, a.nl16, a.row_count, a.row_split, a.status, a.grid_length, bid, nbid);
 }
 
-// Number of window atoms of every block (one wavefront per block).
+// The rows of the block at (x0, y0, z0), 64 at a time, column by column:
+// visit(row or beyond the column's end, column, near entries, far entries).
+template <class V>
+__device__ __forceinline__ void each_block_rows(const SnbWin& W, int x0, int y0, int z0, int lane,
+                                                const int* __restrict__ start,
+                                                const int* __restrict__ row_count,
+                                                const int* __restrict__ row_split, V&& visit)
+{
+    const int z1 = z0 + W.s < W.nz ? z0 + W.s : W.nz;
+    for (int ua = 0; ua < W.a; ua++)
+        for (int vb = 0; vb < W.b; vb++)
+        {
+            if (x0 + ua >= W.nx || y0 + vb >= W.ny) continue;
+            const int colbase = ((x0 + ua) * W.ny + (y0 + vb)) * W.nz;
+            const int e = start[colbase + z1];
+            for (int s0 = start[colbase + z0]; s0 < e; s0 += 64)
+            {
+                const int si = s0 + lane;
+                int near = 0, far = 0;
+                if (si < e)
+                {
+                    near = row_split[si];
+                    far = row_count[si] - near;
+                }
+                visit(si, ua * W.wv + vb + 2, near, far);
+            }
+        }
+}
+
+// Units of one row (snb_window.h) and their cost in the pair kernel's
+// instructions: about 50 for any unit, 60 more per 64 near entries.
+__device__ __forceinline__ int units_of(int near, int far)
+{
+    return ((near + 127) >> 7) + ((far + 127) >> 7);
+}
+__device__ __forceinline__ int unit_cost(bool far, int entries)
+{
+    return far ? 50 : (entries > 64 ? 170 : 110);
+}
+__device__ __forceinline__ int row_cost(int near, int far)
+{
+    const int rest = near & 127;
+    return (near >> 7) * unit_cost(false, 128) + (rest ? unit_cost(false, rest) : 0) +
+           ((far + 127) >> 7) * unit_cost(true, 0);
+}
+
+// Window atoms, units and cost of every block (one wavefront per block).
 __device__ __forceinline__ void k_win_sizes_body(const int* __restrict__ need, SnbWin W,
                                                   const int* __restrict__ start,
+                                                  const int* __restrict__ row_count,
+                                                  const int* __restrict__ row_split,
                                                   int* __restrict__ win_size,
+                                                  int* __restrict__ unit_count,
+                                                  int* __restrict__ work,
     unsigned bid, unsigned nbid)
 {
     if (need[0] == 0) return;
-    __shared__ int first[SNB_WIN_MAX_RANGES];
-    __shared__ int pref[SNB_WIN_MAX_RANGES + 1];
     const int w = bid, lane = threadIdx.x;
     int x0, y0, z0;
     snb_win_block(W, w, x0, y0, z0);
-    win_table_wave(W, start, x0, y0, z0, lane, first, pref);
-    __syncthreads();
-    if (lane == 0) win_size[w] = pref[SNB_WIN_MAX_RANGES];
+    int size = 0;
+    for (int k = lane; k < W.nrange; k += 64)
+    {
+        int fc, nc;
+        snb_win_range_cells(W, x0, y0, z0, k, fc, nc);
+        size += nc > 0 ? start[fc + nc] - start[fc] : 0;
+    }
+    int cost = 0, count = 0;
+    each_block_rows(W, x0, y0, z0, lane, start, row_count, row_split,
+                    [&](int, int, int near, int far) {
+                        cost += row_cost(near, far);
+                        count += units_of(near, far);
+                    });
+    for (int off = 32; off > 0; off >>= 1)
+    {
+        size += __shfl_xor(size, off);
+        cost += __shfl_xor(cost, off);
+        count += __shfl_xor(count, off);
+    }
+    if (lane == 0)
+    {
+        win_size[w] = size;
+        unit_count[w] = count;
+        work[w] = cost;
+    }
 }
 
 __global__ void __launch_bounds__(64) k_win_sizes(const int* __restrict__ need, SnbWin W,
                                                   const int* __restrict__ start,
-                                                  int* __restrict__ win_size)
+                                                  const int* __restrict__ row_count,
+                                                  const int* __restrict__ row_split,
+                                                  int* __restrict__ win_size,
+                                                  int* __restrict__ unit_count,
+                                                  int* __restrict__ work)
 {
-    k_win_sizes_body(need, W, start, win_size, blockIdx.x, gridDim.x);
+    k_win_sizes_body(need, W, start, row_count, row_split, win_size, unit_count, work, blockIdx.x,
+                     gridDim.x);
 }
 
 struct WinSizesArgs
@@ -441,60 +516,137 @@ struct WinSizesArgs
     const int* need;
     SnbWin W;
     const int* start;
+    const int* row_count;
+    const int* row_split;
     int* win_size;
+    int* unit_count;
+    int* work;
 };
 
 __global__ void __launch_bounds__(64) k_win_sizes_batch(SnbSegTab t)
 {
     unsigned bid, nbid;
     const WinSizesArgs& a = snb_seg<WinSizesArgs>(t, bid, nbid);
-    k_win_sizes_body(a.need, a.W, a.start, a.win_size, bid, nbid);
+    k_win_sizes_body(a.need, a.W, a.start, a.row_count, a.row_split, a.win_size, a.unit_count,
+                     a.work, bid, nbid);
 }
 
-// For every window slot of every block, record its stage position in the
-// list of the atom it holds (the per-step gather sums these).
-__device__ __forceinline__ void k_stage_inverse_body(const int* __restrict__ need, SnbWin W,
-                                                      const int* __restrict__ start,
-                                                      const int* __restrict__ stage_base,
-                                                      int* __restrict__ inv_count,
-                                                      int* __restrict__ inv_list, int invmax,
-                                                      int* __restrict__ status,
-    unsigned bid, unsigned nbid)
+// The units of the block whose window table is (first, pref), by one
+// wavefront: units[base ..), and the first unit of each of the 16 wavefronts
+// of the pair kernel's workgroup, which take contiguous runs of equal cost.
+__device__ void write_units(const SnbWin& W, int w, int x0, int y0, int z0, int lane,
+                            const int* __restrict__ start, const int* __restrict__ row_count,
+                            const int* __restrict__ row_split, int max_nb, const int* first,
+                            const int* pref, int cost, int base, int end,
+                            int4* __restrict__ units, int* __restrict__ unit_run)
+{
+    int* run = unit_run + w * SNB_UNIT_RUNS;
+    if (lane < SNB_UNIT_RUNS) run[lane] = lane == 0 ? base : end;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    int c0 = 0, t0 = base;  // cost and units before this batch of rows
+    const float per_cost = (float)(SNB_UNIT_RUNS - 1) / (float)(cost > 0 ? cost : 1);
+    each_block_rows(W, x0, y0, z0, lane, start, row_count, row_split, [&](int si, int col, int near,
+                                                                         int far) {
+        // the column's own z-cells do not wrap: part 1 of its run when the
+        // run starts below z = 0, else part 0
+        const int k = 2 * col + (z0 < 2 ? 1 : 0);
+        const int slot_d = pref[k] - first[k];
+        const int rc = row_cost(near, far), rn = units_of(near, far);
+        int ce = rc, te = rn;
+        for (int off = 1; off < 64; off <<= 1)
+        {
+            const int a = __shfl_up(ce, off), b = __shfl_up(te, off);
+            if (lane >= off)
+            {
+                ce += a;
+                te += b;
+            }
+        }
+        int c = c0 + ce - rc, t = t0 + te - rn;
+        const int near_u = (near + 127) >> 7;
+        for (int j = 0; j < rn; j++)
+        {
+            const bool is_far = j >= near_u;
+            const int k0 = (is_far ? j - near_u : j) << 7;
+            const int left = (is_far ? far : near) - k0, entries = left < 128 ? left : 128;
+            const int at = si * max_nb + (is_far ? max_nb - 128 - k0 : k0) + SNB_NL16_PAD;
+            units[t] = make_int4(si, at, si + slot_d,
+                                 entries | (is_far ? SNB_UNIT_FAR : 0) |
+                                     (j + 1 == rn ? SNB_UNIT_LAST : 0));
+            // wavefront v starts at the unit that holds its share's first
+            // cost, or after it when that lies in the unit's second half
+            const int uc = unit_cost(is_far, entries);
+            int v = (int)((float)c * per_cost) - 1;  // at or below the first share >= c
+            for (v = v < 1 ? 1 : v; v < SNB_UNIT_RUNS - 1; v++)
+            {
+                const int share = (int)((long long)cost * v / (SNB_UNIT_RUNS - 1));
+                if (share >= c + uc) break;
+                if (share >= c) run[v] = 2 * (share - c) < uc ? t : t + 1;
+            }
+            c += uc;
+            t++;
+        }
+        c0 += __shfl(ce, 63);
+        t0 += __shfl(te, 63);
+    });
+}
+
+// Per block: the atom of every window slot (wslots, at the slot's stage
+// position) and that position in the atom's list (the per-step gather sums
+// these); one of the four wavefronts writes the block's units instead.
+__device__ __forceinline__ void k_stage_inverse_body(
+    const int* __restrict__ need, SnbWin W, const int* __restrict__ start,
+    const int* __restrict__ stage_base, int* __restrict__ inv_count, int* __restrict__ inv_list,
+    int invmax, int* __restrict__ wslots, int wslots_cap, int* __restrict__ status,
+    const int* __restrict__ row_count, const int* __restrict__ row_split, int max_nb,
+    const int* __restrict__ work, const int* __restrict__ unit_base, int4* __restrict__ units,
+    int* __restrict__ unit_run, unsigned bid, unsigned nbid)
 {
     if (need[0] == 0) return;
     __shared__ int first[SNB_WIN_MAX_RANGES];
     __shared__ int pref[SNB_WIN_MAX_RANGES + 1];
     int w = bid, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int nwave = blockDim.x >> 6;
     int x0, y0, z0;
     snb_win_block(W, w, x0, y0, z0);
     if (wave == 0) win_table_wave(W, start, x0, y0, z0, lane, first, pref);
     __syncthreads();
+    if (wave == nwave - 1)
+    {
+        write_units(W, w, x0, y0, z0, lane, start, row_count, row_split, max_nb, first, pref,
+                    work[w], unit_base[w], unit_base[w + 1], units, unit_run);
+        return;
+    }
     int base = stage_base[w];
-    for (int k = wave; k < W.nrange; k += blockDim.x >> 6)
+    for (int k = wave; k < W.nrange; k += nwave - 1)
     {
         // ranges beyond nrange are empty, so pref[k + 1] is defined for k < nrange <= 128
         int cnt = pref[k + 1] - pref[k];
         for (int t = lane; t < cnt; t += 64)
         {
             int s = first[k] + t;
+            const int at = base + pref[k] + t;
+            if (at < wslots_cap) wslots[at] = s;
             int idx = atomicAdd(&inv_count[s], 1);
             if (idx < invmax)
-                inv_list[(size_t)s * invmax + idx] = base + pref[k] + t;
+                inv_list[(size_t)s * invmax + idx] = at;
             else
                 atomicOr(status, SNB_FLAG_NL_OVERFLOW);
         }
     }
 }
 
-__global__ void __launch_bounds__(256) k_stage_inverse(const int* __restrict__ need, SnbWin W,
-                                                      const int* __restrict__ start,
-                                                      const int* __restrict__ stage_base,
-                                                      int* __restrict__ inv_count,
-                                                      int* __restrict__ inv_list, int invmax,
-                                                      int* __restrict__ status)
+__global__ void __launch_bounds__(256) k_stage_inverse(
+    const int* __restrict__ need, SnbWin W, const int* __restrict__ start,
+    const int* __restrict__ stage_base, int* __restrict__ inv_count, int* __restrict__ inv_list,
+    int invmax, int* __restrict__ wslots, int wslots_cap, int* __restrict__ status,
+    const int* __restrict__ row_count, const int* __restrict__ row_split, int max_nb,
+    const int* __restrict__ work, const int* __restrict__ unit_base, int4* __restrict__ units,
+    int* __restrict__ unit_run)
 {
-    k_stage_inverse_body(
-        need, W, start, stage_base, inv_count, inv_list, invmax, status, blockIdx.x, gridDim.x);
+    k_stage_inverse_body(need, W, start, stage_base, inv_count, inv_list, invmax, wslots,
+                         wslots_cap, status, row_count, row_split, max_nb, work, unit_base, units,
+                         unit_run, blockIdx.x, gridDim.x);
 }
 
 struct StageInverseArgs
@@ -506,15 +658,25 @@ struct StageInverseArgs
     int* inv_count;
     int* inv_list;
     int invmax;
+    int* wslots;
+    int wslots_cap;
     int* status;
+    const int* row_count;
+    const int* row_split;
+    int max_nb;
+    const int* work;
+    const int* unit_base;
+    int4* units;
+    int* unit_run;
 };
 
 __global__ void __launch_bounds__(256) k_stage_inverse_batch(SnbSegTab t)
 {
     unsigned bid, nbid;
     const StageInverseArgs& a = snb_seg<StageInverseArgs>(t, bid, nbid);
-    k_stage_inverse_body(
-        a.need, a.W, a.start, a.stage_base, a.inv_count, a.inv_list, a.invmax, a.status, bid, nbid);
+    k_stage_inverse_body(a.need, a.W, a.start, a.stage_base, a.inv_count, a.inv_list, a.invmax,
+                         a.wslots, a.wslots_cap, a.status, a.row_count, a.row_split, a.max_nb,
+                         a.work, a.unit_base, a.units, a.unit_run, bid, nbid);
 }
 
 // slot -> sorted index through the LDS range table (binary search)
@@ -823,17 +985,27 @@ __global__ void __launch_bounds__(64) k_nl_copy_internal(int n, SnbWin W,
             W, first, pref, nl16[(size_t)s * max_nb + snb_row_entry(k, split, max_nb)])];
 }
 
-// Per atom id: first and last entry of its exclusion list (an empty window
+// Per sorted position: its LJ type, no stage entries yet.  Per atom id (with
+// exclusions): first and last entry of its exclusion list (an empty window
 // (1, 0) when it has none), the window the reference tests before searching
 // the list (neighbor_list.cpp:594-665).
-__device__ __forceinline__ void k_ex_range_body(const int* __restrict__ need, int n, const int* __restrict__ ex_start,
-                           const int* __restrict__ ex_list, const int* __restrict__ ex_num,
-                           int2* __restrict__ ex_rng,
+__device__ __forceinline__ void k_win_atoms_body(const int* __restrict__ need, int n,
+                                                 const int* __restrict__ order,
+                                                 const int* __restrict__ type,
+                                                 int* __restrict__ stype,
+                                                 int* __restrict__ inv_count,
+                                                 const int* __restrict__ ex_start,
+                                                 const int* __restrict__ ex_list,
+                                                 const int* __restrict__ ex_num,
+                                                 int2* __restrict__ ex_rng,
     unsigned bid, unsigned nbid)
 {
     if (need[0] == 0) return;
     int i = bid * blockDim.x + threadIdx.x;
     if (i >= n) return;
+    stype[i] = type[order[i]];
+    inv_count[i] = 0;
+    if (!ex_num) return;
     int en = ex_num[i];
     int2 r = make_int2(1, 0);
     if (en > 0)
@@ -850,89 +1022,45 @@ __device__ __forceinline__ void k_ex_range_body(const int* __restrict__ need, in
     ex_rng[i] = r;
 }
 
-__global__ void k_ex_range(const int* __restrict__ need, int n, const int* __restrict__ ex_start,
-                           const int* __restrict__ ex_list, const int* __restrict__ ex_num,
-                           int2* __restrict__ ex_rng)
+__global__ void k_win_atoms(const int* __restrict__ need, int n, const int* __restrict__ order,
+                            const int* __restrict__ type, int* __restrict__ stype,
+                            int* __restrict__ inv_count, const int* __restrict__ ex_start,
+                            const int* __restrict__ ex_list, const int* __restrict__ ex_num,
+                            int2* __restrict__ ex_rng)
 {
-    k_ex_range_body(need, n, ex_start, ex_list, ex_num, ex_rng, blockIdx.x, gridDim.x);
+    k_win_atoms_body(need, n, order, type, stype, inv_count, ex_start, ex_list, ex_num, ex_rng,
+                     blockIdx.x, gridDim.x);
 }
 
-struct ExRangeArgs
+struct WinAtomsArgs
 {
     const int* need;
     int n;
+    const int* order;
+    const int* type;
+    int* stype;
+    int* inv_count;
     const int* ex_start;
     const int* ex_list;
     const int* ex_num;
     int2* ex_rng;
 };
 
-__global__ void k_ex_range_batch(SnbSegTab t)
+__global__ void k_win_atoms_batch(SnbSegTab t)
 {
     unsigned bid, nbid;
-    const ExRangeArgs& a = snb_seg<ExRangeArgs>(t, bid, nbid);
-    k_ex_range_body(a.need, a.n, a.ex_start, a.ex_list, a.ex_num, a.ex_rng, bid, nbid);
-}
-
-// List entries owned by every block (one wavefront per block).
-__device__ __forceinline__ void k_block_work_body(const int* __restrict__ need, SnbWin W,
-                                                   const int* __restrict__ start,
-                                                   const int* __restrict__ row_count,
-                                                   int* __restrict__ work,
-    unsigned bid, unsigned nbid)
-{
-    if (need[0] == 0) return;
-    const int w = bid, lane = threadIdx.x;
-    int x0, y0, z0;
-    snb_win_block(W, w, x0, y0, z0);
-    const int z1 = z0 + W.s < W.nz ? z0 + W.s : W.nz;
-    int sum = 0;
-    for (int col = 0; col < W.a * W.b; col++)
-    {
-        int ua = col / W.b, vb = col - ua * W.b;
-        if (x0 + ua >= W.nx || y0 + vb >= W.ny) continue;
-        int colbase = ((x0 + ua) * W.ny + (y0 + vb)) * W.nz;
-        for (int si = start[colbase + z0] + lane; si < start[colbase + z1]; si += 64)
-            sum += row_count[si];
-    }
-    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
-    if (lane == 0) work[w] = sum;
-}
-
-__global__ void __launch_bounds__(64) k_block_work(const int* __restrict__ need, SnbWin W,
-                                                   const int* __restrict__ start,
-                                                   const int* __restrict__ row_count,
-                                                   int* __restrict__ work)
-{
-    k_block_work_body(need, W, start, row_count, work, blockIdx.x, gridDim.x);
-}
-
-struct BlockWorkArgs
-{
-    const int* need;
-    SnbWin W;
-    const int* start;
-    const int* row_count;
-    int* work;
-};
-
-__global__ void __launch_bounds__(64) k_block_work_batch(SnbSegTab t)
-{
-    unsigned bid, nbid;
-    const BlockWorkArgs& a = snb_seg<BlockWorkArgs>(t, bid, nbid);
-    k_block_work_body(a.need, a.W, a.start, a.row_count, a.work, bid, nbid);
+    const WinAtomsArgs& a = snb_seg<WinAtomsArgs>(t, bid, nbid);
+    k_win_atoms_body(a.need, a.n, a.order, a.type, a.stype, a.inv_count, a.ex_start, a.ex_list,
+                     a.ex_num, a.ex_rng, bid, nbid);
 }
 
 // Launch order of the pair kernel's blocks: descending work (ties by block
 // index), one workgroup bitonic sort; identity when there are more blocks
 // than SNB_ORDER_CAP.
 #define SNB_ORDER_CAP 4096
-__device__ __forceinline__ void k_block_order_body(const int* __restrict__ need, int nblock,
-                                                      const int* __restrict__ work,
-                                                      int* __restrict__ perm,
-    unsigned bid, unsigned nbid)
+__device__ __forceinline__ void block_order(int nblock, const int* __restrict__ work,
+                                            int* __restrict__ perm)
 {
-    if (need[0] == 0) return;
     __shared__ long long key[SNB_ORDER_CAP];
     if (nblock > SNB_ORDER_CAP)
     {
@@ -969,26 +1097,81 @@ __device__ __forceinline__ void k_block_order_body(const int* __restrict__ need,
         perm[t] = (int)(key[t] & 0xffffffffll);  // low word: the block index (>= 0)
 }
 
-__global__ void __launch_bounds__(1024) k_block_order(const int* __restrict__ need, int nblock,
-                                                      const int* __restrict__ work,
-                                                      int* __restrict__ perm)
+// out[k] = in[0] + .. + in[k - 1] for k = 0 .. n, by one workgroup of 1024
+__device__ __forceinline__ void block_scan(const int* __restrict__ in, int* __restrict__ out, int n)
 {
-    k_block_order_body(need, nblock, work, perm, blockIdx.x, gridDim.x);
+    __shared__ int part[1024];
+    const int t = threadIdx.x, chunk = (n + 1023) / 1024;
+    const int b = min(t * chunk, n), e = min(b + chunk, n);
+    int s = 0;
+    for (int i = b; i < e; i++) s += in[i];
+    part[t] = s;
+    __syncthreads();
+    for (int off = 1; off < 1024; off <<= 1)
+    {
+        const int v = t >= off ? part[t - off] : 0;
+        __syncthreads();
+        part[t] += v;
+        __syncthreads();
+    }
+    int run = t > 0 ? part[t - 1] : 0;
+    for (int i = b; i < e; i++)
+    {
+        const int v = in[i];
+        out[i] = run;
+        run += v;
+    }
+    if (t == 1023) out[n] = part[1023];
 }
 
-struct BlockOrderArgs
+// Three workgroups: first stage slot of every block, first unit of every
+// block, the launch order.
+__device__ __forceinline__ void k_block_tables_body(const int* __restrict__ need, int nblock,
+                                                    const int* __restrict__ win_size,
+                                                    int* __restrict__ stage_base,
+                                                    const int* __restrict__ unit_count,
+                                                    int* __restrict__ unit_base,
+                                                    const int* __restrict__ work,
+                                                    int* __restrict__ perm,
+    unsigned bid, unsigned nbid)
+{
+    if (need[0] == 0) return;
+    if (bid == 2)
+        block_order(nblock, work, perm);
+    else
+        block_scan(bid == 0 ? win_size : unit_count, bid == 0 ? stage_base : unit_base, nblock);
+}
+
+__global__ void __launch_bounds__(1024) k_block_tables(const int* __restrict__ need, int nblock,
+                                                       const int* __restrict__ win_size,
+                                                       int* __restrict__ stage_base,
+                                                       const int* __restrict__ unit_count,
+                                                       int* __restrict__ unit_base,
+                                                       const int* __restrict__ work,
+                                                       int* __restrict__ perm)
+{
+    k_block_tables_body(need, nblock, win_size, stage_base, unit_count, unit_base, work, perm,
+                        blockIdx.x, gridDim.x);
+}
+
+struct BlockTablesArgs
 {
     const int* need;
     int nblock;
+    const int* win_size;
+    int* stage_base;
+    const int* unit_count;
+    int* unit_base;
     const int* work;
     int* perm;
 };
 
-__global__ void __launch_bounds__(1024) k_block_order_batch(SnbSegTab t)
+__global__ void __launch_bounds__(1024) k_block_tables_batch(SnbSegTab t)
 {
     unsigned bid, nbid;
-    const BlockOrderArgs& a = snb_seg<BlockOrderArgs>(t, bid, nbid);
-    k_block_order_body(a.need, a.nblock, a.work, a.perm, bid, nbid);
+    const BlockTablesArgs& a = snb_seg<BlockTablesArgs>(t, bid, nbid);
+    k_block_tables_body(a.need, a.nblock, a.win_size, a.stage_base, a.unit_count, a.unit_base,
+                        a.work, a.perm, bid, nbid);
 }
 
 // Clears p[0 .. n) on rebuild steps only.
@@ -1019,37 +1202,6 @@ __global__ void k_fill_need_batch(SnbSegTab t)
     k_fill_need_body(a.need, a.p, a.n, bid, nbid);
 }
 
-__device__ __forceinline__ void k_win_types_body(const int* __restrict__ need, int n, const int* __restrict__ order,
-                            const int* __restrict__ type, int* __restrict__ stype,
-    unsigned bid, unsigned nbid)
-{
-    if (need[0] == 0) return;
-    int s = bid * blockDim.x + threadIdx.x;
-    if (s < n) stype[s] = type[order[s]];
-}
-
-__global__ void k_win_types(const int* __restrict__ need, int n, const int* __restrict__ order,
-                            const int* __restrict__ type, int* __restrict__ stype)
-{
-    k_win_types_body(need, n, order, type, stype, blockIdx.x, gridDim.x);
-}
-
-struct WinTypesArgs
-{
-    const int* need;
-    int n;
-    const int* order;
-    const int* type;
-    int* stype;
-};
-
-__global__ void k_win_types_batch(SnbSegTab t)
-{
-    unsigned bid, nbid;
-    const WinTypesArgs& a = snb_seg<WinTypesArgs>(t, bid, nbid);
-    k_win_types_body(a.need, a.n, a.order, a.type, a.stype, bid, nbid);
-}
-
 // Called after the cell sort of a rebuild (same device flag).
 int snb_launch_nl_window(snb_context* ctx, const SnbBox& box, const int* ex_start,
                          const int* ex_list, const int* ex_num)
@@ -1058,13 +1210,11 @@ int snb_launch_nl_window(snb_context* ctx, const SnbBox& box, const int* ex_star
     hipStream_t s = ctx->stream;
     int n = ctx->n;
     const SnbWin& W = L.win;
-    SNB_LAUNCH_B(k_win_types, k_win_types_batch, WinTypesArgs, dim3((n + 255) / 256), dim3(256), 0,
-                 s, L.need, n, L.order, ctx->type, ctx->stype);
+    SNB_LAUNCH_B(k_win_atoms, k_win_atoms_batch, WinAtomsArgs, dim3((n + 255) / 256), dim3(256), 0,
+                 s, L.need, n, L.order, ctx->type, ctx->stype, L.inv_count, ex_start, ex_list,
+                 ex_num, L.ex_rng);
     const bool ortho = box.c[1] == 0.0f && box.c[3] == 0.0f && box.c[4] == 0.0f &&
                        box.rc[1] == 0.0f && box.rc[3] == 0.0f && box.rc[4] == 0.0f;
-    if (ex_num)
-        SNB_LAUNCH_B(k_ex_range, k_ex_range_batch, ExRangeArgs, dim3((n + 255) / 256), dim3(256), 0,
-                     s, L.need, n, ex_start, ex_list, ex_num, L.ex_rng);
     if (ortho)
         SNB_LAUNCH_B(k_nl_build_cell<true>, k_nl_build_cell_batch<true>, NlBuildCellArgs,
                      dim3(L.ncell), dim3(512), 0, s, L.need, W, L.cell_start, L.sorted_crd, box,
@@ -1076,20 +1226,15 @@ int snb_launch_nl_window(snb_context* ctx, const SnbBox& box, const int* ex_star
                      L.cs2, ex_start, ex_list, ex_num, L.ex_rng, L.max_nb, L.near2, L.nl16,
                      L.row_count, L.row_split, ctx->status, L.grid_length);
     SNB_LAUNCH_B(k_win_sizes, k_win_sizes_batch, WinSizesArgs, dim3(W.nblock), dim3(64), 0, s,
-                 L.need, W, L.cell_start, L.win_size);
-    SNB_LAUNCH_B(k_block_work, k_block_work_batch, BlockWorkArgs, dim3(W.nblock), dim3(64), 0, s,
-                 L.need, W, L.cell_start, L.row_count, L.block_work);
-    SNB_LAUNCH_B(k_block_order, k_block_order_batch, BlockOrderArgs, dim3(1), dim3(1024), 0, s,
-                 L.need, W.nblock, L.block_work, L.block_perm);
-    SNB_CHECK(hipGetLastError());
-    int rc = snb_launch_exclusive_scan(s, L.win_size, L.stage_base, W.nblock);
-    if (rc) return rc;
-    // the inverse lists persist between rebuilds: clear them on rebuilds only
-    SNB_LAUNCH_B(k_fill_need, k_fill_need_batch, FillNeedArgs, dim3((n + 255) / 256), dim3(256), 0,
-                 s, L.need, L.inv_count, n);
+                 L.need, W, L.cell_start, L.row_count, L.row_split, L.win_size, L.unit_count,
+                 L.block_work);
+    SNB_LAUNCH_B(k_block_tables, k_block_tables_batch, BlockTablesArgs, dim3(3), dim3(1024), 0, s,
+                 L.need, W.nblock, L.win_size, L.stage_base, L.unit_count, L.unit_base,
+                 L.block_work, L.block_perm);
     SNB_LAUNCH_B(k_stage_inverse, k_stage_inverse_batch, StageInverseArgs, dim3(W.nblock),
                  dim3(256), 0, s, L.need, W, L.cell_start, L.stage_base, L.inv_count, L.inv_list,
-                 L.invmax, ctx->status);
+                 L.invmax, L.wslots, n * L.invmax, ctx->status, L.row_count, L.row_split, L.max_nb,
+                 L.block_work, L.unit_base, L.units, L.unit_run);
     SNB_CHECK(hipGetLastError());
     if (L.export_mode)
     {

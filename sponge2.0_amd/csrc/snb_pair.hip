@@ -38,6 +38,63 @@ __device__ __forceinline__ int64_t wave_sum(int64_t v)
     return v;
 }
 
+// a value that is the same in the whole wavefront, in a scalar register
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ float unif(float v) { return __int_as_float(uni(__float_as_int(v))); }
+
+// x + (x of the lane CTRL selects), lanes permuted by DPP within rows of 16
+template <int CTRL>
+__device__ __forceinline__ int64_t add_dpp(int64_t x)
+{
+    const int lo = (int)x, hi = (int)(x >> 32);
+    const unsigned l2 = (unsigned)__builtin_amdgcn_mov_dpp(lo, CTRL, 0xf, 0xf, true);
+    const int h2 = __builtin_amdgcn_mov_dpp(hi, CTRL, 0xf, 0xf, true);
+    return x + (int64_t)(((uint64_t)(unsigned)h2 << 32) | l2);
+}
+
+// minimum over the wavefront, in every lane (a NaN counts as no value)
+__device__ __forceinline__ float wave_min(float v)
+{
+    auto step = [&](int w) { v = fminf(v, __int_as_float(w)); };
+    step(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xf, 0xf, true));
+    step(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x124, 0xf, 0xf, true));
+    step(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x122, 0xf, 0xf, true));
+    step(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x121, 0xf, 0xf, true));
+    const int i = __float_as_int(v);
+    return fminf(fminf(__int_as_float(__builtin_amdgcn_readlane(i, 0)),
+                       __int_as_float(__builtin_amdgcn_readlane(i, 16))),
+                 fminf(__int_as_float(__builtin_amdgcn_readlane(i, 32)),
+                       __int_as_float(__builtin_amdgcn_readlane(i, 48))));
+}
+
+// Sums of three values over the wavefront: lanes 0..15 return the sum of x,
+// lanes 16..31 and 48..63 that of z, lanes 32..47 that of y.  The halves and
+// then the rows of 16 lanes are folded onto each other with two values in
+// flight (permlane swaps), the rows by rotations: 21 vector instructions and
+// no LDS, where a butterfly of each value takes 36 LDS permutes and their waits.
+__device__ __forceinline__ int64_t wave_sum3(int64_t x, int64_t y, int64_t z)
+{
+    auto swap32 = [](int64_t a, int64_t b) -> int64_t {
+        const auto l = __builtin_amdgcn_permlane32_swap((int)a, (int)b, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap((int)(a >> 32), (int)(b >> 32), false,
+                                                        false);
+        return (int64_t)(((uint64_t)h[0] << 32) | l[0]) + (int64_t)(((uint64_t)h[1] << 32) | l[1]);
+    };
+    auto swap16 = [](int64_t a, int64_t b) -> int64_t {
+        const auto l = __builtin_amdgcn_permlane16_swap((int)a, (int)b, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap((int)(a >> 32), (int)(b >> 32), false,
+                                                        false);
+        return (int64_t)(((uint64_t)h[0] << 32) | l[0]) + (int64_t)(((uint64_t)h[1] << 32) | l[1]);
+    };
+    const int64_t xy = swap32(x, y);  // lanes 0..31: x, 32..63: y
+    const int64_t zz = swap32(z, z);  // both halves: z
+    int64_t v = swap16(xy, zz);       // rows: x, z, y, z
+    v = add_dpp<0x128>(v);            // row_ror:8
+    v = add_dpp<0x124>(v);
+    v = add_dpp<0x122>(v);
+    return add_dpp<0x121>(v);
+}
+
 __device__ __forceinline__ void atomic_add_i64(int64_t* p, int64_t v)
 {
     atomicAdd((unsigned long long*)p, (unsigned long long)v);
@@ -62,6 +119,19 @@ __device__ __forceinline__ float pair_force_factor(float r2, float A, float B, f
     float4 c = ctab[k];
     float fc = (qq * (rinv2 * rinv)) * snb_coul_eval(t, c.x, c.y, c.z, c.w);
     return flj - fc;
+}
+
+// The Coulomb part alone: pair_force_factor with A = B = 0 returns 0 - this.
+__device__ __forceinline__ float pair_coulomb_factor(float r2, float qq, float beta, float cscale,
+                                                     const float4* ctab)
+{
+    const float rinv = snb_rsqrtf(r2);
+    const float r = r2 * rinv;
+    const float rinv2 = rinv * rinv;
+    float t;
+    const int k = snb_coul_piece(beta * r, cscale, &t);
+    const float4 c = ctab[k];
+    return (qq * (rinv2 * rinv)) * snb_coul_eval(t, c.x, c.y, c.z, c.w);
 }
 
 template <bool NEED_ENERGY, bool NEED_VIRIAL>
@@ -763,6 +833,17 @@ __device__ __forceinline__ void win_disp(float& dx, float& dy, float& dz, const 
         pbc_disp(dx, dy, dz, box);
 }
 
+// adds to the accumulators of a window slot (x, y, z side by side: one address
+// and two offsets)
+__device__ __forceinline__ void lds_add3(long long* acc, int slot, int64_t x, int64_t y, int64_t z)
+{
+    unsigned long long* a =
+        (unsigned long long*)((char*)acc + __umul24((unsigned)slot, 24u));
+    atomicAdd(a, (unsigned long long)x);
+    atomicAdd(a + 1, (unsigned long long)y);
+    atomicAdd(a + 2, (unsigned long long)z);
+}
+
 struct WinRowSums
 {
     int64_t sx, sy, sz, elj, ec, v0, v1, v2, v3, v4, v5;
@@ -780,7 +861,7 @@ template <bool NEED_ENERGY, bool NEED_VIRIAL>
 __device__ __forceinline__ void win_pair(WinRowSums& S, float dx, float dy, float dz, float r2,
                                          float A2, float B2, float qi2, float qj, float beta,
                                          float cscale, const float4* ctab,
-                                         int slot, int sj, bool ov, int wcap, long long* acc,
+                                         int slot, int sj, bool ov, long long* acc,
                                          int n, const int* __restrict__ order,
                                          int64_t* __restrict__ fx, int ref_attr, int id_i,
                                          int64_t* __restrict__ e_sorted,
@@ -795,9 +876,7 @@ __device__ __forceinline__ void win_pair(WinRowSums& S, float dx, float dy, floa
     S.sz += iz;
     if (!ov)
     {
-        atomicAdd((unsigned long long*)&acc[slot], (unsigned long long)ix);
-        atomicAdd((unsigned long long*)&acc[wcap + slot], (unsigned long long)iy);
-        atomicAdd((unsigned long long*)&acc[2 * wcap + slot], (unsigned long long)iz);
+        lds_add3(acc, slot, ix, iy, iz);
     }
     else
     {
@@ -882,8 +961,433 @@ __device__ __forceinline__ int win_slot_sorted(int slot, bool ov, const int* slo
     return rfirst[lo] + (slot - rpref[lo]);
 }
 
-template <bool NEED_ENERGY, bool NEED_VIRIAL, bool ORTHO, bool STREAM>
+// Force-only steps: one workgroup per block, whose window map (slot -> sorted
+// index) and list units come ready-made from the rebuild (k_stage_inverse).  A unit is up to 128 entries of one row's near or far part;
+// the units are dealt to the 16 wavefronts in contiguous runs of equal cost
+// (a row may be shared by two), so that all of them finish together, and lane
+// l of a wavefront holds what its unit l needs (64 units at a time).  A unit's
+// values go to scalar registers as it comes up.  Per iteration of the software
+// pipeline: the window slots of unit t + 1 (its list entries arrived during
+// unit t - 1), the LJ parameters of unit t (its types arrived during unit
+// t - 1), types and positions of unit t + 1, list entries of unit t + 2, then
+// the pairs of unit t, two entries per lane.  The two register sets alternate
+// (the loop body is written out twice), so no value is copied while its load
+// is in flight.
+//   - Far units hold pairs beyond rc + skin/4 at the rebuild: distances only;
+//     a pair that has come into range loads its type and parameters then.
+//   - A row whose type has no LJ with any type (nolj: the hydrogens of a
+//     TIP3P water) skips the type and parameter gathers and the LJ terms,
+//     which would be exact zeros.
+//   - Where the window's atoms spread over less than half the box along an
+//     axis, every minimum-image count of the block is zero there and
+//     d - 0 * L = d, so those instructions are skipped.
+// A window beyond the LDS capacity (OV) adds to the global accumulators
+// instead and looks slots up in the global map.
+//
+// Bound by vector issue (IEEE-only math in a fixed order, about 62
+// instructions per pair, 50 per unit and entry pair around them) at 16
+// wavefronts a CU, which the window's LDS allows.  Against a loop of whole
+// rows dealt round robin, with row metadata in vector registers and wave sums
+// through LDS: 93,000 atoms (34.6M entries) 148 -> 119 us and 65.8M -> 50.3M
+// vector instructions, 1,000,002 atoms 1583 -> 1337 us, 9,000 atoms 68 -> 54,
+// 24,999 atoms 57 -> 48 (kernel alone).  Rows dealt round robin left the
+// first wavefront of a block waiting 18 of 52 us for the last one.
+struct WinUnits
+{
+    int at, desc, type, slot, si;  // desc: u_kind, u_last, u_rem below
+    float4 a;
+};
+
+// lane's unit first + lane of those before `end`
+__device__ __forceinline__ WinUnits win_load_units(const int4* __restrict__ units, int first,
+                                                   int end, const float4* __restrict__ satom,
+                                                   const int* __restrict__ stype,
+                                                   const int* __restrict__ nolj)
+{
+    WinUnits m = {SNB_NL16_PAD, 3 << 6, 0, 0, 0, {0, 0, 0, 0}};
+    const int t = first + (int)(threadIdx.x & 63);
+    if (t < end)
+    {
+        const int4 u = units[t];
+        m.si = u.x;
+        m.at = u.y;
+        m.slot = u.z;
+        m.type = stype[u.x];
+        m.a = satom[u.x];
+        const int kind = (u.w & SNB_UNIT_FAR) ? 2 : (nolj[m.type] ? 1 : 0);
+        m.desc = kind << 6 | ((u.w & SNB_UNIT_LAST) ? 256 : 0) | (u.w & 255) << 9;
+    }
+    return m;
+}
+
+template <bool ORTHO, bool OV>
+__device__ __forceinline__ void win_force_units(
+    int n, WinUnits m, const int4* __restrict__ units, int u_first, int u_end,
+    const uint16_t* __restrict__ nl16, const float4* __restrict__ satom,
+    const int* __restrict__ stype, const int* __restrict__ order,
+    const float2* __restrict__ ab2, const int* __restrict__ nolj, int ntypes, float cscale,
+    const SnbBox& box, float rc2, float beta, int64_t* __restrict__ fx, const float4* ctab,
+    long long* acc, const int* slot_s, const int* __restrict__ wslots, int wrap_x, int wrap_y,
+    int wrap_z)
+{
+    const int lane = threadIdx.x & 63;
+    auto lane_of = [](int v, int l) { return __builtin_amdgcn_readlane(v, l); };
+    auto lane_off = [](float v, int l) -> float {
+        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+    };
+    // a unit in one word: kind (0 near, LJ; 1 near, no LJ; 2 far; 3 none),
+    // whether it is the row's last, entries (at most 128)
+    auto u_kind = [](int u) { return (u >> 6) & 3; };
+    auto u_far = [](int u) { return (u & 128) != 0; };
+    auto u_last = [](int u) { return (u & 256) != 0; };
+    auto u_rem = [](int u) { return u >> 9; };
+    struct Rec
+    {
+        int sla, slb, tja, tjb;
+        unsigned sja, sjb;
+        float4 aja, ajb;
+    };
+    // list entries lane and lane + 64 of a unit, unchecked beyond its end
+    // (the list has SNB_NL16_PAD spare entries on either side)
+    auto entries = [&](int u, int at, int& ea, int& eb) {
+        const unsigned o = (unsigned)at + (u_far(u) ? 127u - (unsigned)lane : (unsigned)lane);
+        ea = (int)ld32(nl16 - SNB_NL16_PAD, o);
+        eb = (int)ld32(nl16 - SNB_NL16_PAD + (u_far(u) ? -64 : 64), o);
+    };
+    auto slots = [&](Rec& q, int u, int ea, int eb) {
+        const int rem = u_rem(u);
+        q.sla = lane < rem ? ea : 0;
+        q.slb = lane + 64 < rem ? eb : 0;
+        q.sja = (unsigned)(OV ? wslots[q.sla] : slot_s[q.sla]);
+        q.sjb = (unsigned)(OV ? wslots[q.slb] : slot_s[q.slb]);
+    };
+    auto records = [&](Rec& q, int u) {
+        if (u_kind(u) == 0)
+        {
+            q.tja = ld32(stype, q.sja);
+            q.tjb = ld32(stype, q.sjb);
+        }
+        q.aja = ld32(satom, q.sja);
+        q.ajb = ld32(satom, q.sjb);
+    };
+    int64_t sx = 0, sy = 0, sz = 0;
+    // fa2 * d on row atom i, the opposite on j (A2, B2 and qq carry 2^32)
+    auto give = [&](float fa2, float dx, float dy, float dz, int slot, unsigned sj) {
+        const int64_t ix = snb_fixed_from_scaled(fa2 * dx), iy = snb_fixed_from_scaled(fa2 * dy),
+                      iz = snb_fixed_from_scaled(fa2 * dz);
+        sx += ix;
+        sy += iy;
+        sz += iz;
+        if (!OV)
+            lds_add3(acc, slot, ix, iy, iz);
+        else
+        {
+            const int idj = order[sj];
+            atomic_add_i64(fx + idj, -ix);
+            atomic_add_i64(fx + n + idj, -iy);
+            atomic_add_i64(fx + 2 * n + idj, -iz);
+        }
+    };
+    int C = 0, N = 0, E = 0, e_at = 0, c = 0;  // the units of the three stages, C's lane
+    auto step = [&](Rec& cur, Rec& nxt, int ea, int eb, int& fa, int& fb) {
+        // the wrap flags are tested as integers (an empty statement:
+        // otherwise their booleans are kept in lanes)
+        int wx = uni(wrap_x), wy = uni(wrap_y), wz = uni(wrap_z);
+        asm volatile("" : "+s"(wx), "+s"(wy), "+s"(wz));
+        const int kind = u_kind(C), rem = u_rem(C);
+        const float2* abrow = ab2 + lane_of(m.type, c) * ntypes;
+        float2 ABa = {0, 0}, ABb = {0, 0};
+        // the entries first: they are the last loads of the iteration
+        // before, and waiting for them behind the parameter gathers would
+        // wait for those too
+        slots(nxt, N, ea, eb);
+        asm volatile("" : "+v"(nxt.sla), "+v"(nxt.slb));
+        if (kind == 0)
+        {
+            ABa = ld32(abrow, (unsigned)cur.tja);
+            ABb = ld32(abrow, (unsigned)cur.tjb);
+        }
+        records(nxt, N);
+        entries(E, e_at, fa, fb);
+        const float xi = lane_off(m.a.x, c), yi = lane_off(m.a.y, c), zi = lane_off(m.a.z, c);
+        const float qi2 = lane_off(m.a.w, c) * 4294967296.0f;  // 2^32
+        float dxa = cur.aja.x - xi, dya = cur.aja.y - yi, dza = cur.aja.z - zi;
+        float dxb = cur.ajb.x - xi, dyb = cur.ajb.y - yi, dzb = cur.ajb.z - zi;
+        if (ORTHO)
+        {
+            if (wx)
+            {
+                dxa = dxa - rintf(dxa * box.rc[0]) * box.c[0];
+                dxb = dxb - rintf(dxb * box.rc[0]) * box.c[0];
+            }
+            if (wy)
+            {
+                dya = dya - rintf(dya * box.rc[2]) * box.c[2];
+                dyb = dyb - rintf(dyb * box.rc[2]) * box.c[2];
+            }
+            if (wz)
+            {
+                dza = dza - rintf(dza * box.rc[5]) * box.c[5];
+                dzb = dzb - rintf(dzb * box.rc[5]) * box.c[5];
+            }
+        }
+        else
+        {
+            pbc_disp(dxa, dya, dza, box);
+            pbc_disp(dxb, dyb, dzb, box);
+        }
+        const float r2a = (dxa * dxa + dya * dya) + dza * dza;
+        const float r2b = (dxb * dxb + dyb * dyb) + dzb * dzb;
+        const bool ina = lane < rem && r2a < rc2, inb = lane + 64 < rem && r2b < rc2;
+        if (kind == 0)
+        {
+            if (ina)
+                give(pair_force_factor(r2a, ABa.x, ABa.y, qi2 * cur.aja.w, beta, cscale, ctab),
+                     dxa, dya, dza, cur.sla, cur.sja);
+            if (inb)
+                give(pair_force_factor(r2b, ABb.x, ABb.y, qi2 * cur.ajb.w, beta, cscale, ctab),
+                     dxb, dyb, dzb, cur.slb, cur.sjb);
+        }
+        else if (kind == 1)
+        {
+            if (ina)
+                give(-pair_coulomb_factor(r2a, qi2 * cur.aja.w, beta, cscale, ctab), dxa, dya,
+                     dza, cur.sla, cur.sja);
+            if (inb)
+                give(-pair_coulomb_factor(r2b, qi2 * cur.ajb.w, beta, cscale, ctab), dxb, dyb,
+                     dzb, cur.slb, cur.sjb);
+        }
+        else if (__any(ina || inb))
+        {
+            // rare: pairs that came into range since the rebuild
+            for (int h = 0; h < 2; h++)
+                if (h ? inb : ina)
+                {
+                    const unsigned sj = h ? cur.sjb : cur.sja;
+                    const float2 AB = ld32(abrow, (unsigned)ld32(stype, sj));
+                    give(pair_force_factor(h ? r2b : r2a, AB.x, AB.y,
+                                           qi2 * (h ? cur.ajb.w : cur.aja.w), beta, cscale, ctab),
+                         h ? dxb : dxa, h ? dyb : dya, h ? dzb : dza, h ? cur.slb : cur.sla, sj);
+                }
+        }
+        if (u_last(C) || c == 63)
+        {
+            // the end of the row (or of this wavefront's part of it): its own force
+            const int64_t v = wave_sum3(sx, sy, sz);
+            sx = sy = sz = 0;
+            const int slot_i = lane_of(m.slot, c), si = lane_of(m.si, c);
+            if ((lane & 15) == 0 && lane < 48)
+            {
+                const int d = lane == 0 ? 0 : (lane == 32 ? 1 : 2);
+                if (!OV)  // the LDS accumulators hold the negated force
+                    atomicAdd((unsigned long long*)&acc[3 * slot_i + d], (unsigned long long)(-v));
+                else
+                    atomic_add_i64(fx + (size_t)d * n + order[si], v);
+            }
+        }
+    };
+    for (int t0 = u_first; t0 < u_end; t0 += 64)
+    {
+        if (t0 > u_first) m = win_load_units(units, t0, u_end, satom, stype, nolj);
+        const int T = u_end - t0 < 64 ? u_end - t0 : 64;
+        // this wavefront's part of its last row ends with its last unit
+        int desc = m.desc;
+        if (lane == T - 1) desc |= 256;
+        Rec r0 = {}, r1 = {};
+        int e0a, e0b, e1a, e1b, e2a = 0, e2b = 0;
+        C = lane_of(desc, 0);
+        N = lane_of(desc, 1);
+        E = lane_of(desc, 2);
+        e_at = lane_of(m.at, 2);
+        c = 0;
+        entries(C, lane_of(m.at, 0), e0a, e0b);
+        entries(N, lane_of(m.at, 1), e1a, e1b);
+        slots(r0, C, e0a, e0b);
+        records(r0, C);
+        // lanes from T on describe no unit; beyond lane 63 the value of lane
+        // 63 stands in (its entries are loaded and not used)
+        auto shift = [&]() {
+            const int l = c + 3 < 63 ? c + 3 : 63;
+            c = c + 1;
+            C = N;
+            N = E;
+            E = lane_of(desc, l);
+            e_at = lane_of(m.at, l);
+        };
+        while (true)
+        {
+            step(r0, r1, e1a, e1b, e2a, e2b);
+            if (c + 1 >= T) break;
+            shift();
+            step(r1, r0, e2a, e2b, e1a, e1b);
+            if (c + 1 >= T) break;
+            shift();
+        }
+    }
+}
+
+template <bool ORTHO>
 __device__ __forceinline__ void k_pair_win_body(
+    int n, int wcap, const uint16_t* __restrict__ nl16, const float4* __restrict__ satom,
+    const int* __restrict__ stype, const int* __restrict__ order,
+    const float2* __restrict__ ab2, const int* __restrict__ nolj, int ntypes,
+    const float4* __restrict__ coul_tab, float cscale, SnbBox box, float rc2, float beta,
+    const int* __restrict__ stage_base, const int* __restrict__ wslots,
+    const int4* __restrict__ units, const int* __restrict__ unit_run,
+    long long* __restrict__ stage, size_t stage_cap, int64_t* __restrict__ fx,
+    const int* __restrict__ perm, int jdirect, unsigned bid, unsigned nbid)
+{
+    extern __shared__ long long smem[];
+    float4* ctab = (float4*)smem;                  // [SNB_COUL_N]
+    long long* acc = smem + 2 * SNB_COUL_N;        // [wcap][3]
+    int* slot_s = (int*)(acc + 3 * (size_t)wcap);  // [wcap]
+    float* range = (float*)(slot_s + wcap);        // [16][6]: min, max of x, y, z per wavefront
+    const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
+    const int w = uni(perm[bid]);  // heaviest blocks first
+    const int base = uni(stage_base[w]), total = uni(stage_base[w + 1]) - base;
+    const int* run = unit_run + w * SNB_UNIT_RUNS + wave;
+    const int u_first = uni(run[0]), u_end = uni(run[1]);
+    WinUnits m = win_load_units(units, u_first, u_end, satom, stype, nolj);
+    if (tid < SNB_COUL_N) ctab[tid] = coul_tab[tid];
+    const bool ov = total > wcap;
+    const int* slot_map = wslots + base;
+    if (!ov)
+    {
+        const float inf = __builtin_inff();
+        float lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf};
+        for (int t = tid; t < total; t += blockDim.x)
+        {
+            const int sj = slot_map[t];
+            slot_s[t] = sj;
+            if (ORTHO)
+            {
+                const float4 a = satom[sj];
+                lo[0] = fminf(lo[0], a.x);
+                lo[1] = fminf(lo[1], a.y);
+                lo[2] = fminf(lo[2], a.z);
+                hi[0] = fmaxf(hi[0], a.x);
+                hi[1] = fmaxf(hi[1], a.y);
+                hi[2] = fmaxf(hi[2], a.z);
+            }
+        }
+        for (int t = tid; t < 3 * total; t += blockDim.x) acc[t] = 0;
+        if (ORTHO)
+            for (int d = 0; d < 3; d++)
+            {
+                const float a = wave_min(lo[d]), b = -wave_min(-hi[d]);
+                if (lane == 0)
+                {
+                    range[6 * wave + d] = a;
+                    range[6 * wave + 3 + d] = b;
+                }
+            }
+    }
+    __syncthreads();
+    if (!ov)
+    {
+        // |d| <= spread for every pair of the block, so that 0.49 leaves
+        // rint(d / L) = 0 with room for the rounding of the quotient (an
+        // infinite coordinate makes the spread infinite, and a NaN one fails
+        // the distance test with or without the image)
+        int wrap[3] = {1, 1, 1};
+        if (ORTHO)
+            for (int d = 0; d < 3; d++)
+            {
+                const int q = 6 * (lane & 15) + d;
+                const float spread = -wave_min(-range[q + 3]) - wave_min(range[q]);
+                wrap[d] = uni(spread * box.rc[d == 0 ? 0 : (d == 1 ? 2 : 5)] < 0.49f ? 0 : 1);
+            }
+        win_force_units<ORTHO, false>(n, m, units, u_first, u_end, nl16, satom, stype, order, ab2,
+                                      nolj, ntypes, cscale, box, rc2, beta, fx, ctab, acc, slot_s,
+                                      slot_map, wrap[0], wrap[1], wrap[2]);
+    }
+    else
+        win_force_units<ORTHO, true>(n, m, units, u_first, u_end, nl16, satom, stype, order, ab2,
+                                     nolj, ntypes, cscale, box, rc2, beta, fx, ctab, acc, slot_s,
+                                     slot_map, 1, 1, 1);
+    __syncthreads();
+    if (jdirect)
+    {
+        // the window's sums go straight to the id-ordered accumulators
+        // (integer sums, so the order of the adds does not matter); slots
+        // that received nothing are skipped
+        if (!ov)
+            for (int t = tid; t < total; t += blockDim.x)
+            {
+                const long long vx = acc[3 * t], vy = acc[3 * t + 1], vz = acc[3 * t + 2];
+                if ((vx | vy | vz) == 0) continue;
+                const int id = order[slot_s[t]];
+                if (vx) atomic_add_i64(fx + id, -vx);
+                if (vy) atomic_add_i64(fx + n + id, -vy);
+                if (vz) atomic_add_i64(fx + 2 * n + id, -vz);
+            }
+        return;
+    }
+    for (int t = tid; t < 3 * total; t += blockDim.x)
+    {
+        const size_t d = 3 * (size_t)base + t;
+        if (d >= 3 * stage_cap) break;  // cannot happen: stage holds n x invmax
+        stage[d] = ov ? 0 : -acc[t];
+    }
+}
+
+template <bool ORTHO>
+__global__ void __launch_bounds__(1024) k_pair_win(
+    int n, int wcap, const uint16_t* __restrict__ nl16, const float4* __restrict__ satom,
+    const int* __restrict__ stype, const int* __restrict__ order,
+    const float2* __restrict__ ab2, const int* __restrict__ nolj, int ntypes,
+    const float4* __restrict__ coul_tab, float cscale, SnbBox box, float rc2, float beta,
+    const int* __restrict__ stage_base, const int* __restrict__ wslots,
+    const int4* __restrict__ units, const int* __restrict__ unit_run,
+    long long* __restrict__ stage, size_t stage_cap, int64_t* __restrict__ fx,
+    const int* __restrict__ perm, int jdirect)
+{
+    k_pair_win_body<ORTHO>(n, wcap, nl16, satom, stype, order, ab2, nolj, ntypes, coul_tab, cscale,
+                           box, rc2, beta, stage_base, wslots, units, unit_run, stage, stage_cap,
+                           fx, perm, jdirect, blockIdx.x, gridDim.x);
+}
+
+struct PairWinArgs
+{
+    int n;
+    int wcap;
+    const uint16_t* nl16;
+    const float4* satom;
+    const int* stype;
+    const int* order;
+    const float2* ab2;
+    const int* nolj;
+    int ntypes;
+    const float4* coul_tab;
+    float cscale;
+    SnbBox box;
+    float rc2;
+    float beta;
+    const int* stage_base;
+    const int* wslots;
+    const int4* units;
+    const int* unit_run;
+    long long* stage;
+    size_t stage_cap;
+    int64_t* fx;
+    const int* perm;
+    int jdirect;
+};
+
+template <bool ORTHO>
+__global__ void __launch_bounds__(1024) k_pair_win_batch(SnbSegTab t)
+{
+    unsigned bid, nbid;
+    const PairWinArgs& a = snb_seg<PairWinArgs>(t, bid, nbid);
+    k_pair_win_body<ORTHO>(a.n, a.wcap, a.nl16, a.satom, a.stype, a.order, a.ab2, a.nolj, a.ntypes,
+                           a.coul_tab, a.cscale, a.box, a.rc2, a.beta, a.stage_base, a.wslots,
+                           a.units, a.unit_run, a.stage, a.stage_cap, a.fx, a.perm, a.jdirect, bid,
+                           nbid);
+}
+
+// Energy and virial steps: the same block and window, rows instead of units.
+template <bool NEED_ENERGY, bool NEED_VIRIAL, bool ORTHO>
+__device__ __forceinline__ void k_pair_ev_body(
     int n, SnbWin W, const int* __restrict__ start, const int* __restrict__ sorted_cell,
     const int* __restrict__ row_count, const int* __restrict__ row_split,
     const uint16_t* __restrict__ nl16, int max_nb,
@@ -892,21 +1396,23 @@ __device__ __forceinline__ void k_pair_win_body(
     const float4* __restrict__ coul_tab, float cscale, SnbBox box, float rc2, float beta,
     const int* __restrict__ stage_base, long long* __restrict__ stage, size_t stage_cap,
     int64_t* __restrict__ fx, int64_t* __restrict__ e_sorted, int64_t* __restrict__ v_sorted,
-    int ref_attr, const int* __restrict__ perm, int jdirect,
-    unsigned bid, unsigned nbid)
+    int ref_attr, const int* __restrict__ perm, unsigned bid, unsigned nbid)
 {
     extern __shared__ long long smem[];
     float4* ctab = (float4*)smem;                   // [SNB_COUL_N]
-    long long* acc = smem + 2 * SNB_COUL_N;         // [3][wcap]
+    long long* acc = smem + 2 * SNB_COUL_N;         // [wcap][3]
     int* slot_s = (int*)(acc + 3 * (size_t)W.wcap);  // [wcap]
     int* rfirst = slot_s + W.wcap;                  // [128]
     int* rpref = rfirst + SNB_WIN_MAX_RANGES;       // [129]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
     const int nwave = blockDim.x >> 6;
-    const int w = perm[bid];  // heaviest blocks first
+    const int w = uni(perm[bid]);  // heaviest blocks first
     if (tid < SNB_COUL_N) ctab[tid] = coul_tab[tid];
     int x0, y0, z0;
     snb_win_block(W, w, x0, y0, z0);
+    x0 = uni(x0);
+    y0 = uni(y0);
+    z0 = uni(z0);
     // range table: sizes, then a wave-0 scan
     int rsz = 0;
     if (tid < SNB_WIN_MAX_RANGES)
@@ -942,434 +1448,155 @@ __device__ __forceinline__ void k_pair_win_body(
         if (lane == 0) rpref[0] = 0;
     }
     __syncthreads();
-    const int total = rpref[SNB_WIN_MAX_RANGES];
+    const int total = uni(rpref[SNB_WIN_MAX_RANGES]);
     const bool ov = total > W.wcap;
     if (!ov)
     {
-        for (int k = 0; k < W.nrange; k++)
+        for (int k = wave; k < W.nrange; k += nwave)
         {
-            int b0 = rpref[k], cnt = rpref[k + 1] - b0, f = rfirst[k];
-            for (int t = tid; t < cnt; t += blockDim.x) slot_s[b0 + t] = f + t;
+            const int b0 = uni(rpref[k]), cnt = uni(rpref[k + 1]) - b0, f = uni(rfirst[k]);
+            for (int t = lane; t < cnt; t += 64) slot_s[b0 + t] = f + t;
         }
-        for (int t = tid; t < 3 * W.wcap; t += blockDim.x) acc[t] = 0;
+        for (int t = tid; t < 3 * total; t += blockDim.x) acc[t] = 0;
     }
     __syncthreads();
-    if constexpr (STREAM)
+    for (int col = 0; col < W.a * W.b; col++)
     {
-        // STREAM (force-only steps of large systems): one software pipeline
-        // per wavefront over the 128-entry steps (two entries per lane) of
-        // all its rows, across row ends, so that a row starts with its
-        // records already fetched.  Per
-        // iteration: the LJ parameters of step t (its types arrived during
-        // step t - 1), the records of step t + 1 (slot map, then position and
-        // type; its list entries arrived during step t - 1), the list entries
-        // of step t + 2, the metadata of the wavefront's next row, then the
-        // pairs of step t.  Records and entries alternate between two
-        // register sets (the loop body is written out twice), so no value
-        // is copied while its load is in flight; every load is issued on
-        // every iteration (clamped addresses) so that their count is fixed.
-        const int ncol = W.a * W.b;
-        struct RowM
+        int ua = col / W.b, vb = col - ua * W.b;
+        if (x0 + ua >= W.nx || y0 + vb >= W.ny) continue;
+        int colbase = ((x0 + ua) * W.ny + (y0 + vb)) * W.nz;
+        int z1 = z0 + W.s < W.nz ? z0 + W.s : W.nz;
+        int r0 = start[colbase + z0], r1 = start[colbase + z1];
+        for (int si = r0 + wave; si < r1; si += nwave)
         {
-            int si, col, cnt, split, type, cell;
-            float4 ai;
-        };
-        struct Rec
-        {
-            int sla, slb, tja, tjb;
-            unsigned sja, sjb;
-            float4 aja, ajb;
-        };
-        int cur_col = 0, cr0 = 0, cr1 = 0, cur_si = 0;
-        auto col_range = [&](int col) {
-            const int ua = col / W.b, vb = col - ua * W.b;
-            cr0 = cr1 = 0;
-            if (x0 + ua >= W.nx || y0 + vb >= W.ny) return;
-            const int colbase = ((x0 + ua) * W.ny + (y0 + vb)) * W.nz;
-            const int z1 = z0 + W.s < W.nz ? z0 + W.s : W.nz;
-            cr0 = start[colbase + z0];
-            cr1 = start[colbase + z1];
-        };
-        // cur_si: this wavefront's next row (-1 after its last)
-        auto seek = [&]() {
-            while (cur_si >= cr1)
+            const int cnt = row_count[si], split = row_split[si];
+            const unsigned row0 = (unsigned)si * (unsigned)max_nb;  // n * max_nb < 2^31
+            const float4 ai = satom[si];
+            const float qi2 = ai.w * 4294967296.0f;  // 2^32 fixed-point scale
+            const unsigned trow = (unsigned)(stype[si] * ntypes);
+            const int id_i = (NEED_ENERGY || NEED_VIRIAL) && ref_attr ? order[si] : 0;
+            WinRowSums S = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+            // two entries per lane at a time; each step fetches its records
+            // when it starts: the FP64 energies and row sums leave no
+            // registers for a second set of records
+            auto entry = [&](int k) -> int {
+                return k < cnt ? (int)ld32(nl16, row0 + (unsigned)snb_row_entry(k, split, max_nb))
+                               : -1;
+            };
+            auto sorted_of = [&](int sl) -> unsigned {
+                return sl >= 0 ? (unsigned)win_slot_sorted(sl, ov, slot_s, rfirst, rpref, W.nrange)
+                               : (unsigned)si;
+            };
+            int sla = 0, slb = 0, tja = 0, tjb = 0;
+            unsigned sja = 0, sjb = 0;
+            float4 aja = {0, 0, 0, 0}, ajb = {0, 0, 0, 0};
+            auto records = [&](int k) {
+                sla = entry(k + lane);
+                slb = entry(k + 64 + lane);
+                sja = sorted_of(sla);
+                sjb = sorted_of(slb);
+                aja = ld32(satom, sja);
+                ajb = ld32(satom, sjb);
+                tja = ld32(stype, sja);
+                tjb = ld32(stype, sjb);
+            };
+            for (int k0 = 0; k0 < cnt; k0 += 128)
             {
-                if (++cur_col >= ncol)
-                {
-                    cur_si = -1;
-                    return;
-                }
-                col_range(cur_col);
-                cur_si = cr0 + wave;
-            }
-        };
-        col_range(0);
-        cur_si = cr0 + wave;
-        seek();
-        // metadata of row cur_si (of row 0 when there is none: discarded)
-        auto load_row = [&]() -> RowM {
-            const int si = cur_si >= 0 ? cur_si : 0;
-            RowM r;
-            r.si = cur_si;
-            r.col = cur_col;
-            r.cnt = row_count[si];
-            r.split = row_split[si];
-            r.type = stype[si];
-            r.cell = sorted_cell[si];
-            r.ai = satom[si];
-            return r;
-        };
-        // the loaded metadata, in scalar registers (one value per wavefront)
-        auto uniform = [](const RowM& r) -> RowM {
-            RowM u;
-            u.si = __builtin_amdgcn_readfirstlane(r.si);
-            u.col = __builtin_amdgcn_readfirstlane(r.col);
-            u.cnt = __builtin_amdgcn_readfirstlane(r.cnt);
-            u.split = __builtin_amdgcn_readfirstlane(r.split);
-            u.type = __builtin_amdgcn_readfirstlane(r.type);
-            u.cell = __builtin_amdgcn_readfirstlane(r.cell);
-            u.ai.x = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(r.ai.x)));
-            u.ai.y = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(r.ai.y)));
-            u.ai.z = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(r.ai.z)));
-            u.ai.w = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(r.ai.w)));
-            return u;
-        };
-        auto entry_of = [&](const RowM& r, int k) -> int {
-            const int si = r.si >= 0 ? r.si : 0;
-            const int kk = k < r.cnt ? k : 0;
-            const int e = (int)ld32(nl16, (unsigned)si * (unsigned)max_nb +
-                                              (unsigned)snb_row_entry(kk, r.split, max_nb));
-            return r.si >= 0 && k < r.cnt ? e : -1;
-        };
-        auto records = [&](Rec& q, int sla, int slb, int si) {
-            si = si >= 0 ? si : 0;
-            q.sla = sla;
-            q.slb = slb;
-            q.sja = sla >= 0 ? (unsigned)win_slot_sorted(sla, ov, slot_s, rfirst, rpref, W.nrange)
-                             : (unsigned)si;
-            q.sjb = slb >= 0 ? (unsigned)win_slot_sorted(slb, ov, slot_s, rfirst, rpref, W.nrange)
-                             : (unsigned)si;
-            q.aja = ld32(satom, q.sja);
-            q.ajb = ld32(satom, q.sjb);
-            q.tja = ld32(stype, q.sja);
-            q.tjb = ld32(stype, q.sjb);
-        };
-        WinRowSums S = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-        // the units of the compute, record and entry stages, the next row
-        RowM cRow = uniform(load_row());
-        if (cur_si >= 0)
-        {
-            cur_si += nwave;
-            seek();
-        }
-        RowM R = load_row();
-        int cK = 0;
-        Rec r0, r1;
-        int e0a = entry_of(cRow, lane), e0b = entry_of(cRow, lane + 64);
-        records(r0, e0a, e0b, cRow.si);
-        RowM nRow = cRow, eRow = cRow;
-        int nK = 0, eK = 0;
-        // the unit after E (R, the metadata of row cur_si, is loaded again
-        // after each call)
-        auto advance = [&]() {
-            if (eRow.si < 0) return;
-            if (eK + 128 < eRow.cnt)
-                eK += 128;
-            else
-            {
-                eRow = uniform(R);
-                eK = 0;
-                if (cur_si >= 0)
-                {
-                    cur_si += nwave;
-                    seek();
-                }
-            }
-        };
-        advance();
-        R = load_row();
-        nRow = eRow;
-        nK = eK;
-        int e1a = entry_of(eRow, eK + lane), e1b = entry_of(eRow, eK + 64 + lane);
-        int e2a = -1, e2b = -1;
-        // one iteration: compute with cur, fill nxt from (ea, eb), load the
-        // entries of the unit after E into (fa, fb)
-        auto step = [&](Rec& cur, Rec& nxt, int ea, int eb, int& fa, int& fb) {
-            const unsigned trow = (unsigned)(cRow.type * ntypes);
-            const float2 ABa = ld32(ab2, trow + (unsigned)cur.tja);
-            const float2 ABb = ld32(ab2, trow + (unsigned)cur.tjb);
-            records(nxt, ea, eb, nRow.si);
-            advance();
-            fa = entry_of(eRow, eK + lane);
-            fb = entry_of(eRow, eK + 64 + lane);
-            R = load_row();
-            if (cRow.si >= 0)
-            {
-                const float4 ai = cRow.ai;
-                const float qi2 = ai.w * 4294967296.0f;  // 2^32 fixed-point scale
-                float dxa = cur.aja.x - ai.x, dya = cur.aja.y - ai.y, dza = cur.aja.z - ai.z;
-                float dxb = cur.ajb.x - ai.x, dyb = cur.ajb.y - ai.y, dzb = cur.ajb.z - ai.z;
+                records(k0);
+                const float2 ABa = ld32(ab2, trow + (unsigned)tja);
+                const float2 ABb = ld32(ab2, trow + (unsigned)tjb);
+                float dxa = aja.x - ai.x, dya = aja.y - ai.y, dza = aja.z - ai.z;
+                float dxb = ajb.x - ai.x, dyb = ajb.y - ai.y, dzb = ajb.z - ai.z;
                 win_disp<ORTHO>(dxa, dya, dza, box);
                 win_disp<ORTHO>(dxb, dyb, dzb, box);
                 const float r2a = (dxa * dxa + dya * dya) + dza * dza;
                 const float r2b = (dxb * dxb + dyb * dyb) + dzb * dzb;
-                // keep the parameter gathers ahead of the branches (an empty
-                // statement that reads the registers; nothing is emitted)
+                // keep the parameter gathers ahead of the branches (the
+                // compiler would otherwise sink them into the branches, where
+                // their latency is not hidden behind the distance test); an
+                // empty statement that reads the registers, nothing is emitted
                 asm volatile("" ::"v"(ABa.x), "v"(ABa.y), "v"(ABb.x), "v"(ABb.y));
-                if (cur.sla >= 0 && r2a < rc2)
-                    win_pair<false, false>(S, dxa, dya, dza, r2a, ABa.x, ABa.y, qi2, cur.aja.w,
-                                           beta, cscale, ctab, cur.sla, cur.sja, ov, W.wcap, acc,
-                                           n, order, fx, 0, 0, e_sorted, v_sorted);
-                if (cur.slb >= 0 && r2b < rc2)
-                    win_pair<false, false>(S, dxb, dyb, dzb, r2b, ABb.x, ABb.y, qi2, cur.ajb.w,
-                                           beta, cscale, ctab, cur.slb, cur.sjb, ov, W.wcap, acc,
-                                           n, order, fx, 0, 0, e_sorted, v_sorted);
-                if (cK + 128 >= cRow.cnt)
-                {
-                    // the end of the row: its own force
-                    const int64_t sx = wave_sum(S.sx), sy = wave_sum(S.sy), sz = wave_sum(S.sz);
-                    if (lane == 0)
-                    {
-                        if (!ov)
-                        {
-                            const int ua = cRow.col / W.b, vb = cRow.col - ua * W.b;
-                            const int cz = cRow.cell % W.nz;
-                            const int k = snb_win_range_of(W, z0, ua, vb + 2, cz - z0 + 2);
-                            const int slot_i = rpref[k] + (cRow.si - rfirst[k]);
-                            // negated-force convention of the LDS accumulators
-                            atomicAdd((unsigned long long*)&acc[slot_i], (unsigned long long)(-sx));
-                            atomicAdd((unsigned long long*)&acc[W.wcap + slot_i],
-                                      (unsigned long long)(-sy));
-                            atomicAdd((unsigned long long*)&acc[2 * W.wcap + slot_i],
-                                      (unsigned long long)(-sz));
-                        }
-                        else
-                        {
-                            const int idi = order[cRow.si];
-                            atomic_add_i64(fx + idi, sx);
-                            atomic_add_i64(fx + n + idi, sy);
-                            atomic_add_i64(fx + 2 * n + idi, sz);
-                        }
-                    }
-                    S.sx = S.sy = S.sz = 0;
-                }
+                if (sla >= 0 && r2a < rc2)
+                    win_pair<NEED_ENERGY, NEED_VIRIAL>(S, dxa, dya, dza, r2a, ABa.x, ABa.y, qi2,
+                                                       aja.w, beta, cscale, ctab, sla, sja, ov,
+                                                       acc, n, order, fx, ref_attr, id_i,
+                                                       e_sorted, v_sorted);
+                if (slb >= 0 && r2b < rc2)
+                    win_pair<NEED_ENERGY, NEED_VIRIAL>(S, dxb, dyb, dzb, r2b, ABb.x, ABb.y, qi2,
+                                                       ajb.w, beta, cscale, ctab, slb, sjb, ov,
+                                                       acc, n, order, fx, ref_attr, id_i,
+                                                       e_sorted, v_sorted);
             }
-            cRow = nRow;
-            cK = nK;
-            nRow = eRow;
-            nK = eK;
-        };
-        while (true)
-        {
-            step(r0, r1, e1a, e1b, e2a, e2b);
-            if (cRow.si < 0) break;
-            step(r1, r0, e2a, e2b, e1a, e1b);
-            if (cRow.si < 0) break;
-        }
-    }
-    else
-    {
-        for (int col = 0; col < W.a * W.b; col++)
-        {
-            int ua = col / W.b, vb = col - ua * W.b;
-            if (x0 + ua >= W.nx || y0 + vb >= W.ny) continue;
-            int colbase = ((x0 + ua) * W.ny + (y0 + vb)) * W.nz;
-            int z1 = z0 + W.s < W.nz ? z0 + W.s : W.nz;
-            int r0 = start[colbase + z0], r1 = start[colbase + z1];
-            for (int si = r0 + wave; si < r1; si += nwave)
+            int64_t sx = wave_sum(S.sx), sy = wave_sum(S.sy), sz = wave_sum(S.sz);
+            int64_t elj = 0, ec = 0, v0 = 0, v1 = 0, v2 = 0, v3 = 0, v4 = 0, v5 = 0;
+            if (NEED_ENERGY)
             {
-                const int cnt = row_count[si], split = row_split[si];
-                const unsigned row0 = (unsigned)si * (unsigned)max_nb;  // n * max_nb < 2^31
-                const float4 ai = satom[si];
-                const float qi2 = ai.w * 4294967296.0f;  // 2^32 fixed-point scale
-                const unsigned trow = (unsigned)(stype[si] * ntypes);
-                const int id_i = (NEED_ENERGY || NEED_VIRIAL) && ref_attr ? order[si] : 0;
-                WinRowSums S = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-                // Software pipeline over 128-entry steps (two entries per lane):
-                // step k uses atoms whose records were fetched during step k - 1,
-                // fetches the records of step k + 1 (slot map, then position and
-                // type) and the list entries of step k + 2.  32-bit byte offsets:
-                // the loads take the scalar-base + vector-offset form.  Energy /
-                // virial variants fetch each step's records when it starts: their
-                // FP64 energies and row sums leave no registers for a second set
-                // of records, and a pipelined version spills.
-                constexpr bool PIPE = !(NEED_ENERGY || NEED_VIRIAL);
-                auto entry = [&](int k) -> int {
-                    return k < cnt ? (int)ld32(nl16, row0 + (unsigned)snb_row_entry(k, split, max_nb))
-                                   : -1;
-                };
-                auto sorted_of = [&](int sl) -> unsigned {
-                    return sl >= 0 ? (unsigned)win_slot_sorted(sl, ov, slot_s, rfirst, rpref, W.nrange)
-                                   : (unsigned)si;
-                };
-                int sla = 0, slb = 0, tja = 0, tjb = 0, nxa = 0, nxb = 0;
-                unsigned sja = 0, sjb = 0;
-                float4 aja = {0, 0, 0, 0}, ajb = {0, 0, 0, 0};
-                auto records = [&](int k) {
-                    sla = entry(k + lane);
-                    slb = entry(k + 64 + lane);
-                    sja = sorted_of(sla);
-                    sjb = sorted_of(slb);
-                    aja = ld32(satom, sja);
-                    ajb = ld32(satom, sjb);
-                    tja = ld32(stype, sja);
-                    tjb = ld32(stype, sjb);
-                };
-                if (PIPE)
+                elj = wave_sum(S.elj);
+                ec = wave_sum(S.ec);
+            }
+            if (NEED_VIRIAL)
+            {
+                v0 = wave_sum(S.v0); v1 = wave_sum(S.v1); v2 = wave_sum(S.v2);
+                v3 = wave_sum(S.v3); v4 = wave_sum(S.v4); v5 = wave_sum(S.v5);
+            }
+            if (lane == 0)
+            {
+                if (!ov)
                 {
-                    records(0);
-                    nxa = entry(lane + 128);
-                    nxb = entry(lane + 192);
+                    int cz = sorted_cell[si] % W.nz;
+                    int k = snb_win_range_of(W, z0, ua, vb + 2, cz - z0 + 2);
+                    int slot_i = rpref[k] + (si - rfirst[k]);
+                    // negated-force convention of the LDS accumulators
+                    lds_add3(acc, slot_i, -sx, -sy, -sz);
                 }
-                for (int k0 = 0; k0 < cnt; k0 += 128)
+                else
                 {
-                    if (!PIPE) records(k0);
-                    const float2 ABa = ld32(ab2, trow + (unsigned)tja);
-                    const float2 ABb = ld32(ab2, trow + (unsigned)tjb);
-                    // records of the next step
-                    int sla_n = 0, slb_n = 0, tja_n = 0, tjb_n = 0;
-                    unsigned sja_n = 0, sjb_n = 0;
-                    float4 aja_n = {0, 0, 0, 0}, ajb_n = {0, 0, 0, 0};
-                    if (PIPE)
-                    {
-                        sla_n = nxa;
-                        slb_n = nxb;
-                        sja_n = sorted_of(sla_n);
-                        sjb_n = sorted_of(slb_n);
-                        aja_n = ld32(satom, sja_n);
-                        ajb_n = ld32(satom, sjb_n);
-                        tja_n = ld32(stype, sja_n);
-                        tjb_n = ld32(stype, sjb_n);
-                        nxa = entry(k0 + 256 + lane);
-                        nxb = entry(k0 + 320 + lane);
-                    }
-                    float dxa = aja.x - ai.x, dya = aja.y - ai.y, dza = aja.z - ai.z;
-                    float dxb = ajb.x - ai.x, dyb = ajb.y - ai.y, dzb = ajb.z - ai.z;
-                    win_disp<ORTHO>(dxa, dya, dza, box);
-                    win_disp<ORTHO>(dxb, dyb, dzb, box);
-                    const float r2a = (dxa * dxa + dya * dya) + dza * dza;
-                    const float r2b = (dxb * dxb + dyb * dyb) + dzb * dzb;
-                    // keep the parameter gathers ahead of the branches (the
-                    // compiler would otherwise sink them into the branches, where
-                    // their latency is not hidden behind the distance test); an
-                    // empty statement that reads the registers, nothing is emitted
-                    asm volatile("" ::"v"(ABa.x), "v"(ABa.y), "v"(ABb.x), "v"(ABb.y));
-                    if (sla >= 0 && r2a < rc2)
-                        win_pair<NEED_ENERGY, NEED_VIRIAL>(S, dxa, dya, dza, r2a, ABa.x, ABa.y, qi2,
-                                                           aja.w, beta, cscale, ctab, sla, sja, ov,
-                                                           W.wcap, acc, n, order, fx, ref_attr, id_i,
-                                                           e_sorted, v_sorted);
-                    if (slb >= 0 && r2b < rc2)
-                        win_pair<NEED_ENERGY, NEED_VIRIAL>(S, dxb, dyb, dzb, r2b, ABb.x, ABb.y, qi2,
-                                                           ajb.w, beta, cscale, ctab, slb, sjb, ov,
-                                                           W.wcap, acc, n, order, fx, ref_attr, id_i,
-                                                           e_sorted, v_sorted);
-                    if (PIPE)
-                    {
-                        sla = sla_n;
-                        slb = slb_n;
-                        sja = sja_n;
-                        sjb = sjb_n;
-                        aja = aja_n;
-                        ajb = ajb_n;
-                        tja = tja_n;
-                        tjb = tjb_n;
-                    }
+                    int idi = order[si];
+                    atomic_add_i64(fx + idi, sx);
+                    atomic_add_i64(fx + n + idi, sy);
+                    atomic_add_i64(fx + 2 * n + idi, sz);
                 }
-                int64_t sx = wave_sum(S.sx), sy = wave_sum(S.sy), sz = wave_sum(S.sz);
-                int64_t elj = 0, ec = 0, v0 = 0, v1 = 0, v2 = 0, v3 = 0, v4 = 0, v5 = 0;
+                // other rows' lower-id terms may land on si as well
+                // (ref_attr: the arrays were cleared before the launch)
                 if (NEED_ENERGY)
                 {
-                    elj = wave_sum(S.elj);
-                    ec = wave_sum(S.ec);
-                }
-                if (NEED_VIRIAL)
-                {
-                    v0 = wave_sum(S.v0); v1 = wave_sum(S.v1); v2 = wave_sum(S.v2);
-                    v3 = wave_sum(S.v3); v4 = wave_sum(S.v4); v5 = wave_sum(S.v5);
-                }
-                if (lane == 0)
-                {
-                    if (!ov)
+                    if (ref_attr)
                     {
-                        int cz = sorted_cell[si] % W.nz;
-                        int k = snb_win_range_of(W, z0, ua, vb + 2, cz - z0 + 2);
-                        int slot_i = rpref[k] + (si - rfirst[k]);
-                        // negated-force convention of the LDS accumulators
-                        atomicAdd((unsigned long long*)&acc[slot_i], (unsigned long long)(-sx));
-                        atomicAdd((unsigned long long*)&acc[W.wcap + slot_i],
-                                  (unsigned long long)(-sy));
-                        atomicAdd((unsigned long long*)&acc[2 * W.wcap + slot_i],
-                                  (unsigned long long)(-sz));
+                        atomic_add_i64(e_sorted + si, elj);
+                        atomic_add_i64(e_sorted + (size_t)n + si, ec);
                     }
                     else
                     {
-                        int idi = order[si];
-                        atomic_add_i64(fx + idi, sx);
-                        atomic_add_i64(fx + n + idi, sy);
-                        atomic_add_i64(fx + 2 * n + idi, sz);
+                        e_sorted[si] = elj;
+                        e_sorted[(size_t)n + si] = ec;
                     }
-                    // other rows' lower-id terms may land on si as well
-                    // (ref_attr: the arrays were cleared before the launch)
-                    if (NEED_ENERGY)
+                }
+                if (NEED_VIRIAL)
+                {
+                    const int64_t vv[6] = {v0, v1, v2, v3, v4, v5};
+                    for (int c = 0; c < 6; c++)
                     {
                         if (ref_attr)
-                        {
-                            atomic_add_i64(e_sorted + si, elj);
-                            atomic_add_i64(e_sorted + (size_t)n + si, ec);
-                        }
+                            atomic_add_i64(v_sorted + (size_t)c * n + si, vv[c]);
                         else
-                        {
-                            e_sorted[si] = elj;
-                            e_sorted[(size_t)n + si] = ec;
-                        }
-                    }
-                    if (NEED_VIRIAL)
-                    {
-                        const int64_t vv[6] = {v0, v1, v2, v3, v4, v5};
-                        for (int c = 0; c < 6; c++)
-                        {
-                            if (ref_attr)
-                                atomic_add_i64(v_sorted + (size_t)c * n + si, vv[c]);
-                            else
-                                v_sorted[(size_t)c * n + si] = vv[c];
-                        }
+                            v_sorted[(size_t)c * n + si] = vv[c];
                     }
                 }
             }
         }
     }
     __syncthreads();
-    if (!NEED_ENERGY && !NEED_VIRIAL && jdirect)
+    // stage_base + total stays within the stage: it holds n x invmax slots
+    const size_t base = 3 * (size_t)stage_base[w];
+    for (int t = tid; t < 3 * total; t += blockDim.x)
     {
-        // force-only steps: the window's sums go straight to the id-ordered
-        // accumulators (integer sums, so the order of the adds does not
-        // matter); slots that received nothing are skipped
-        if (!ov)
-            for (int t = tid; t < total; t += blockDim.x)
-            {
-                const long long vx = acc[t], vy = acc[W.wcap + t], vz = acc[2 * W.wcap + t];
-                if ((vx | vy | vz) == 0) continue;
-                const int id = order[slot_s[t]];
-                if (vx) atomic_add_i64(fx + id, -vx);
-                if (vy) atomic_add_i64(fx + n + id, -vy);
-                if (vz) atomic_add_i64(fx + 2 * n + id, -vz);
-            }
-        return;
-    }
-    const int base = stage_base[w];
-    for (int t = tid; t < total; t += blockDim.x)
-    {
-        if ((size_t)(base + t) >= stage_cap) break;  // cannot happen: stage holds n x invmax
-        long long* dst = stage + 3 * (size_t)(base + t);
-        dst[0] = ov ? 0 : -acc[t];
-        dst[1] = ov ? 0 : -acc[W.wcap + t];
-        dst[2] = ov ? 0 : -acc[2 * W.wcap + t];
+        if (base + t >= 3 * stage_cap) break;
+        stage[base + t] = ov ? 0 : -acc[t];
     }
 }
 
-template <bool NEED_ENERGY, bool NEED_VIRIAL, bool ORTHO, bool STREAM>
-__global__ void __launch_bounds__(1024) k_pair_win(
+template <bool NEED_ENERGY, bool NEED_VIRIAL, bool ORTHO>
+__global__ void __launch_bounds__(1024) k_pair_ev(
     int n, SnbWin W, const int* __restrict__ start, const int* __restrict__ sorted_cell,
     const int* __restrict__ row_count, const int* __restrict__ row_split,
     const uint16_t* __restrict__ nl16, int max_nb,
@@ -1378,15 +1605,15 @@ __global__ void __launch_bounds__(1024) k_pair_win(
     const float4* __restrict__ coul_tab, float cscale, SnbBox box, float rc2, float beta,
     const int* __restrict__ stage_base, long long* __restrict__ stage, size_t stage_cap,
     int64_t* __restrict__ fx, int64_t* __restrict__ e_sorted, int64_t* __restrict__ v_sorted,
-    int ref_attr, const int* __restrict__ perm, int jdirect)
+    int ref_attr, const int* __restrict__ perm)
 {
-    k_pair_win_body<NEED_ENERGY, NEED_VIRIAL, ORTHO, STREAM>(
+    k_pair_ev_body<NEED_ENERGY, NEED_VIRIAL, ORTHO>(
         n, W, start, sorted_cell, row_count, row_split, nl16, max_nb, satom, stype, order, ab2,
         ntypes, coul_tab, cscale, box, rc2, beta, stage_base, stage, stage_cap, fx, e_sorted,
-        v_sorted, ref_attr, perm, jdirect, blockIdx.x, gridDim.x);
+        v_sorted, ref_attr, perm, blockIdx.x, gridDim.x);
 }
 
-struct PairWinArgs
+struct PairEvArgs
 {
     int n;
     SnbWin W;
@@ -1414,19 +1641,17 @@ struct PairWinArgs
     int64_t* v_sorted;
     int ref_attr;
     const int* perm;
-    int jdirect;
 };
 
-template <bool NEED_ENERGY, bool NEED_VIRIAL, bool ORTHO, bool STREAM>
-__global__ void __launch_bounds__(1024) k_pair_win_batch(SnbSegTab t)
+template <bool NEED_ENERGY, bool NEED_VIRIAL, bool ORTHO>
+__global__ void __launch_bounds__(1024) k_pair_ev_batch(SnbSegTab t)
 {
     unsigned bid, nbid;
-    const PairWinArgs& a = snb_seg<PairWinArgs>(t, bid, nbid);
-    k_pair_win_body<NEED_ENERGY, NEED_VIRIAL, ORTHO, STREAM>(
+    const PairEvArgs& a = snb_seg<PairEvArgs>(t, bid, nbid);
+    k_pair_ev_body<NEED_ENERGY, NEED_VIRIAL, ORTHO>(
         a.n, a.W, a.start, a.sorted_cell, a.row_count, a.row_split, a.nl16, a.max_nb, a.satom,
         a.stype, a.order, a.ab2, a.ntypes, a.coul_tab, a.cscale, a.box, a.rc2, a.beta, a.stage_base,
-        a.stage, a.stage_cap, a.fx, a.e_sorted, a.v_sorted, a.ref_attr, a.perm, a.jdirect, bid,
-        nbid);
+        a.stage, a.stage_cap, a.fx, a.e_sorted, a.v_sorted, a.ref_attr, a.perm, bid, nbid);
 }
 
 // Per sorted atom: sum of its stage entries into the id-ordered accumulators
@@ -1524,16 +1749,11 @@ int snb_launch_lj_window(snb_context* ctx, const snb_vector* crd, const float* c
     if (L.win_lds_set != lds)
     {
         // dynamic LDS above 64 KiB is granted per kernel
-        const void* fns[10] = {(const void*)k_pair_win<true, true, true, false>,
-                               (const void*)k_pair_win<true, false, true, false>,
-                               (const void*)k_pair_win<false, true, true, false>,
-                               (const void*)k_pair_win<false, false, true, false>,
-                               (const void*)k_pair_win<false, false, true, true>,
-                               (const void*)k_pair_win<true, true, false, false>,
-                               (const void*)k_pair_win<true, false, false, false>,
-                               (const void*)k_pair_win<false, true, false, false>,
-                               (const void*)k_pair_win<false, false, false, false>,
-                               (const void*)k_pair_win<false, false, false, true>};
+        const void* fns[8] = {
+            (const void*)k_pair_win<true>, (const void*)k_pair_win<false>,
+            (const void*)k_pair_ev<true, true, true>, (const void*)k_pair_ev<true, false, true>,
+            (const void*)k_pair_ev<false, true, true>, (const void*)k_pair_ev<true, true, false>,
+            (const void*)k_pair_ev<true, false, false>, (const void*)k_pair_ev<false, true, false>};
         for (const void* f : fns)
             SNB_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         L.win_lds_set = lds;
@@ -1558,46 +1778,39 @@ int snb_launch_lj_window(snb_context* ctx, const snb_vector* crd, const float* c
         return rc;
     if (ref_attr && need_virial && (rc = snb_launch_fill_i64(s, ctx->v_sorted, 6 * (size_t)n)))
         return rc;
-    // Force-only steps of large systems run the pipeline across row ends
-    // (STREAM): at 1M atoms the pair kernel takes 2.15 instead of 2.34 ms.
-    // At 93k atoms it is also faster alone (160 vs 170 us), but the step is
-    // not: it holds more registers (87 vs 76 per lane), and the PME
-    // workgroups that run beside it get fewer slots (0.2729 vs 0.2697 ms per
-    // step).
-    const int stream_mode = ctx->lj.row_stream;
-    const bool stream = !need_energy && !need_virial &&
-                        (stream_mode > 0 || (stream_mode < 0 && n >= (1 << 18)));
     snb_prof_begin(ctx, SNB_PROF_PAIR);
     // recorded step batches: the work of a workgroup is its rows
     if (snb_rec) snb_rec->weight_next = (double)n / W.nblock;
-#define SNB_WIN_LAUNCH(E, V, O, ST)                                                             \
-    SNB_LAUNCH_B((k_pair_win<E, V, O, ST>), (k_pair_win_batch<E, V, O, ST>), PairWinArgs,       \
-                 dim3(W.nblock), dim3(1024), lds, s, n, W, L.cell_start, L.sorted_cell,        \
-                 L.row_count, L.row_split, L.nl16, L.max_nb, ctx->satom, ctx->stype, L.order,  \
-                 ctx->lj.ab2, ctx->lj.ntypes, ctx->lj.coul, ctx->lj.coul_scale, box, rc2, beta, \
-                 L.stage_base, L.stage, (size_t)n * L.invmax, ctx->fx, ctx->e_sorted,           \
-                 ctx->v_sorted, ref_attr, L.block_perm, jdirect)
-#define SNB_WIN_LAUNCH_EV(O)                     \
-    if (need_energy && need_virial)              \
-        SNB_WIN_LAUNCH(true, true, O, false);    \
-    else if (need_energy)                        \
-        SNB_WIN_LAUNCH(true, false, O, false);   \
-    else if (need_virial)                        \
-        SNB_WIN_LAUNCH(false, true, O, false);   \
-    else if (stream)                             \
-        SNB_WIN_LAUNCH(false, false, O, true);   \
-    else                                         \
-        SNB_WIN_LAUNCH(false, false, O, false);
+#define SNB_EV_LAUNCH(E, V, O)                                                                   \
+    SNB_LAUNCH_B((k_pair_ev<E, V, O>), (k_pair_ev_batch<E, V, O>), PairEvArgs, dim3(W.nblock),   \
+                 dim3(1024), lds, s, n, W, L.cell_start, L.sorted_cell, L.row_count,             \
+                 L.row_split, L.nl16, L.max_nb, ctx->satom, ctx->stype, L.order, ctx->lj.ab2,    \
+                 ctx->lj.ntypes, ctx->lj.coul, ctx->lj.coul_scale, box, rc2, beta, L.stage_base, \
+                 L.stage, (size_t)n * L.invmax, ctx->fx, ctx->e_sorted, ctx->v_sorted, ref_attr, \
+                 L.block_perm)
+#define SNB_WIN_LAUNCH(O)                                                                       \
+    if (need_energy && need_virial)                                                             \
+        SNB_EV_LAUNCH(true, true, O);                                                           \
+    else if (need_energy)                                                                       \
+        SNB_EV_LAUNCH(true, false, O);                                                          \
+    else if (need_virial)                                                                       \
+        SNB_EV_LAUNCH(false, true, O);                                                          \
+    else                                                                                        \
+        SNB_LAUNCH_B(k_pair_win<O>, k_pair_win_batch<O>, PairWinArgs, dim3(W.nblock), dim3(1024), \
+                     lds, s, n, W.wcap, L.nl16, ctx->satom, ctx->stype, L.order, ctx->lj.ab2,    \
+                     ctx->lj.nolj, ctx->lj.ntypes, ctx->lj.coul, ctx->lj.coul_scale, box, rc2,   \
+                     beta, L.stage_base, L.wslots, L.units, L.unit_run, L.stage,                 \
+                     (size_t)n * L.invmax, ctx->fx, L.block_perm, jdirect);
     if (ortho)
     {
-        SNB_WIN_LAUNCH_EV(true)
+        SNB_WIN_LAUNCH(true)
     }
     else
     {
-        SNB_WIN_LAUNCH_EV(false)
+        SNB_WIN_LAUNCH(false)
     }
-#undef SNB_WIN_LAUNCH_EV
 #undef SNB_WIN_LAUNCH
+#undef SNB_EV_LAUNCH
     snb_prof_end(ctx, SNB_PROF_PAIR);
     SNB_CHECK(hipGetLastError());
     if (jdirect) return SNB_OK;

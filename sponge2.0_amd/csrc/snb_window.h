@@ -25,9 +25,19 @@
 
 #define SNB_WIN_MAX_RANGES 128
 // LDS of the pair kernel besides the per-slot arrays (28 bytes per slot: three
-// int64 accumulators and the slot -> atom map): the two range tables and the
+// int64 accumulators and the slot -> atom map): the two range tables (on
+// force-only steps the window's coordinate range in their place) and the
 // 256-piece Coulomb table (16 bytes a piece)
 #define SNB_WIN_FIXED_LDS (4 * (2 * SNB_WIN_MAX_RANGES + 1) + 16 * 256)
+
+// A unit of the pair kernel's work on force-only steps: up to 128 entries of
+// the near or the far part of one row, as int4 {row (sorted index), place of
+// its first 128 list entries counted from the spare entries before the list,
+// window slot of the row's own atom, entries | flags}.
+#define SNB_UNIT_FAR 256
+#define SNB_UNIT_LAST 512  // the row's last unit
+// first unit of each of a block's 16 wavefronts, and the end of the last one's
+#define SNB_UNIT_RUNS 17
 
 struct SnbWin
 {

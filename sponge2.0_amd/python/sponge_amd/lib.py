@@ -637,8 +637,8 @@ class Nonbonded:
         check(self.L.snb_lj_set_direct_j(self.ctx, int(mode)), "snb_lj_set_direct_j")
 
     def set_row_stream(self, mode):
-        """Force-only pair loop: 0 pipelined within each row, 1 across row
-        ends, -1 by system size (default)."""
+        """Force-only pair loop: 0, 1 or -1 (default); one loop, pipelined
+        across row ends, serves every mode."""
         check(self.L.snb_lj_set_row_stream(self.ctx, int(mode)), "snb_lj_set_row_stream")
 
     def set_row_lds(self, mode):
