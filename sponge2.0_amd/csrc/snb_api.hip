@@ -368,10 +368,13 @@ int snb_join_pme(snb_context* c)
 // read only coordinates, charges and module tables, so they may run beside
 // the direct-space kernels, on pme_stream ahead of the reciprocal pipeline,
 // adding into the reciprocal accumulator (fx_pme).  That balances the two
-// streams of a step; the integer sums are the same either way.
+// streams of a step; the integer sums are the same either way.  Below 65,536
+// atoms the reciprocal chain, a row of kernels bound by latency, is the longer
+// stream by far (60 us against 35 at 1,500 atoms), so there they stay with the
+// direct-space kernels; at 93,000 both streams take about 145 us.
 static bool side_ok(const snb_context* c, int need_energy, int need_virial, const void* d_frc)
 {
-    return c->overlap && c->pme_stream && !need_energy && !need_virial && !d_frc;
+    return c->overlap && c->pme_stream && !need_energy && !need_virial && !d_frc && c->n >= 65536;
 }
 
 // Points the context at pme_stream after the step's inputs are final (the

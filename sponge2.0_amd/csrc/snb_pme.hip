@@ -765,6 +765,54 @@ __global__ void __launch_bounds__(SNB_PLANE_THREADS) k_fft_plane_inv_batch(SnbSe
         a.spec, a.real, a.fy, a.fz, a.fc, a.plan_z, a.plan_y, a.twzg, a.twyg, bid, nbid);
 }
 
+// Forward plane pass of small grids: z R2C then y in one workgroup per
+// x-plane, the same line transforms as the two line kernels (results bit for
+// bit the same).  It saves a launch and its wait in the chain of dependent
+// kernels that a small system's step is bound by; larger planes would find no
+// LDS beside the direct-space kernel (rule at the launch).
+// LDS: tw_z[fz] | tw_y[fy] | A[cap] | B[cap], cap = max(fy*lsz, fc*lsy).
+__host__ __device__ static size_t plane_fwd_cap(int fy, int fz, int fc)
+{
+    size_t a = (size_t)fy * fft_ls(fz), b = (size_t)fc * fft_ls(fy);
+    return a > b ? a : b;
+}
+
+static size_t plane_fwd_lds(int fy, int fz, int fc)
+{
+    return sizeof(float2) * ((size_t)fz + fy + 2 * plane_fwd_cap(fy, fz, fc));
+}
+
+__global__ void __launch_bounds__(SNB_PLANE_THREADS) k_fft_plane_fwd(
+    const float* __restrict__ real, float2* __restrict__ spec, int fy, int fz, int fc,
+    SnbFftPlan plan_z, SnbFftPlan plan_y, const float2* __restrict__ twzg,
+    const float2* __restrict__ twyg)
+{
+    extern __shared__ float2 smem[];
+    const int cap = (int)plane_fwd_cap(fy, fz, fc);
+    float2* twz = smem;
+    float2* twy = twz + fz;
+    float2* A = twy + fy;
+    float2* B = A + cap;
+    load_twiddles(twz, twzg, fz);
+    load_twiddles(twy, twyg, fy);
+    const int x = blockIdx.x, lsy = fft_ls(fy), lsz = fft_ls(fz);
+    const float* in = real + (size_t)x * fy * fz;
+    float2* out = spec + (size_t)x * fy * fc;
+    float2* mid = fft_last_src(plan_z, A, B);
+    float2* res = mid == A ? B : A;
+    fft_run<-1, false>(
+        plan_z, fy, lsz, A, B, twzg, twz,
+        [=](int l, int i, int d) { return make_float2(at32(in + d, l * fz + i), 0.0f); },
+        [=](int l, int i, int d, float2 v) {
+            if (i + d < fc) res[(i + d) * lsy + l] = v;
+        });
+    __syncthreads();
+    fft_run<-1, true>(
+        plan_y, fc, lsy, mid, res, twyg, twy,
+        [=](int l, int i, int d) { return res[l * lsy + i + d]; },
+        [=](int l, int i, int d, float2 v) { at32(out + d * fc, i * fc + l) = v; });
+}
+
 // Fixed-order reduction of the per-block partials into dscal[0..6] and the
 // self + neutralising energy into dscal[7] (PM_force.cpp:1146-1159).
 __global__ void k_pme_finalize(const double* __restrict__ partials, int nblocks,
@@ -983,6 +1031,88 @@ __global__ void k_pme_scatter_batch(SnbSegTab t)
     unsigned bid, nbid;
     const PmeScatterArgs& a = snb_seg<PmeScatterArgs>(t, bid, nbid);
     k_pme_scatter_body(a.n, a.atom_u, a.slot, a.start, a.brick_atoms, bid, nbid);
+}
+
+// Small systems (n <= SNB_BIN_MAX_ATOMS, nbrick <= SNB_BIN_MAX_BRICKS): prep,
+// scan and scatter in one workgroup, brick counts in LDS and each thread's
+// atoms in its registers.  Three dependent launches of 3 to 4 us each become
+// one of 5 to 8 us.
+#define SNB_BIN_PER_THREAD 16
+#define SNB_BIN_MAX_ATOMS (1024 * SNB_BIN_PER_THREAD)
+#define SNB_BIN_MAX_BRICKS 4096
+__global__ void __launch_bounds__(1024) k_pme_bin(int n, const snb_vector* __restrict__ crd,
+                                                  const float* __restrict__ charge, SnbRc rc,
+                                                  int fx, int fy, int fz, int bx, int by, int bz,
+                                                  int nby, int nbz, int nbrick,
+                                                  int4* __restrict__ atom_u,
+                                                  float4* __restrict__ atom_fr,
+                                                  int* __restrict__ start,
+                                                  int* __restrict__ brick_atoms)
+{
+    __shared__ int hist[SNB_BIN_MAX_BRICKS];
+    __shared__ int wsum[16];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+#pragma unroll
+    for (int k = 0; k < SNB_BIN_MAX_BRICKS / 1024; k++) hist[k * 1024 + t] = 0;
+    __syncthreads();
+    int br[SNB_BIN_PER_THREAD], at[SNB_BIN_PER_THREAD];
+#pragma unroll
+    for (int k0 = 0; k0 < SNB_BIN_PER_THREAD; k0 += 4)
+    {
+        if (k0 * 1024 >= n) break;
+        float4 r[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+        {
+            const int i = (k0 + k) * 1024 + t;
+            const int j = i < n ? i : 0;
+            const snb_vector v = crd[j];
+            r[k] = make_float4(v.x, v.y, v.z, charge[j]);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+        {
+            const int i = (k0 + k) * 1024 + t;
+            br[k0 + k] = -1;
+            if (i >= n) continue;
+            int ux, uy, uz;
+            float a, b, c;
+            atom_near(r[k], rc.v, fx, fy, fz, ux, uy, uz, a, b, c);
+            const int q = ((ux / bx) * nby + uy / by) * nbz + uz / bz;
+            atom_u[i] = make_int4(ux, uy, uz, q);
+            atom_fr[i] = make_float4(a, b, c, r[k].w);
+            br[k0 + k] = q;
+            at[k0 + k] = atomicAdd(&hist[q], 1);
+        }
+    }
+    __syncthreads();
+    // exclusive scan: four bricks a thread, then the wavefronts' sums
+    int4 h = ((int4*)hist)[t];
+    const int sum = h.x + h.y + h.z + h.w;
+    int incl = sum;
+    for (int off = 1; off < 64; off <<= 1)
+    {
+        const int up = __shfl_up(incl, off);
+        if (lane >= off) incl += up;
+    }
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    int before = incl - sum;
+    for (int k = 0; k < wave; k++) before += wsum[k];
+    h = make_int4(before, before + h.x, before + h.x + h.y, before + h.x + h.y + h.z);
+    ((int4*)hist)[t] = h;
+    const int hk[4] = {h.x, h.y, h.z, h.w};
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        if (4 * t + k < nbrick) start[4 * t + k] = hk[k];
+    if (t == 0) start[nbrick] = n;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < SNB_BIN_PER_THREAD; k++)
+    {
+        if (k * 1024 >= n) break;
+        if (br[k] >= 0) brick_atoms[hist[br[k]] + at[k]] = k * 1024 + t;
+    }
 }
 
 __device__ __forceinline__ int wrap_axis(int v, int n) { return v < 0 ? v + n : v; }
@@ -1475,6 +1605,17 @@ int snb_launch_fft_r2c(snb_context* ctx, const float* real, float2* cplx)
 {
     SnbPme& P = ctx->pme;
     hipStream_t s = ctx->stream;
+    // A plane of at most 64 KB (60 x 60 points) takes one kernel.  Not in a
+    // recorded step batch, where members of all sizes share one dispatch per
+    // kernel and the line passes are the form that they have in common.
+    const size_t plds = plane_fwd_lds(P.fy, P.fz, P.fc);
+    if (plds <= 65536 && !snb_rec)
+    {
+        SNB_LAUNCH(k_fft_plane_fwd, dim3(P.fx), dim3(SNB_PLANE_THREADS), plds, s, real, cplx, P.fy,
+                   P.fz, P.fc, P.plan_z, P.plan_y, P.tw_z, P.tw_y);
+        SNB_CHECK(hipGetLastError());
+        return SNB_OK;
+    }
     // the forward transform runs while the direct-space kernel holds most of
     // the LDS: line passes with small LDS share compute units with it
     int nrow = P.fx * P.fy;
@@ -1564,8 +1705,15 @@ int snb_launch_pme_recip(snb_context* ctx, const snb_vector* crd, const float* c
     if (n > 0)
     {
         // brick counts are zero on entry (cleared at set-up and by the scan
-        // of the previous call)
-        if (P.nbrick <= SNB_PREP_HIST_MAX)
+        // of the previous call; the single binning kernel leaves them alone).
+        // Members of a recorded step batch keep the kernels that all sizes
+        // have in common.
+        const bool one = n <= SNB_BIN_MAX_ATOMS && P.nbrick <= SNB_BIN_MAX_BRICKS && !snb_rec;
+        if (one)
+            SNB_LAUNCH(k_pme_bin, dim3(1), dim3(1024), 0, s, n, crd, charge, r6, P.fx, P.fy, P.fz,
+                       P.bx, P.by, P.bz, P.nby, P.nbz, P.nbrick, P.atom_u, P.atom_fr,
+                       P.brick_start, P.brick_atoms);
+        else if (P.nbrick <= SNB_PREP_HIST_MAX)
             SNB_LAUNCH_B(k_pme_prep<true>, k_pme_prep_batch<true>, PmePrepArgs,
                          dim3((n + 255) / 256), dim3(256), 0, s, n, crd, charge, r6, P.fx, P.fy,
                          P.fz, P.bx, P.by, P.bz, P.nby, P.nbz, P.nbrick, P.brick_atoms, P.atom_u,
@@ -1575,10 +1723,13 @@ int snb_launch_pme_recip(snb_context* ctx, const snb_vector* crd, const float* c
                          dim3((n + 255) / 256), dim3(256), 0, s, n, crd, charge, r6, P.fx, P.fy,
                          P.fz, P.bx, P.by, P.bz, P.nby, P.nbz, P.nbrick, P.brick_atoms, P.atom_u,
                          P.atom_fr, P.atom_slot, P.brick_count);
-        if ((rc = snb_launch_exclusive_scan_clear(s, P.brick_count, P.brick_start, P.nbrick)))
-            return rc;
-        SNB_LAUNCH_B(k_pme_scatter, k_pme_scatter_batch, PmeScatterArgs, dim3((n + 255) / 256),
-                     dim3(256), 0, s, n, P.atom_u, P.atom_slot, P.brick_start, P.brick_atoms);
+        if (!one)
+        {
+            if ((rc = snb_launch_exclusive_scan_clear(s, P.brick_count, P.brick_start, P.nbrick)))
+                return rc;
+            SNB_LAUNCH_B(k_pme_scatter, k_pme_scatter_batch, PmeScatterArgs, dim3((n + 255) / 256),
+                         dim3(256), 0, s, n, P.atom_u, P.atom_slot, P.brick_start, P.brick_atoms);
+        }
     }
     else
     {
