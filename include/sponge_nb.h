@@ -74,7 +74,8 @@ int snb_context_create(snb_context** out, int device, void* hip_stream, int atom
 int snb_context_destroy(snb_context* ctx);
 int snb_set_stream(snb_context* ctx, void* hip_stream);
 /* Runs the PME reciprocal pipeline on a second, library-owned stream beside
- * the direct-space work (default 1).  It starts once the step's coordinates
+ * the direct-space work (default 1; systems of up to 8,192 atoms without
+ * windows keep to one stream).  It starts once the step's coordinates
  * are final -- at the last snb_nl_update, or at the reciprocal call when no
  * update came since the previous one -- and every later call that reads its
  * results (force flush, copies, energies, status) waits for it on the
@@ -196,13 +197,14 @@ int snb_lj_set_direct_j(snb_context* ctx, int mode);
  * reference). */
 int snb_lj_set_row_stream(snb_context* ctx, int mode);
 /* Force-only steps of the row kernel (the plain path, used when the windowed
- * path is off) for systems of at most 2,560 atoms: 1 = every atom's force
- * accumulators in LDS, one workgroup per 64 rows and one global add per
- * nonzero sum; 0 = global integer atomics per pair; -1 (default) = LDS only
- * while recording a step batch, where several small systems share the
- * device and the global atomics' throughput bounds the kernel (alone it is
- * bound by their latency, and the two measure the same).  Results are the
- * same either way (no counterpart in the reference). */
+ * path is off): -1 (default) = up to 8,192 atoms each atom sums the pairs of
+ * all its neighbours, of lower and of higher ids, without scattered adds
+ * (those are what bounds the other two forms); 0 = every pair once, global
+ * integer atomics for the higher id; 1 = every pair once, up to 2,560 atoms
+ * with every atom's accumulators in LDS, one workgroup per 64 rows and one
+ * global add per nonzero sum.  Larger systems and lists that are not the
+ * library's own take form 0.  Results are the same either way (no counterpart
+ * in the reference). */
 int snb_lj_set_row_lds(snb_context* ctx, int mode);
 /* Geometry of the windowed pair path (windowed = 0 when not used). */
 int snb_nl_window_info(snb_context* ctx, int* windowed, int* a, int* b, int* s, int* wcap,

@@ -101,6 +101,8 @@ void free_nl(SnbNl& L)
     dfree(L.sorted_id);
     dfree(L.sorted_crd);
     dfree(L.serial);
+    dfree(L.lo_rows);
+    dfree(L.lo_count);
     dfree(L.dnl);
     dfree(L.need);
     dfree(L.old_crd);
@@ -374,7 +376,7 @@ int snb_join_pme(snb_context* c)
 // direct-space kernels; at 93,000 both streams take about 145 us.
 static bool side_ok(const snb_context* c, int need_energy, int need_virial, const void* d_frc)
 {
-    return c->overlap && c->pme_stream && !need_energy && !need_virial && !d_frc && c->n >= 65536;
+    return snb_pme_side(c) && c->pme_stream && !need_energy && !need_virial && !d_frc && c->n >= 65536;
 }
 
 // Points the context at pme_stream after the step's inputs are final (the
@@ -690,6 +692,22 @@ static int setup_window(snb_context* c)
     return SNB_OK;
 }
 
+// Rows of lower ids of a small system's plain-path list (filled at rebuilds).
+static int setup_full_list(snb_context* c)
+{
+    SnbNl& L = c->nl;
+    const int n = c->n;
+    if (n <= 0 || n > SNB_FULL_MAX || L.lo_rows) return SNB_OK;
+    int rc = dalloc(&L.lo_rows, (size_t)n * n);
+    if (!rc) rc = dalloc(&L.lo_count, n);
+    if (rc)
+    {
+        dfree(L.lo_rows);
+        dfree(L.lo_count);
+    }
+    return rc;
+}
+
 // Find_Neighor_Grids_Device (neighbor_list.cpp:5-48) for a triclinic cell:
 // cell j is a neighbour of cell i when some periodic image (sx, sy, sz in
 // {-1, 0, 1}) puts j within [lx, 2] x [ly, 2] x [-2, 2] cells of i, an image
@@ -805,6 +823,11 @@ int snb_nl_initial(snb_context* c, float cutoff, float skin, snb_ltmatrix3 cell,
         free_nl(L);
         return rc;
     }
+    if (!L.windowed && (rc = setup_full_list(c)))
+    {
+        free_nl(L);
+        return rc;
+    }
     // ATOM_GROUP rows point into the padded table (neighbor_list.cpp:764-771)
     std::vector<snb_atom_group> h(n > 0 ? n : 1);
     for (int i = 0; i < n; i++)
@@ -847,7 +870,7 @@ int snb_nl_update(snb_context* c, const int* d_atom_local, int local_atom_number
     if (!d_ex_num && !c->has_excl) es = el = en = nullptr;
     // the step's coordinates are final here: the reciprocal pipeline of this
     // step may start from this point of the stream
-    if (c->overlap)
+    if (snb_pme_side(c))
     {
         SNB_CHECK(hipEventRecord(c->ev_inputs, c->stream));
         c->inputs_marked = true;
@@ -944,9 +967,11 @@ int snb_nl_set_window_shape(snb_context* c, int a, int b, int s)
     int rc = snb_join_pme(c);
     if (rc) return rc;
     SNB_CHECK(hipStreamSynchronize(c->stream));  // no launch in flight uses the old buffers
+    c->inputs_marked = false;  // the path decides whether the pipeline takes its own stream
+    c->pme_waits_inputs = false;
     free_window(L);
     L.built = false;  // the next snb_nl_update rebuilds for the new path
-    if (plain) return SNB_OK;
+    if (plain) return setup_full_list(c);
     L.win = W;
     return setup_window(c);
 }
@@ -1126,10 +1151,8 @@ int snb_lj_pme_direct_force(snb_context* c, int atom_numbers, int local_atom_num
         rc = snb_launch_lj_window(c, d_crd, d_charge, box, pme_beta, need_atom_energy,
                                   need_virial);
     else
-    {
-        if ((rc = snb_launch_pack_atoms(c, d_crd, d_charge))) return rc;
-        rc = snb_launch_lj_direct(c, d_nl, box, pme_beta, need_atom_energy, need_virial);
-    }
+        rc = snb_launch_lj_direct(c, d_nl, d_crd, d_charge, box, pme_beta, need_atom_energy,
+                                  need_virial);
     if (rc) return rc;
     if (d_frc && (rc = snb_launch_flush_forces(c, d_frc))) return rc;
     if (need_atom_energy)
@@ -1704,7 +1727,7 @@ int snb_pme_update_box(snb_context* c, snb_ltmatrix3 cell, snb_ltmatrix3 rcell, 
     if ((rc = snb_pme_compute_bc(c, snb_box(cell, rcell)))) return rc;
     // a pipeline of this step that was already cleared to start must also
     // see the new table
-    if (c->overlap && c->inputs_marked)
+    if (snb_pme_side(c) && c->inputs_marked)
     {
         SNB_CHECK(hipEventRecord(c->ev_inputs, c->stream));
         c->pme_waits_inputs = false;
@@ -1807,7 +1830,8 @@ int snb_pme_reciprocal_force(snb_context* c, const snb_vector* d_crd, snb_ltmatr
         // fx_pme / dscal / the Q slots, so it may run beside the direct-space
         // work: on pme_stream, after the step's inputs are final
         hipStream_t home = c->stream;
-        if (c->overlap)
+        const bool side = snb_pme_side(c);
+        if (side)
         {
             // ev_inputs is recorded after every earlier use of the reciprocal
             // accumulator on the context stream (a flush comes before the next
@@ -1829,7 +1853,7 @@ int snb_pme_reciprocal_force(snb_context* c, const snb_vector* d_crd, snb_ltmatr
             if (!rc)
                 rc = snb_launch_pme_recip(c, d_crd, d_charge, box, keep_energy, need_virial, 1);
         }
-        if (c->overlap)
+        if (side)
         {
             c->stream = home;
             if (!rc && hipEventRecord(c->ev_pme, c->pme_stream) != hipSuccess) rc = SNB_ERR_HIP;

@@ -36,6 +36,11 @@ enum SnbDoubleSlot
     SNB_D_COUNT = 8
 };
 
+// Largest system whose plain-path list is kept in both directions: 2 n^2 bytes,
+// 128 MiB here.  Faster than scattered adds over all of that range (1,500 atoms
+// 5.3 us against 25.4, 2,400 at 10 A 9.8 against 53.8, 3,900 9.9 against 38.1).
+#define SNB_FULL_MAX 8192
+
 // Atoms per cell the windowed list builder keeps row counts for in LDS.  The
 // windowed path is taken only when max_atom_in_grid_numbers is at most this
 // (the reference's default is 150), so its overflow flag keeps the meaning
@@ -68,7 +73,7 @@ struct SnbNl
     int refresh_interval = 0;
     int max_nb = 1200, max_in_cell = 150;
     int nx = 0, ny = 0, nz = 0, ncell = 0;
-    int* cell_count = nullptr;   // ncell + 1
+    int* cell_count = nullptr;   // ncell + 1; the last: set by a cut row of the plain path's list
     int* cell_start = nullptr;   // ncell + 1 (exclusive scan)
     int* atom_cell = nullptr;    // n
     int* atom_slot = nullptr;    // n
@@ -78,6 +83,10 @@ struct SnbNl
     int* sorted_cell = nullptr;  // n: cell of sorted position s
     int* serial = nullptr;       // n * max_nb
     snb_atom_group* dnl = nullptr;  // n
+    // small plain-path systems: each atom's neighbours with lower ids, the
+    // other half of the list (n * n, n)
+    uint16_t* lo_rows = nullptr;
+    int* lo_count = nullptr;
     int* need = nullptr;         // rebuild flag (device)
     snb_vector* old_crd = nullptr;
     // triclinic cell: each cell's neighbour cells from a table (the stencil
@@ -136,8 +145,9 @@ struct SnbLj
     // window forces of force-only steps: -1 by size, 0 through the stage and
     // its per-atom gather, 1 by atomic adds at the end of each block
     int j_direct = -1;
-    // force-only row kernel of small systems with LDS accumulators: -1 inside
-    // recorded step batches only, 0 never, 1 always
+    // force-only row kernel of small systems: -1 over the list in both
+    // directions (no scattered adds) where it is kept, 0 global atomics, 1 LDS
+    // accumulators
     int row_lds = -1;
 };
 
@@ -432,6 +442,17 @@ __device__ __forceinline__ const A& snb_seg(const SnbSegTab& t, unsigned& bid, u
     return *(const A*)(t.args + (size_t)s * t.stride);
 }
 
+// Whether the reciprocal pipeline runs on its own stream.  A system whose list
+// is kept in both directions has a direct-space part of under 10 us, less
+// than the fork and join of the second stream cost the step's launches (25
+// steps of 1,500 atoms in a graph 1431 us on one stream and 1570 on two, 2,400
+// atoms at 10 A 1501 and 1613); with windows the pair kernel is long enough
+// (9,000 atoms: 1949 and 1601).
+inline bool snb_pme_side(const snb_context* c)
+{
+    return c->overlap && (c->nl.windowed || !c->nl.lo_rows);
+}
+
 // A launch of a kernel without a batched form.
 #define SNB_LAUNCH(K, G, B, LDS, S, ...)                                                  \
     do                                                                                    \
@@ -522,8 +543,9 @@ int snb_launch_lj_window(snb_context* ctx, const snb_vector* crd, const float* c
                          const SnbBox& box, float beta, int need_energy, int need_virial);
 
 // pair kernel (snb_pair.hip)
-int snb_launch_lj_direct(snb_context* ctx, const snb_atom_group* nl, const SnbBox& box,
-                         float beta, int need_energy, int need_virial);
+int snb_launch_lj_direct(snb_context* ctx, const snb_atom_group* nl, const snb_vector* crd,
+                         const float* charge, const SnbBox& box, float beta, int need_energy,
+                         int need_virial);
 // k_excl on any stream and accumulators: fx [3][n], e_atom with the
 // correction energy in its third slot (e_atom[2n + i]), vir [6][n]
 int snb_launch_excl_to(hipStream_t s, int n, const snb_vector* crd, const float* charge,

@@ -303,6 +303,7 @@ __device__ __forceinline__ void k_nl_search_body(
     const int* __restrict__ ex_num, int max_nb, int* __restrict__ serial,
     snb_atom_group* __restrict__ nl, int* __restrict__ status,
     const int* __restrict__ nbr_cells, const int* __restrict__ nbr_count,
+    uint16_t* __restrict__ lo_rows, int* __restrict__ lo_count, int* __restrict__ cut,
     unsigned bid, unsigned nbid)
 {
     if (need[0] == 0) return;
@@ -343,9 +344,12 @@ __device__ __forceinline__ void k_nl_search_body(
         zr0[0] = 0; zr1[0] = nz - 1; nzr = 1;
     }
     int* row = serial + (size_t)i * max_nb;
-    int count = 0;
+    uint16_t* lo_row = lo_rows ? lo_rows + (size_t)i * n : nullptr;
+    int count = 0, lo = 0;
     const uint64_t lower = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    // the candidates p0 .. p1 - 1 in cell order: the pairs of i among them
+    // the candidates p0 .. p1 - 1 in cell order: the pairs of i among them.  A
+    // pair is decided as in the lower id's row: displacement from the higher
+    // to the lower id, the lower id's exclusions.
     auto scan = [&](int p0, int p1) {
         for (int base = p0; base < p1; base += 64)
         {
@@ -356,9 +360,15 @@ __device__ __forceinline__ void k_nl_search_body(
             {
                 float4 q = sorted_crd[p];
                 j = __float_as_int(q.w);
-                if (j > i)
+                if (j > i || (lo_row && j < i))
                 {
                     float dx = ri.x - q.x, dy = ri.y - q.y, dz = ri.z - q.z;
+                    if (j < i)
+                    {
+                        dx = -dx;
+                        dy = -dy;
+                        dz = -dz;
+                    }
                     float sx = (dx * box.rc[0] + dy * box.rc[1]) + dz * box.rc[3];
                     float sy = dy * box.rc[2] + dz * box.rc[4];
                     float sz = dz * box.rc[5];
@@ -368,7 +378,7 @@ __device__ __forceinline__ void k_nl_search_body(
                     dy = dy - (ky * box.c[2] + kz * box.c[4]);
                     dz = dz - kz * box.c[5];
                     ok = (dx * dx + dy * dy) + dz * dz < cs2;
-                    if (ok && j >= elo && j <= ehi)
+                    if (ok && j > i && j >= elo && j <= ehi)
                     {
                         for (int t = es; t < es + en; t++)
                             if (ex_list[t] == j)
@@ -377,15 +387,32 @@ __device__ __forceinline__ void k_nl_search_body(
                                 break;
                             }
                     }
+                    if (ok && j < i && ex_num)
+                    {
+                        const int jn = ex_num[j], js = ex_start[j];
+                        if (jn > 0 && i >= ex_list[js] && i <= ex_list[js + jn - 1])
+                            for (int t = js; t < js + jn; t++)
+                                if (ex_list[t] == i)
+                                {
+                                    ok = false;
+                                    break;
+                                }
+                    }
                 }
             }
-            uint64_t mask = __ballot(ok);
-            if (ok)
+            uint64_t mask = __ballot(ok && j > i);
+            if (ok && j > i)
             {
                 int slot = count + __popcll(mask & lower);
                 if (slot < max_nb) row[slot] = j;
             }
             count += __popcll(mask);
+            if (lo_row)
+            {
+                mask = __ballot(ok && j < i);
+                if (ok && j < i) lo_row[lo + __popcll(mask & lower)] = (uint16_t)j;
+                lo += __popcll(mask);
+            }
         }
     };
     if (nbr_cells)
@@ -407,7 +434,12 @@ __device__ __forceinline__ void k_nl_search_body(
     {
         nl[i].atom_numbers = count < max_nb ? count : max_nb;
         nl[i].ghost_numbers = 0;
-        if (count > max_nb) atomicOr(status, SNB_FLAG_NL_OVERFLOW);
+        if (count > max_nb)
+        {
+            atomicOr(status, SNB_FLAG_NL_OVERFLOW);
+            *cut = 1;
+        }
+        if (lo_row) lo_count[i] = lo;
     }
 }
 
@@ -418,11 +450,13 @@ __global__ void __launch_bounds__(256) k_nl_search(
     const int* __restrict__ ex_start, const int* __restrict__ ex_list,
     const int* __restrict__ ex_num, int max_nb, int* __restrict__ serial,
     snb_atom_group* __restrict__ nl, int* __restrict__ status,
-    const int* __restrict__ nbr_cells, const int* __restrict__ nbr_count)
+    const int* __restrict__ nbr_cells, const int* __restrict__ nbr_count,
+    uint16_t* __restrict__ lo_rows, int* __restrict__ lo_count, int* __restrict__ cut)
 {
     k_nl_search_body(
         need, n, crd, atom_cell, start, sorted_crd, box, cs2, nx, ny, nz, ex_start, ex_list, ex_num,
-        max_nb, serial, nl, status, nbr_cells, nbr_count, blockIdx.x, gridDim.x);
+        max_nb, serial, nl, status, nbr_cells, nbr_count, lo_rows, lo_count, cut,
+        blockIdx.x, gridDim.x);
 }
 
 struct NlSearchArgs
@@ -447,6 +481,9 @@ struct NlSearchArgs
     int* status;
     const int* nbr_cells;
     const int* nbr_count;
+    uint16_t* lo_rows;
+    int* lo_count;
+    int* cut;
 };
 
 __global__ void __launch_bounds__(256) k_nl_search_batch(SnbSegTab t)
@@ -456,7 +493,7 @@ __global__ void __launch_bounds__(256) k_nl_search_batch(SnbSegTab t)
     k_nl_search_body(
         a.need, a.n, a.crd, a.atom_cell, a.start, a.sorted_crd, a.box, a.cs2, a.nx, a.ny, a.nz,
         a.ex_start, a.ex_list, a.ex_num, a.max_nb, a.serial, a.nl, a.status, a.nbr_cells,
-        a.nbr_count, bid, nbid);
+        a.nbr_count, a.lo_rows, a.lo_count, a.cut, bid, nbid);
 }
 
 int snb_launch_nl_update(snb_context* ctx, const snb_vector* crd, const SnbBox& box, int forced,
@@ -502,7 +539,8 @@ int snb_launch_nl_update(snb_context* ctx, const snb_vector* crd, const SnbBox& 
         SNB_LAUNCH_B(k_nl_search, k_nl_search_batch, NlSearchArgs, dim3((n + 3) / 4), dim3(256), 0,
                      s, L.need, n, crd, L.atom_cell, L.cell_start, L.sorted_crd, box, L.cs2, L.nx,
                      L.ny, L.nz, ex_start, ex_list, ex_num, L.max_nb, L.serial, L.dnl, ctx->status,
-                     L.nbr_cells, L.nbr_count);
+                     L.nbr_cells, L.nbr_count, L.lo_rows, L.lo_count,
+                     L.cell_count + L.ncell);
     snb_prof_end(ctx, SNB_PROF_NL);
     SNB_CHECK(hipGetLastError());
     return SNB_OK;

@@ -274,8 +274,8 @@ __global__ void __launch_bounds__(256) k_lj_direct_batch(SnbSegTab t)
         a.fx, a.e_atom, a.vir, bid, nbid);
 }
 
-// Force-only steps of the row kernel for small systems: every atom's force
-// accumulators in LDS (3 x n int64, n <= SNB_LJ_LDS_MAX), each workgroup a
+// Force-only steps of the row kernel for small systems, on request: every
+// atom's force accumulators in LDS (3 x n int64, n <= SNB_LJ_LDS_MAX), each workgroup a
 // run of SNB_LJ_LDS_ROWS consecutive rows, and one global add per nonzero
 // sum at the end.  The same integer sums as the global atomics of
 // k_lj_direct, with about a quarter of the global atomics: where several
@@ -375,16 +375,176 @@ __global__ void __launch_bounds__(1024) k_lj_lds_batch(SnbSegTab t)
                   a.rc2, a.beta, a.fx, bid, nbid);
 }
 
-int snb_launch_lj_direct(snb_context* ctx, const snb_atom_group* nl, const SnbBox& box,
-                         float beta, int need_energy, int need_virial)
+// Force-only steps of the row kernel for small systems over the list in both
+// directions: a workgroup per atom i sums the pairs of all its neighbours, those
+// of lower ids with the displacement and sign of their own row's entry, so the
+// terms are the ones that k_lj_direct rounds and scatters, each evaluated on
+// both sides.  Twice the pair math (230 k pairs at 1,500 atoms: under 1 us of
+// the device) for none of its three 64-bit global atomics per pair, whose
+// throughput (about 31 per ns) is what bounds k_lj_direct.  Reads the caller's coordinates and
+// charges and the square parameter table: no packing kernel precedes it.  At
+// 1,500 atoms 25.4 us and 2 for packing -> 5.3 us.
+// A list with rows cut at max_nb (*cut) is taken in one direction with the
+// atomics, as k_lj_direct takes it.
+__device__ __forceinline__ void k_lj_full_body(
+    int n, const snb_atom_group* __restrict__ nl, const uint16_t* __restrict__ lo_rows,
+    const int* __restrict__ lo_count, const snb_vector* __restrict__ crd,
+    const float* __restrict__ charge, const int* __restrict__ type,
+    const float2* __restrict__ ab2, int ntypes, const float4* __restrict__ coul_tab, float cscale,
+    const SnbBox& box, float rc2, float beta, int64_t* __restrict__ fx,
+    const int* __restrict__ cut, int* __restrict__ status, unsigned bid)
+{
+    __shared__ float4 ctab[SNB_COUL_N];
+    __shared__ unsigned long long sum[3];
+    const int i = uni(bid), tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
+    const snb_atom_group g = nl[i];
+    const int lo_n = lo_count[i];
+    const bool both = *cut == 0;
+    const snb_vector ri = crd[i];
+    const float qi2 = charge[i] * 4294967296.0f;  // 2^32 fixed-point scale
+    const float2* abrow = ab2 + (size_t)type[i] * ntypes;
+    const uint16_t* lo_row = lo_rows + (size_t)i * n;
+    ctab[tid] = coul_tab[tid];
+    if (tid < 3) sum[tid] = 0;
+    if (tid == 0 &&
+        !(__builtin_isfinite(ri.x) && __builtin_isfinite(ri.y) && __builtin_isfinite(ri.z)))
+        atomicOr(status, SNB_FLAG_NONFINITE_CRD);
+    __syncthreads();
+    const int hi_n = g.atom_numbers, cnt = hi_n + (both ? lo_n : 0);
+    int64_t sx = 0, sy = 0, sz = 0;
+    for (int k0 = wave * 128; k0 < cnt; k0 += 512)
+    {
+        int jj[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+        {
+            const int k = k0 + 64 * h + lane;
+            jj[h] = k < hi_n ? g.atom_serial[k] : (k < cnt ? (int)lo_row[k - hi_n] : i);
+        }
+        snb_vector rj[2];
+        float qj[2];
+        int tj[2];
+        float2 AB[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+        {
+            rj[h] = crd[jj[h]];
+            qj[h] = charge[jj[h]];
+            tj[h] = type[jj[h]];
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++) AB[h] = abrow[tj[h]];
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+        {
+            const int j = jj[h];
+            float dx = rj[h].x - ri.x, dy = rj[h].y - ri.y, dz = rj[h].z - ri.z;
+            // the row of the lower id takes the displacement from it to the other
+            const bool lo = j < i;
+            if (lo)
+            {
+                dx = -dx;
+                dy = -dy;
+                dz = -dz;
+            }
+            pbc_disp(dx, dy, dz, box);
+            const float r2 = (dx * dx + dy * dy) + dz * dz;
+            if (j == i || !(r2 < rc2)) continue;
+            const float fa2 =
+                pair_force_factor(r2, AB[h].x, AB[h].y, qi2 * qj[h], beta, cscale, ctab);
+            const int64_t ix = snb_fixed_from_scaled(fa2 * dx),
+                          iy = snb_fixed_from_scaled(fa2 * dy),
+                          iz = snb_fixed_from_scaled(fa2 * dz);
+            const int64_t m = lo ? -1 : 0;  // the higher id's force: the negated integers
+            sx += (ix ^ m) - m;
+            sy += (iy ^ m) - m;
+            sz += (iz ^ m) - m;
+            if (!both)
+            {
+                atomic_add_i64(fx + j, -ix);
+                atomic_add_i64(fx + n + j, -iy);
+                atomic_add_i64(fx + 2 * n + j, -iz);
+            }
+        }
+    }
+    if (wave * 128 < cnt)
+    {
+        const int64_t v = wave_sum3(sx, sy, sz);
+        if ((lane & 15) == 0 && lane < 48)
+            atomicAdd(&sum[lane == 0 ? 0 : (lane == 32 ? 1 : 2)], (unsigned long long)v);
+    }
+    __syncthreads();
+    if (tid < 3) atomic_add_i64(fx + (size_t)tid * n + i, (int64_t)sum[tid]);
+}
+
+__global__ void __launch_bounds__(256) k_lj_full(
+    int n, const snb_atom_group* __restrict__ nl, const uint16_t* __restrict__ lo_rows,
+    const int* __restrict__ lo_count, const snb_vector* __restrict__ crd,
+    const float* __restrict__ charge, const int* __restrict__ type,
+    const float2* __restrict__ ab2, int ntypes, const float4* __restrict__ coul_tab, float cscale,
+    SnbBox box, float rc2, float beta, int64_t* __restrict__ fx, const int* __restrict__ cut,
+    int* __restrict__ status)
+{
+    k_lj_full_body(n, nl, lo_rows, lo_count, crd, charge, type, ab2, ntypes, coul_tab, cscale, box,
+                   rc2, beta, fx, cut, status, blockIdx.x);
+}
+
+struct LjFullArgs
+{
+    int n;
+    const snb_atom_group* nl;
+    const uint16_t* lo_rows;
+    const int* lo_count;
+    const snb_vector* crd;
+    const float* charge;
+    const int* type;
+    const float2* ab2;
+    int ntypes;
+    const float4* coul_tab;
+    float cscale;
+    SnbBox box;
+    float rc2;
+    float beta;
+    int64_t* fx;
+    const int* cut;
+    int* status;
+};
+
+__global__ void __launch_bounds__(256) k_lj_full_batch(SnbSegTab t)
+{
+    unsigned bid, nbid;
+    const LjFullArgs& a = snb_seg<LjFullArgs>(t, bid, nbid);
+    k_lj_full_body(a.n, a.nl, a.lo_rows, a.lo_count, a.crd, a.charge, a.type, a.ab2, a.ntypes,
+                   a.coul_tab, a.cscale, a.box, a.rc2, a.beta, a.fx, a.cut, a.status, bid);
+}
+
+int snb_launch_lj_direct(snb_context* ctx, const snb_atom_group* nl, const snb_vector* crd,
+                         const float* charge, const SnbBox& box, float beta, int need_energy,
+                         int need_virial)
 {
     int n = ctx->n;
     if (n <= 0) return SNB_OK;
     float rc2 = ctx->lj.cutoff * ctx->lj.cutoff;
-    // LDS accumulators: on request, or by default inside a recorded step batch
-    const int lds_mode = ctx->lj.row_lds;
-    if (!need_energy && !need_virial && n <= SNB_LJ_LDS_MAX &&
-        (lds_mode > 0 || (lds_mode < 0 && snb_rec)))
+    const int row_mode = ctx->lj.row_lds;
+    const bool force_only = !need_energy && !need_virial;
+    // both directions: the library's own list, kept that way by its rebuild
+    const SnbNl& L = ctx->nl;
+    if (force_only && row_mode < 0 && L.init && L.built && !L.windowed && L.lo_rows && nl == L.dnl)
+    {
+        snb_prof_begin(ctx, SNB_PROF_PAIR);
+        if (snb_rec) snb_rec->weight_next = (double)n;
+        SNB_LAUNCH_B(k_lj_full, k_lj_full_batch, LjFullArgs, dim3(n), dim3(256), 0, ctx->stream, n,
+                     nl, L.lo_rows, L.lo_count, crd, charge, ctx->type, ctx->lj.ab2,
+                     ctx->lj.ntypes, ctx->lj.coul, ctx->lj.coul_scale, box, rc2, beta, ctx->fx,
+                     L.cell_count + L.ncell, ctx->status);
+        snb_prof_end(ctx, SNB_PROF_PAIR);
+        SNB_CHECK(hipGetLastError());
+        return SNB_OK;
+    }
+    int rc = snb_launch_pack_atoms(ctx, crd, charge);
+    if (rc) return rc;
+    // LDS accumulators: on request, or for another list in a recorded step batch
+    if (force_only && n <= SNB_LJ_LDS_MAX && (row_mode > 0 || (row_mode < 0 && snb_rec)))
     {
         snb_prof_begin(ctx, SNB_PROF_PAIR);
         SNB_LAUNCH_B(k_lj_lds, k_lj_lds_batch, LjLdsArgs,

@@ -643,7 +643,8 @@ class Nonbonded:
 
     def set_row_lds(self, mode):
         """Row kernel of small systems on force-only steps: 1 LDS accumulators,
-        0 global atomics, -1 LDS only inside recorded step batches (snb_lj_set_row_lds)."""
+        0 global atomics, -1 (default) both directions of the list, no scattered
+        adds (snb_lj_set_row_lds)."""
         check(self.L.snb_lj_set_row_lds(self.ctx, int(mode)), "snb_lj_set_row_lds")
 
     def window_info(self):
