@@ -581,10 +581,10 @@ def main():
 
     if args.workload == "water1m":
         sysd = systems.config_water_1m()
-        # corner cells take the remainder of 215.24 / 6 A, about 1.9 times a
-        # cell width per axis, and hold about 145 atoms: the capacity key of
-        # the reference's neighbour list is raised from 150 to 256, the most
-        # the windowed list path takes
+        # the reference's corner cells take the remainder of 215.24 / 6 A, about
+        # 1.9 times a cell width per axis, and hold about 145 atoms: its
+        # capacity key is raised from 150 to 256, the most the windowed list
+        # path takes
         nb = lib.Nonbonded(sysd, refresh_interval=args.refresh, max_atom_in_grid_numbers=256)
     else:
         sysd = systems.config_gpu_93k()

@@ -104,7 +104,9 @@ int snb_set_exclusions(snb_context* ctx, const int* h_excluded_list_start,
  * resolved by the caller: neighbor_list_max_neighbor_numbers (default 1200),
  * neighbor_list_max_atom_in_grid_numbers (150), neighbor_list_refresh_interval
  * (0 = displacement criterion), neighbor_list_skin_permit (0.5).  Cells are
- * (cutoff+skin)/2 wide; boxes with < 3 cells on an axis return
+ * (cutoff+skin)/2 wide or, in an orthorhombic box, the even share of its axis
+ * above that (max_atom_in_grid_numbers then counts per (cutoff+skin)/2 cube);
+ * boxes with < 3 cells on an axis return
  * SNB_ERR_BOX_TOO_SMALL.  The windowed pair path (below) is chosen only when
  * max_atom_in_grid_numbers <= 256; a larger capacity keeps the plain path,
  * whose cells hold up to max_atom_in_grid_numbers atoms as the reference's.
@@ -126,10 +128,11 @@ int snb_nl_initial(snb_context* ctx, float cutoff, float skin, snb_ltmatrix3 cel
  * atom_local may be
  * NULL (identity); ghost_numbers must be 0.  The exclusion arrays may be NULL
  * when snb_set_exclusions was called.  The cell may differ from the initial
- * one (barostat steps): cells keep the initial width and the last cell of an
- * axis takes the remainder, as in the reference; a box smaller than the
- * initial cell count times that width returns SNB_ERR_BOX_TOO_SMALL
- * (re-initialise, as Main_Box_Change_Largely does). */
+ * one (barostat steps): the number of cells stays and they share each axis
+ * evenly (a triclinic cell keeps the initial width and its last cell takes the
+ * remainder, as in the reference); a box smaller than the initial cell count
+ * times the initial width returns SNB_ERR_BOX_TOO_SMALL (re-initialise, as
+ * Main_Box_Change_Largely does). */
 int snb_nl_update(snb_context* ctx, const int* d_atom_local, int local_atom_numbers,
                   int ghost_numbers, const snb_vector* d_crd, snb_ltmatrix3 cell,
                   snb_ltmatrix3 rcell, int step, int update,

@@ -5,6 +5,9 @@
 
 #include <algorithm>
 #include <cmath>
+#include <functional>
+#include <queue>
+#include <utility>
 #include <vector>
 
 #include "snb_internal.h"
@@ -135,21 +138,6 @@ void free_window(SnbNl& L)
     L.windowed = false;
 }
 
-// Chooses the block of the windowed pair path (snb_window.h): the largest
-// owned block whose expected window fills at most 75% of the LDS capacity and
-// that still gives at least min_blocks blocks (two per compute unit, so the
-// heaviest-first launch order can even out dense and sparse regions); when no
-// block gives that many, the largest that fits.  Needs >= 5 cells on every
-// axis (unique forward displacements).
-bool choose_window_pass(int nx, int ny, int nz, double atoms_per_cell, int max_lds,
-                        int min_blocks, SnbWin* W);
-bool choose_window(int nx, int ny, int nz, double atoms_per_cell, int max_lds, int min_blocks,
-                   SnbWin* W)
-{
-    return choose_window_pass(nx, ny, nz, atoms_per_cell, max_lds, min_blocks, W) ||
-           choose_window_pass(nx, ny, nz, atoms_per_cell, max_lds, 1, W);
-}
-
 // LDS slots of the largest window one workgroup can hold: 3 x int64
 // accumulator + an int slot map per slot, plus the fixed part
 static int window_slots_max(int max_lds)
@@ -191,19 +179,82 @@ static bool window_shape(int nx, int ny, int nz, int a, int b, int s, double ato
     return true;
 }
 
-bool choose_window_pass(int nx, int ny, int nz, double atoms_per_cell, int max_lds,
-                        int min_blocks, SnbWin* W)
+// Time of the windowed pair kernel with blocks of shape W, in pair
+// evaluations: the blocks, each its pairs, its window's atoms and a fixed part,
+// go heaviest first to the compute units.  Fitted to pair calls at 3,900 to
+// 200,000 atoms with 8 to 10 A, 7 to 15 shapes each: 4.3 us per block, 1.21 ns
+// per pair, 1.93 ns per window atom; root mean square error 8% wherever the
+// windows fit.
+static double window_time(const SnbWin& W, double atoms_per_cell, double pairs_per_atom, int num_cu)
 {
-    static const int cand[][3] = {{2, 2, 8}, {2, 2, 6}, {2, 2, 4}, {2, 2, 3}, {2, 2, 2},
-                                  {1, 2, 4}, {1, 1, 4}, {1, 1, 2}, {1, 1, 1}};
-    for (const auto& c : cand)
+    const double fixed = 3530.0, per_window_atom = 1.6;
+    const int n[3] = {W.nx, W.ny, W.nz}, sz[3] = {W.a, W.b, W.s}, halo[3] = {2, 4, 4};
+    std::vector<std::pair<double, long>> kinds;  // cost of a block, blocks of it
+    double total = 0.0;
+    for (int k = 0; k < 8; k++)
     {
-        int a = c[0], b = c[1], s = c[2];
-        long nblk = (long)((nx + a - 1) / a) * ((ny + b - 1) / b) * ((nz + s - 1) / s);
-        if (nblk < min_blocks) continue;
-        if (window_shape(nx, ny, nz, a, b, s, atoms_per_cell, max_lds, 0.75, W)) return true;
+        double cells = 1.0, window = 1.0;
+        long count = 1;
+        for (int d = 0; d < 3; d++)  // whole blocks of the axis or its partial last one
+        {
+            const int size = (k >> d & 1) ? n[d] % sz[d] : sz[d];
+            cells *= size;
+            window *= size + halo[d];
+            count *= (k >> d & 1) ? (n[d] % sz[d] ? 1 : 0) : n[d] / sz[d];
+        }
+        if (!count) continue;
+        kinds.push_back({fixed + (cells * pairs_per_atom + window * per_window_atom) * atoms_per_cell,
+                         count});
+        total += kinds.back().first * count;
     }
-    return false;
+    std::sort(kinds.rbegin(), kinds.rend());
+    if (W.nblock > 16 * num_cu) return total / num_cu + 0.5 * kinds[0].first;
+    std::priority_queue<double, std::vector<double>, std::greater<double>> cu;
+    for (int i = 0; i < num_cu; i++) cu.push(0.0);
+    double last = 0.0;
+    for (const auto& kind : kinds)
+        for (long i = 0; i < kind.second; i++)
+        {
+            const double end = cu.top() + kind.first;
+            cu.pop();
+            cu.push(end);
+            last = end > last ? end : last;
+        }
+    return last;
+}
+
+// Chooses the block of the windowed pair path (snb_window.h): among the shapes
+// whose expected window fills at most 60% of the LDS, the one of the shortest
+// modelled time.  Needs >= 5 cells on every axis (unique forward
+// displacements).  A pair call at 9,000 atoms and 10 A with 64 blocks of 2 x 2
+// x 2 takes 75.6 us and with 196 of 1 x 1 x 2 30.1; at 25,000 and 9 A 726 of 1
+// x 1 x 2 53.1 and 264 of 1 x 2 x 3 41.5.  Larger windows than that leave the
+// reciprocal pipeline's kernels, which run beside it, no LDS: ten steps of
+// 93,000 atoms take 2445 us with 2 x 2 x 4 (7 us faster by itself) and 2030
+// with 2 x 2 x 2, of 52,500 1585 with 1 x 2 x 4 and 1448 with 1 x 1 x 5.
+static bool choose_window(int nx, int ny, int nz, double atoms_per_cell, double pairs_per_atom,
+                          int max_lds, int num_cu, SnbWin* W)
+{
+    double best = 0.0;
+    bool found = false;
+    // dense cells, whose smallest window exceeds the 60%: up to 75%
+    for (double fill : {0.6, 0.75})
+    {
+        if (found) break;
+        for (int a = 2; a >= 1; a--)
+            for (int b = 2; b >= 1; b--)
+                for (int s = 1; s <= 8; s++)
+                {
+                    SnbWin V;
+                    if (!window_shape(nx, ny, nz, a, b, s, atoms_per_cell, max_lds, fill, &V)) continue;
+                    const double time = window_time(V, atoms_per_cell, pairs_per_atom, num_cu);
+                    if (found && time >= best) continue;
+                    best = time;
+                    *W = V;
+                    found = true;
+                }
+    }
+    return found;
 }
 
 // blocks whose window can contain one cell, per axis (+1 when a partial last
@@ -816,8 +867,10 @@ int snb_nl_initial(snb_context* c, float cutoff, float skin, snb_ltmatrix3 cell,
     // the windowed kernels address the list with 32-bit byte offsets; they
     // take orthorhombic cells
     L.windowed = !L.triclinic && window_list_fits(c) && max_atom_in_grid_numbers <= SNB_NLC_MAXA &&
-                 choose_window(L.nx, L.ny, L.nz, (double)n / L.ncell, c->max_lds, 2 * c->num_cu,
-                               &L.win);
+                 choose_window(L.nx, L.ny, L.nz, (double)n / L.ncell,
+                               2.0 * M_PI / 3.0 * cutoff * cutoff * cutoff * n /
+                                   ((double)cell.a11 * cell.a22 * cell.a33),
+                               c->max_lds, c->num_cu, &L.win);
     if (L.windowed && (rc = setup_window(c)))
     {
         free_nl(L);
@@ -854,10 +907,10 @@ int snb_nl_update(snb_context* c, const int* d_atom_local, int local_atom_number
     if (local_atom_numbers != c->n || (c->n > 0 && !d_crd)) return SNB_ERR_ARGUMENT;
     // a triclinic cell needs the neighbour-cell table made at snb_nl_initial
     if (!orthorhombic(cell) && !c->nl.triclinic) return SNB_ERR_UNSUPPORTED;
-    // cells keep the width of the initial box (grid_length) and the last one on
-    // each axis takes the remainder; a box that shrank below n cells of that
-    // width would leave a thinner cell and pairs beyond the +-2-cell stencil:
-    // re-initialise then (the reference does, main.cpp:880-884)
+    // the number of cells stays that of the initial box; a box that shrank below
+    // that many cells of grid_length would leave thinner cells and pairs beyond
+    // the +-2-cell stencil: re-initialise then (the reference does,
+    // main.cpp:880-884)
     if (cell.a11 < c->nl.nx * c->nl.grid_length || cell.a22 < c->nl.ny * c->nl.grid_length ||
         cell.a33 < c->nl.nz * c->nl.grid_length)
         return SNB_ERR_BOX_TOO_SMALL;

@@ -41,10 +41,8 @@ enum SnbDoubleSlot
 // 5.3 us against 25.4, 2,400 at 10 A 9.8 against 53.8, 3,900 9.9 against 38.1).
 #define SNB_FULL_MAX 8192
 
-// Atoms per cell the windowed list builder keeps row counts for in LDS.  The
-// windowed path is taken only when max_atom_in_grid_numbers is at most this
-// (the reference's default is 150), so its overflow flag keeps the meaning
-// "a cell held more than max_atom_in_grid_numbers atoms".
+// The windowed path is taken only when max_atom_in_grid_numbers is at most
+// this (the reference's default is 150).
 #define SNB_NLC_MAXA 256
 // neighbour cells per cell of a triclinic grid (MAX_GRID_NEIGHBORS, neighbor_list.cpp:3)
 #define SNB_NL_MAX_NBR 192
@@ -440,6 +438,15 @@ __device__ __forceinline__ const A& snb_seg(const SnbSegTab& t, unsigned& bid, u
     bid = (unsigned)(b - t.blk0[s]);
     nbid = (unsigned)(t.blk0[s + 1] - t.blk0[s]);
     return *(const A*)(t.args + (size_t)s * t.stride);
+}
+
+// Widths of the list's cells in this box (the last one of an axis takes a
+// triclinic cell's remainder).
+inline void snb_cell_widths(const SnbNl& L, const SnbBox& box, float w[3])
+{
+    w[0] = L.triclinic ? L.grid_length : box.c[0] / (float)L.nx;
+    w[1] = L.triclinic ? L.grid_length : box.c[2] / (float)L.ny;
+    w[2] = L.triclinic ? L.grid_length : box.c[5] / (float)L.nz;
 }
 
 // Whether the reciprocal pipeline runs on its own stream.  A system whose list

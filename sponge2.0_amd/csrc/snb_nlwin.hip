@@ -79,24 +79,34 @@ __device__ __forceinline__ void win_block_of_cell(const SnbWin& W, int c, int& c
     z0 = (cz / W.s) * W.s;
 }
 
-// Candidate capacity of one LDS chunk (the atoms per cell whose row counts
-// live in LDS, SNB_NLC_MAXA, are in snb_internal.h).
-// 1408 candidates (22 groups, 37 KB of LDS) hold a mean stencil of ~1,360
-// atoms at 6 A cells; four workgroups then fit a CU beside the reciprocal
-// pipeline's (1792 measured slower per step, though not alone)
+// Candidate capacity of one LDS chunk.  1408 candidates (22 groups, 32 KB of
+// LDS) hold a mean stencil of ~1,360 atoms at 6 A cells; four workgroups then
+// fit a CU beside the reciprocal pipeline's.
 #define SNB_NLC_CAP 1408
 #define SNB_NLC_MAXRUN 63
+#define SNB_NLC_WAVES 8
 
-// One 512-thread workgroup per cell.  The candidates of the cell's forward
-// stencil -- 13 columns of up to 5 cells, one run per cell, at most 63 runs
-// -- are staged in LDS once (in chunks of SNB_NLC_CAP) with their window
-// slots, and every atom of the cell tests them from LDS: wave w builds the
-// rows of atoms w, w + 8, ...  Candidate order is column, z (unwrapped), sorted
+// One 512-thread workgroup per cell.  The candidates are the cell's forward
+// stencil: 13 columns of up to 5 cells, one run per cell, at most 63 runs, in
+// chunks of SNB_NLC_CAP.  Candidate order is column, z (unwrapped), sorted
 // index, so a row lists its entries in that order; the first run is the cell
 // itself, where only larger sorted indices count.  For a diagonal box each
 // atom first marks the stencil cells whose box lies within the list radius
-// of its (wrapped) position, with a margin over float rounding, and skips the
-// groups of 64 candidates that lie in unmarked cells only.
+// of its (wrapped) position, with a margin over float rounding; groups of 64
+// candidates that lie in unmarked cells only are skipped for that atom.
+//
+// What bounds this kernel is the number of instructions per pair of (atom,
+// group).  A wavefront keeps a group of candidates in its lanes and goes over
+// the cell's atoms, whose positions are scalars; the two distance comparisons
+// are the ballots of the row's near and far entries, which lane a keeps for
+// atom a.  The minimum image is one shift per candidate wherever every atom of
+// the cell has the same one (rounding is monotone, so the extremes of the
+// cell's positions decide); where they differ the pair is folded by itself.
+// Row positions come from prefix sums of the ballots' counts over the groups,
+// then the wavefront writes its groups' entries.  About 45 instructions per
+// (atom, group), half of them scalar, where a wavefront per row took 85: 292 us
+// -> 262 at 45,000 atoms and 10 A while the widest cell set the time, 134 over
+// cells of equal width.
 //
 // The distance is taken as q_i - q_j for the row atom i.  The reference takes
 // it from the higher id to the lower; the two agree bit for bit (negation is
@@ -104,6 +114,53 @@ __device__ __forceinline__ void win_block_of_cell(const SnbWin& W, int c, int& c
 // i.e. where the minimum image is half a box away in that dimension.  With
 // >= 5 cells of >= (rc + skin)/2 per axis that is >= 1.25 (rc + skin), so
 // such a pair fails the test either way.
+#define SNB_NLC_GROUPS (SNB_NLC_CAP / 64)
+typedef float SnbF4 __attribute__((ext_vector_type(4)));
+typedef const SnbF4 __attribute__((address_space(4)))* SnbConstF4;
+
+__device__ __forceinline__ float readlane_f(float v, int l)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+// v of the lane that DPP control C names, the lane's own where that has none
+template <int C>
+__device__ __forceinline__ float dpp_f(float v)
+{
+    const int x = __float_as_int(v);
+    return __int_as_float(__builtin_amdgcn_update_dpp(x, x, C, 0xf, 0xf, false));
+}
+
+// smallest and largest of the wavefront's values (NaN left out)
+__device__ __forceinline__ float wave_fmin(float v)
+{
+    v = fminf(v, dpp_f<0x111>(v));  // row_shr 1, 2, 4, 8: rows of 16
+    v = fminf(v, dpp_f<0x112>(v));
+    v = fminf(v, dpp_f<0x114>(v));
+    v = fminf(v, dpp_f<0x118>(v));
+    v = fminf(v, dpp_f<0x142>(v));  // lane 15 of a row to the next row, then lane 31
+    v = fminf(v, dpp_f<0x143>(v));
+    return readlane_f(v, 63);
+}
+
+__device__ __forceinline__ float wave_fmax(float v) { return -wave_fmin(-v); }
+
+__device__ __forceinline__ int mbcnt(uint64_t mask)
+{
+    return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
+                                          __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+}
+
+// v with lane l's value replaced by the scalar x (no clang builtin names it)
+extern "C" __device__ unsigned snb_writelane(unsigned x, unsigned l, unsigned v) __asm(
+    "llvm.amdgcn.writelane.i32");
+
+__device__ __forceinline__ uint64_t lane_value(uint2 v, int l)
+{
+    return (uint64_t)(unsigned)__builtin_amdgcn_readlane((int)v.x, l) |
+           ((uint64_t)(unsigned)__builtin_amdgcn_readlane((int)v.y, l) << 32);
+}
+
 template <bool ORTHO>
 __device__ __forceinline__ void k_nl_build_cell_body(
     const int* __restrict__ need, SnbWin W, const int* __restrict__ start,
@@ -111,35 +168,27 @@ __device__ __forceinline__ void k_nl_build_cell_body(
     const int* __restrict__ ex_start, const int* __restrict__ ex_list,
     const int* __restrict__ ex_num, const int2* __restrict__ ex_rng, int max_nb, float near2,
     uint16_t* __restrict__ nl16, int* __restrict__ row_count, int* __restrict__ row_split,
-    int* __restrict__ status, float grid_length,
+    int* __restrict__ status, float wx, float wy, float wz,
     unsigned bid, unsigned nbid)
 {
     if (need[0] == 0) return;
     __shared__ int first[SNB_WIN_MAX_RANGES];
     __shared__ int pref[SNB_WIN_MAX_RANGES + 1];
-    __shared__ float4 cand[SNB_NLC_CAP];
-    __shared__ int2 cex[SNB_NLC_CAP];  // exclusion id window of each candidate
+    __shared__ uint4 masks[SNB_NLC_GROUPS][64];    // near and far ballots of (group, atom)
+    __shared__ uint16_t cnts[SNB_NLC_GROUPS][64];  // their counts: near | far << 8
     __shared__ uint16_t cslot[SNB_NLC_CAP];
+    __shared__ uint64_t reach_s[64];
     __shared__ int run_off[SNB_NLC_MAXRUN + 1];
     __shared__ int run_p0[SNB_NLC_MAXRUN];
     __shared__ int run_slot0[SNB_NLC_MAXRUN];
-    __shared__ int run_rel[SNB_NLC_MAXRUN];  // (dx + 2) << 6 | (dy + 2) << 3 | (dz + 2)
-    __shared__ int grp_r0[SNB_NLC_CAP / 64], grp_r1[SNB_NLC_CAP / 64];  // runs of each group
-    __shared__ int nrun_s;
-    __shared__ int rowcnt[SNB_NLC_MAXA];   // near pairs (front of the row)
-    __shared__ int rowfar[SNB_NLC_MAXA];   // skin pairs (back of the row)
     const int c = bid;
     const int cb = start[c], m = start[c + 1] - cb;
     if (m == 0) return;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int cz = c % W.nz, cy = (c / W.nz) % W.ny, cx = c / (W.nz * W.ny);
     const int x0 = (cx / W.a) * W.a, y0 = (cy / W.b) * W.b, z0 = (cz / W.s) * W.s;
     if (wave == 0) win_table_wave(W, start, x0, y0, z0, lane, first, pref);
-    for (int a = tid; a < SNB_NLC_MAXA; a += blockDim.x)
-    {
-        rowcnt[a] = 0;
-        rowfar[a] = 0;
-    }
     __syncthreads();
     if (pref[SNB_WIN_MAX_RANGES] > 65535)
     {
@@ -189,7 +238,6 @@ __device__ __forceinline__ void k_nl_build_cell_body(
             const int p0 = start[base + zw], p1 = start[base + zw + 1];
             run_p0[lane] = p0;
             run_slot0[lane] = pref[k] + (p0 - first[k]);
-            run_rel[lane] = ((dx + 2) << 6) | ((dy + 2) << 3) | (zu - cz + 2);
             size = p1 - p0;
         }
         int incl = size;
@@ -199,98 +247,140 @@ __device__ __forceinline__ void k_nl_build_cell_body(
             if (lane >= off) incl += up;
         }
         if (lane < SNB_NLC_MAXRUN) run_off[lane] = incl - size;
-        if (lane == SNB_NLC_MAXRUN - 1)
-        {
-            run_off[SNB_NLC_MAXRUN] = incl;
-            nrun_s = SNB_NLC_MAXRUN;
-        }
+        if (lane == SNB_NLC_MAXRUN - 1) run_off[SNB_NLC_MAXRUN] = incl;
     }
     __syncthreads();
-    const int nrun = nrun_s, total = run_off[nrun];
-    const uint64_t lower = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    for (int chunk0 = 0; chunk0 < total; chunk0 += SNB_NLC_CAP)
+    const int total = __builtin_amdgcn_readfirstlane(run_off[SNB_NLC_MAXRUN]);
+    const SnbConstF4 cell_crd = (SnbConstF4)(sorted_crd + cb);
+    // lane r: where run r lies in the stencil
+    const int rcol = lane < 3 ? 0 : 1 + (lane - 3) / 5;
+    const int rdx = rcol < 3 ? 0 : 1 + (rcol - 3) / 5;
+    const int rdy = rcol < 3 ? rcol : (rcol - 3) % 5 - 2;
+    const int rdz = lane < 3 ? lane : (lane - 3) % 5 - 2;
+    for (int a0 = 0; a0 < m; a0 += 64)
     {
-        const int clen = total - chunk0 < SNB_NLC_CAP ? total - chunk0 : SNB_NLC_CAP;
-        for (int t = tid; t < clen; t += blockDim.x)
+        const int ma = m - a0 < 64 ? m - a0 : 64;
+        // lane a: atom a0 + a of the cell
+        float4 qa = make_float4(__builtin_nanf(""), 0.0f, 0.0f, 0.0f);
+        qa.y = qa.z = qa.x;
+        int ilo = 0, iwid = 0;  // the id window of its exclusions
+        if (lane < ma)
         {
-            // the last run starting at or before g (empty runs share offsets)
-            const int g = chunk0 + t;
-            int lo = 0, hi = nrun - 1;
-            while (lo < hi)
+            qa = sorted_crd[cb + a0 + lane];
+            if (ex_num)
             {
-                const int mid = (lo + hi + 1) >> 1;
-                if (run_off[mid] <= g)
-                    lo = mid;
-                else
-                    hi = mid - 1;
+                const int2 r = ex_rng[__float_as_int(qa.w)];
+                ilo = r.x >= 0 ? r.x : ~r.x;
+                iwid = r.y - ilo + 1;
             }
-            const int r = lo;
-            int off = g - run_off[r];
-            float4 q = sorted_crd[run_p0[r] + off];
-            cand[t] = q;
-            cex[t] = ex_num ? ex_rng[__float_as_int(q.w)] : make_int2(1, 0);
-            cslot[t] = (uint16_t)(run_slot0[r] + off);
-            if ((t & 63) == 0) grp_r0[t >> 6] = r;
-            if ((t & 63) == 63 || t == clen - 1) grp_r1[t >> 6] = r;
         }
-        __syncthreads();
-        for (int a = wave; a < m && a < SNB_NLC_MAXA; a += (int)(blockDim.x >> 6))
+        // stencil cells within reach of atom a: per axis the gap from its
+        // wrapped position (the binning's arithmetic) to the cell, a lower
+        // bound of the minimum-image distance
+        for (int a = wave; a < ma; a += SNB_NLC_WAVES)
         {
-            const int s = cb + a;
-            const float4 qi = sorted_crd[s];
-            const int id_i = __float_as_int(qi.w);
-            const int2 rng_i = ex_num ? ex_rng[id_i] : make_int2(1, 0);
-            uint16_t* row = nl16 + (size_t)s * max_nb;
-            int count = rowcnt[a], cfar = rowfar[a];
-            // stencil cells within reach of atom i: per axis the gap from its
-            // wrapped position (the binning's arithmetic) to the cell, a lower
-            // bound of the minimum-image distance (the last cell of an axis
-            // is wider, which only lengthens the true gap)
             uint64_t reach = ~0ull;
             if (ORTHO)
             {
-                const float xw = qi.x - floorf(qi.x / box.c[0]) * box.c[0];
-                const float yw = qi.y - floorf(qi.y / box.c[2]) * box.c[2];
-                const float zw = qi.z - floorf(qi.z / box.c[5]) * box.c[5];
-                auto gap = [&](int d, int c, float w) -> float {
-                    float g = d > 0 ? (float)(c + d) * grid_length - w
-                                    : (d < 0 ? w - (float)(c + d + 1) * grid_length : 0.0f);
+                const float qx = readlane_f(qa.x, a), qy = readlane_f(qa.y, a),
+                            qz = readlane_f(qa.z, a);
+                const float xw = qx - floorf(qx / box.c[0]) * box.c[0];
+                const float yw = qy - floorf(qy / box.c[2]) * box.c[2];
+                const float zw = qz - floorf(qz / box.c[5]) * box.c[5];
+                auto gap = [](int d, int c, float x, float w) -> float {
+                    float g = d > 0 ? (float)(c + d) * w - x
+                                    : (d < 0 ? x - (float)(c + d + 1) * w : 0.0f);
                     return g > 0.0f ? g : 0.0f;
                 };
-                bool in = false;
-                if (lane < nrun)
-                {
-                    const int rel = run_rel[lane];
-                    const float gx = gap((rel >> 6) - 2, cx, xw);
-                    const float gy = gap(((rel >> 3) & 7) - 2, cy, yw);
-                    const float gz = gap((rel & 7) - 2, cz, zw);
-                    in = (gx * gx + gy * gy) + gz * gz < cs2 + 0.05f;
-                }
-                reach = __ballot(in);
+                const float gx = gap(rdx, cx, xw, wx), gy = gap(rdy, cy, yw, wy),
+                            gz = gap(rdz, cz, zw, wz);
+                reach = __ballot(lane < SNB_NLC_MAXRUN &&
+                                 (gx * gx + gy * gy) + gz * gz < cs2 + 0.05f);
             }
-            for (int t0 = 0; t0 < clen; t0 += 64)
+            if (lane == 0) reach_s[a] = reach;
+        }
+        const float lo3[3] = {wave_fmin(qa.x), wave_fmin(qa.y), wave_fmin(qa.z)};
+        const float hi3[3] = {wave_fmax(qa.x), wave_fmax(qa.y), wave_fmax(qa.z)};
+        __syncthreads();
+        const uint64_t reach_a = lane < ma ? reach_s[lane] : 0ull;
+        int near0 = 0, far0 = 0;  // the entries of row a so far
+        for (int chunk0 = 0; chunk0 < total; chunk0 += SNB_NLC_CAP)
+        {
+            const int clen = total - chunk0 < SNB_NLC_CAP ? total - chunk0 : SNB_NLC_CAP;
+            const int ngroup = (clen + 63) >> 6;
+            for (int k = wave; k < ngroup; k += SNB_NLC_WAVES)
             {
+                const int t = k * 64 + lane, g0 = chunk0 + k * 64;
+                const bool valid = t < clen;
+                // the last run starting at or before the candidate (empty runs
+                // share offsets)
+                const int g = valid ? g0 + lane : chunk0 + clen - 1;
+                int lo = 0, hi = SNB_NLC_MAXRUN - 1;
+                while (lo < hi)
                 {
-                    const int r0 = grp_r0[t0 >> 6], r1 = grp_r1[t0 >> 6];
-                    if (!(reach & (((2ull << (r1 - r0)) - 1ull) << r0))) continue;
+                    const int mid = (lo + hi + 1) >> 1;
+                    if (run_off[mid] <= g)
+                        lo = mid;
+                    else
+                        hi = mid - 1;
                 }
-                const int t = t0 + lane;
-                const int g = chunk0 + t;
-                bool ok = false, nearp = false;
-                // the cell's own atoms come first (g < m): larger sorted index only
-                if (t < clen && (g >= m || g > a))
+                const int off = g - run_off[lo];
+                const float4 qj = sorted_crd[run_p0[lo] + off];
+                const int id_j = __float_as_int(qj.w);
+                cslot[t] = (uint16_t)(run_slot0[lo] + off);
+                int jlo = 0, jwid = 0;
+                if (ex_num)
                 {
-                    const float4 qj = cand[t];
-                    const int id_j = __float_as_int(qj.w);
-                    float ddx = qi.x - qj.x, ddy = qi.y - qj.y, ddz = qi.z - qj.z;
-                    if (ORTHO)
+                    const int2 r = ex_rng[id_j];
+                    jlo = r.x >= 0 ? r.x : ~r.x;
+                    jwid = r.y - jlo + 1;
+                }
+                // the image shifts, where they are the same for the whole cell
+                const float qj3[3] = {qj.x, qj.y, qj.z};
+                float sh[3] = {0.0f, 0.0f, 0.0f};
+                bool same = ORTHO;
+                if (ORTHO)
+                {
+                    const float rc3[3] = {box.rc[0], box.rc[2], box.rc[5]};
+                    const float c3[3] = {box.c[0], box.c[2], box.c[5]};
+#pragma unroll
+                    for (int d = 0; d < 3; d++)
                     {
                         // rint(s) == floorf(s + 0.5) for every pair within
                         // rc + skin (s lies within (rc + skin)/L < 1/2 of an
                         // integer); they differ only half a box away
-                        float kx = rintf(ddx * box.rc[0]);
-                        float ky = rintf(ddy * box.rc[2]);
-                        float kz = rintf(ddz * box.rc[5]);
+                        const float k0 = rintf((lo3[d] - qj3[d]) * rc3[d]);
+                        const float k1 = rintf((hi3[d] - qj3[d]) * rc3[d]);
+                        same = same && k0 == k1;
+                        sh[d] = k0 * c3[d];
+                        asm volatile("" : "+v"(sh[d]));  // here, not once per atom
+                    }
+                }
+                const bool fold = __ballot(!same) != 0;
+                const int r0 = __builtin_amdgcn_readlane(lo, 0);
+                const int r1 = __builtin_amdgcn_readlane(lo, 63);
+                const uint64_t live = __ballot(valid);
+                const bool own = g0 < m;
+                uint64_t todo = __ballot((reach_a & (((2ull << (r1 - r0)) - 1ull) << r0)) != 0);
+                uint2 mnear = make_uint2(0u, 0u), mfar = make_uint2(0u, 0u);
+                while (todo)
+                {
+                    const int a = __builtin_ctzll(todo);
+                    todo &= todo - 1;
+                    const SnbF4 qi = cell_crd[a0 + a];
+                    const int id_i = __float_as_int(qi.w);
+                    float ddx = qi.x - qj.x, ddy = qi.y - qj.y, ddz = qi.z - qj.z;
+                    if (!fold)
+                    {
+                        ddx = ddx - sh[0];
+                        ddy = ddy - sh[1];
+                        ddz = ddz - sh[2];
+                    }
+                    else if (ORTHO)
+                    {
+                        const float kx = rintf(ddx * box.rc[0]);
+                        const float ky = rintf(ddy * box.rc[2]);
+                        const float kz = rintf(ddz * box.rc[5]);
                         ddx = ddx - kx * box.c[0];
                         ddy = ddy - ky * box.c[2];
                         ddz = ddz - kz * box.c[5];
@@ -307,78 +397,100 @@ __device__ __forceinline__ void k_nl_build_cell_body(
                         ddz = ddz - kz * box.c[5];
                     }
                     const float d2 = (ddx * ddx + ddy * ddy) + ddz * ddz;
-                    ok = d2 < cs2;
-                    nearp = d2 < near2;
+                    uint64_t ok = __ballot(d2 < cs2) & live;
+                    const uint64_t nearp = __ballot(d2 < near2);
+                    // the cell's own atoms come first: larger sorted index only
+                    if (own && g0 <= a0 + a)
+                    {
+                        const int skip = a0 + a - g0 + 1;
+                        ok = skip < 64 ? ok & (~0ull << skip) : 0ull;
+                    }
                     // the lower id's list decides; its id window rules out
                     // most pairs without touching the list, and decides alone
                     // for a list of consecutive ids (first stored >= 0)
-                    const int2 rl = id_i < id_j ? rng_i : cex[t];
-                    const int hi = id_i < id_j ? id_j : id_i;
-                    const int lo_id = rl.x >= 0 ? rl.x : ~rl.x;
-                    if (ok && hi >= lo_id && hi <= rl.y)
-                        ok = rl.x < 0 && !excluded_pair(id_i, id_j, ex_start, ex_list, ex_num);
-                }
-                // near pairs (within rc + skin/4, the ones that can come into
-                // range before the next rebuild) from the front, the rest from
-                // the back: the pair kernel meets them in that order and whole
-                // wavefronts of far pairs skip the force evaluation
-                const uint64_t mnear = __ballot(ok && nearp);
-                const uint64_t mfar = __ballot(ok && !nearp);
-                if (ok)
-                {
-                    if (nearp)
+                    const int wlo = __builtin_amdgcn_readlane(ilo, a);
+                    const int wwid = __builtin_amdgcn_readlane(iwid, a);
+                    const uint64_t maybe =
+                        (__ballot((unsigned)(id_j - wlo) < (unsigned)wwid) |
+                         __ballot((unsigned)(id_i - jlo) < (unsigned)jwid)) & ok;
+                    if (maybe)
                     {
-                        int pos = count + __popcll(mnear & lower);
-                        if (pos < max_nb) row[pos] = cslot[t];
+                        bool ex = false;
+                        if ((maybe >> lane) & 1)
+                        {
+                            const int lo_id = id_i < id_j ? id_i : id_j;
+                            const int hi_id = id_i < id_j ? id_j : id_i;
+                            const int2 rl = ex_rng[lo_id];
+                            if (hi_id >= (rl.x >= 0 ? rl.x : ~rl.x) && hi_id <= rl.y)
+                                ex = rl.x >= 0 ||
+                                     excluded_pair(id_i, id_j, ex_start, ex_list, ex_num);
+                        }
+                        ok &= ~__ballot(ex);
                     }
-                    else
-                    {
-                        int pos = cfar + __popcll(mfar & lower);
-                        if (pos < max_nb) row[max_nb - 1 - pos] = cslot[t];
-                    }
+                    const uint64_t mn = ok & nearp, mf = ok & ~nearp;
+                    mnear.x = snb_writelane((unsigned)mn, a, mnear.x);
+                    mnear.y = snb_writelane((unsigned)(mn >> 32), a, mnear.y);
+                    mfar.x = snb_writelane((unsigned)mf, a, mfar.x);
+                    mfar.y = snb_writelane((unsigned)(mf >> 32), a, mfar.y);
                 }
-                count += __popcll(mnear);
-                cfar += __popcll(mfar);
+                masks[k][lane] = make_uint4(mnear.x, mnear.y, mfar.x, mfar.y);
+                cnts[k][lane] = (uint16_t)((__popc(mnear.x) + __popc(mnear.y)) |
+                                           ((__popc(mfar.x) + __popc(mfar.y)) << 8));
             }
-            if (lane == 0)
+            __syncthreads();
+            // Near pairs (within rc + skin/4, the ones that can come into
+            // range before the next rebuild) from the front, the rest from
+            // the back: the pair kernel meets them in that order and whole
+            // wavefronts of far pairs skip the force evaluation.
+            for (int k = 0; k < ngroup; k++)
             {
-                rowcnt[a] = count;
-                rowfar[a] = cfar;
+                if (k % SNB_NLC_WAVES == wave)
+                {
+                    const uint4 mk = masks[k][lane];
+                    const int slot = cslot[k * 64 + lane];
+                    uint64_t todo = __ballot((mk.x | mk.y | mk.z | mk.w) != 0);
+                    while (todo)
+                    {
+                        const int a = __builtin_ctzll(todo);
+                        todo &= todo - 1;
+                        const uint64_t mn = lane_value(make_uint2(mk.x, mk.y), a);
+                        const uint64_t mf = lane_value(make_uint2(mk.z, mk.w), a);
+                        const int pn = __builtin_amdgcn_readlane(near0, a) + mbcnt(mn);
+                        const int pf = max_nb - 1 - __builtin_amdgcn_readlane(far0, a) - mbcnt(mf);
+                        const int pos = __builtin_amdgcn_inverse_ballot_w64(mn) ? pn : pf;
+                        if (__builtin_amdgcn_inverse_ballot_w64(mn | mf) &&
+                            (unsigned)pos < (unsigned)max_nb)
+                            nl16[(size_t)(cb + a0 + a) * max_nb + pos] = (uint16_t)slot;
+                    }
+                }
+                const int v = cnts[k][lane];
+                near0 += v & 255;
+                far0 += v >> 8;
             }
+            __syncthreads();
         }
-        __syncthreads();
-    }
-    for (int a = tid; a < m; a += blockDim.x)
-    {
-        if (a < SNB_NLC_MAXA)
+        if (wave == 0 && lane < ma)
         {
             // an overflowing row (flagged) keeps max_nb valid slots
-            int cn = rowcnt[a], cf = rowfar[a];
-            row_count[cb + a] = cn + cf < max_nb ? cn + cf : max_nb;
-            row_split[cb + a] = cn < max_nb ? cn : max_nb;
-            if (cn + cf > max_nb) atomicOr(status, SNB_FLAG_NL_OVERFLOW);
-        }
-        else
-        {
-            row_count[cb + a] = 0;
-            row_split[cb + a] = 0;
-            atomicOr(status, SNB_FLAG_CELL_OVERFLOW);
+            row_count[cb + a0 + lane] = near0 + far0 < max_nb ? near0 + far0 : max_nb;
+            row_split[cb + a0 + lane] = near0 < max_nb ? near0 : max_nb;
+            if (near0 + far0 > max_nb) atomicOr(status, SNB_FLAG_NL_OVERFLOW);
         }
     }
 }
 
 template <bool ORTHO>
-__global__ void __launch_bounds__(512) k_nl_build_cell(
+__global__ void __launch_bounds__(64 * SNB_NLC_WAVES, 8) k_nl_build_cell(
     const int* __restrict__ need, SnbWin W, const int* __restrict__ start,
     const float4* __restrict__ sorted_crd, SnbBox box, float cs2,
     const int* __restrict__ ex_start, const int* __restrict__ ex_list,
     const int* __restrict__ ex_num, const int2* __restrict__ ex_rng, int max_nb, float near2,
     uint16_t* __restrict__ nl16, int* __restrict__ row_count, int* __restrict__ row_split,
-    int* __restrict__ status, float grid_length)
+    int* __restrict__ status, float wx, float wy, float wz)
 {
     k_nl_build_cell_body<ORTHO>(
         need, W, start, sorted_crd, box, cs2, ex_start, ex_list, ex_num, ex_rng, max_nb, near2,
-        nl16, row_count, row_split, status, grid_length, blockIdx.x, gridDim.x);
+        nl16, row_count, row_split, status, wx, wy, wz, blockIdx.x, gridDim.x);
 }
 
 struct NlBuildCellArgs
@@ -399,17 +511,19 @@ struct NlBuildCellArgs
     int* row_count;
     int* row_split;
     int* status;
-    float grid_length;
+    float wx;
+    float wy;
+    float wz;
 };
 
 template <bool ORTHO>
-__global__ void __launch_bounds__(512) k_nl_build_cell_batch(SnbSegTab t)
+__global__ void __launch_bounds__(64 * SNB_NLC_WAVES, 8) k_nl_build_cell_batch(SnbSegTab t)
 {
     unsigned bid, nbid;
     const NlBuildCellArgs& a = snb_seg<NlBuildCellArgs>(t, bid, nbid);
     k_nl_build_cell_body<ORTHO>(
         a.need, a.W, a.start, a.sorted_crd, a.box, a.cs2, a.ex_start, a.ex_list, a.ex_num, a.ex_rng,
-        a.max_nb, a.near2, a.nl16, a.row_count, a.row_split, a.status, a.grid_length, bid, nbid);
+        a.max_nb, a.near2, a.nl16, a.row_count, a.row_split, a.status, a.wx, a.wy, a.wz, bid, nbid);
 }
 
 // The rows of the block at (x0, y0, z0), 64 at a time, column by column:
@@ -1213,18 +1327,20 @@ int snb_launch_nl_window(snb_context* ctx, const SnbBox& box, const int* ex_star
     SNB_LAUNCH_B(k_win_atoms, k_win_atoms_batch, WinAtomsArgs, dim3((n + 255) / 256), dim3(256), 0,
                  s, L.need, n, L.order, ctx->type, ctx->stype, L.inv_count, ex_start, ex_list,
                  ex_num, L.ex_rng);
+    float w[3];
+    snb_cell_widths(L, box, w);
     const bool ortho = box.c[1] == 0.0f && box.c[3] == 0.0f && box.c[4] == 0.0f &&
                        box.rc[1] == 0.0f && box.rc[3] == 0.0f && box.rc[4] == 0.0f;
     if (ortho)
         SNB_LAUNCH_B(k_nl_build_cell<true>, k_nl_build_cell_batch<true>, NlBuildCellArgs,
-                     dim3(L.ncell), dim3(512), 0, s, L.need, W, L.cell_start, L.sorted_crd, box,
+                     dim3(L.ncell), dim3(64 * SNB_NLC_WAVES), 0, s, L.need, W, L.cell_start, L.sorted_crd, box,
                      L.cs2, ex_start, ex_list, ex_num, L.ex_rng, L.max_nb, L.near2, L.nl16,
-                     L.row_count, L.row_split, ctx->status, L.grid_length);
+                     L.row_count, L.row_split, ctx->status, w[0], w[1], w[2]);
     else
         SNB_LAUNCH_B(k_nl_build_cell<false>, k_nl_build_cell_batch<false>, NlBuildCellArgs,
-                     dim3(L.ncell), dim3(512), 0, s, L.need, W, L.cell_start, L.sorted_crd, box,
+                     dim3(L.ncell), dim3(64 * SNB_NLC_WAVES), 0, s, L.need, W, L.cell_start, L.sorted_crd, box,
                      L.cs2, ex_start, ex_list, ex_num, L.ex_rng, L.max_nb, L.near2, L.nl16,
-                     L.row_count, L.row_split, ctx->status, L.grid_length);
+                     L.row_count, L.row_split, ctx->status, w[0], w[1], w[2]);
     SNB_LAUNCH_B(k_win_sizes, k_win_sizes_batch, WinSizesArgs, dim3(W.nblock), dim3(64), 0, s,
                  L.need, W, L.cell_start, L.row_count, L.row_split, L.win_size, L.unit_count,
                  L.block_work);

@@ -1921,16 +1921,19 @@ int snb_launch_lj_window(snb_context* ctx, const snb_vector* crd, const float* c
     // diagonal cell and rcell: the displacement skips the zero terms
     const bool ortho = box.c[1] == 0.0f && box.c[3] == 0.0f && box.c[4] == 0.0f &&
                        box.rc[1] == 0.0f && box.rc[3] == 0.0f && box.rc[4] == 0.0f;
-    // Force-only steps: the stage (about 430 bytes per atom at the preferred
-    // shapes) and its gather stay in the 256 MB last-level cache for
-    // mid-size systems, where they beat the blocks' atomic adds.  Past 128 MiB
-    // of stage the atomic adds are cheaper than the stage's HBM round trip;
-    // below 64k atoms the gather has too few workgroups to hide its chains
-    // of dependent loads (48 us at 2,100 atoms, against 17 us for the pair
-    // kernel), so the atomic adds win there too.
+    // Force-only steps: the blocks add their window forces to the accumulators
+    // by atomics, or write them to the stage (one slot per window atom) which
+    // k_stage_gather sums.  The stage pays only where its gather is wide enough
+    // and its slots are few: ten steps of 66,000 atoms at 10 A 1726 us through
+    // the stage and 1771 by atomics, 93,000 2030 and 2074; but 52,500 1620 and
+    // 1448, 81,000 with 27 slots per atom 2178 and 1905, 126,000 2995 and
+    // 2697, 200,000 3819 and 3667, 1,000,000 22340 and 19412.
     int jdirect = ctx->lj.j_direct;
     if (jdirect < 0)
-        jdirect = (n < 65536 || (size_t)n * 432 > ((size_t)128 << 20)) ? 1 : 0;
+    {
+        const bool few_slots = W.wu * W.wv * W.wz <= 22 * W.a * W.b * W.s;
+        jdirect = (n >= 65536 && n <= 98304 && few_slots) ? 0 : 1;
+    }
     if (need_energy || need_virial) jdirect = 0;
     const int ref_attr = ctx->lj.owner_attribution ? 0 : 1;
     int rc;

@@ -27,7 +27,7 @@ from . import autotune, systems
 from .lib import Nonbonded, StepBatch
 
 WATER_VOLUME = 29.915      # A^3 per TIP3P water at 1.0 g/cm^3
-MAX_ATOMS_IN_CELL = 256    # the largest per-cell capacity the windowed list builder keeps
+MAX_ATOMS_IN_CELL = 256    # the largest per-cell capacity that takes the windowed path
 BATCH_SHAPE = (2, 2, 2)    # window shape of windowed members of a step batch
 NS_PER_STEP = 2.0e-6       # 2 fs
 
@@ -70,10 +70,8 @@ class Segment:
         s = req.system()
         free0 = torch.cuda.mem_get_info()[0]
         self.stream = torch.cuda.Stream()
-        # the last cell of each axis takes the remainder of box / cell width
-        # and can be nearly twice as wide, so a corner cell can hold ~8x the
-        # mean occupancy (~17 atoms here): the per-cell capacity key is raised
-        # from its default of 150
+        # the per-cell capacity key is raised from its default of 150 to the
+        # most that takes the windowed path
         nb = Nonbonded(s, cutoff=s["cutoff"], refresh_interval=chunk, stream=self.stream,
                        max_atom_in_grid_numbers=MAX_ATOMS_IN_CELL)
         nb.set_pme_overlap(overlap)
