@@ -12,7 +12,7 @@ CASES = {
     "most_atoms": dict(waters=5461, box=54.7, grid=(56, 56, 56)),
     "more_atoms": dict(waters=5462, box=54.7, grid=(56, 56, 56)),
     "most_bricks": dict(waters=216, box=18.7, grid=(128, 128, 128)),
-    "more_bricks": dict(waters=216, box=18.7, grid=(128, 136, 128)),
+    "more_bricks": dict(waters=216, box=18.7, grid=(128, 140, 128)),
     "odd_planes": dict(waters=216, box=18.7, grid=(9, 49, 45)),
     "large_plane": dict(waters=216, box=18.7, grid=(16, 60, 60)),
     "larger_plane": dict(waters=216, box=18.7, grid=(16, 80, 64)),
