@@ -96,6 +96,8 @@ void free_nl(SnbNl& L)
 {
     dfree(L.nbr_cells);
     dfree(L.nbr_count);
+    dfree(L.nbr_of_cells);
+    dfree(L.nbr_of_count);
     L.triclinic = false;
     dfree(L.cell_count);
     dfree(L.cell_start);
@@ -749,6 +751,7 @@ static int setup_full_list(snb_context* c)
     SnbNl& L = c->nl;
     const int n = c->n;
     if (n <= 0 || n > SNB_FULL_MAX || L.lo_rows) return SNB_OK;
+    if (L.triclinic && !L.nbr_of_cells) return SNB_OK;
     int rc = dalloc(&L.lo_rows, (size_t)n * n);
     if (!rc) rc = dalloc(&L.lo_count, n);
     if (rc)
@@ -766,7 +769,11 @@ static int setup_full_list(snb_context* c)
 // sz nz, with the tilts in whole cells, (int)(a21 / grid_length) etc., and
 // lx = -3 (ly = -3) where the image moves x (y) by a tilt.  Each cell's list
 // in ascending cell order, as the reference's search over all cells finds it.
-static int triclinic_neighbour_cells(SnbNl& L, const snb_ltmatrix3& cell)
+// [-3, 2] holds for an image and for its opposite, so j may be a neighbour of i
+// and i none of j: a pair is in the list by the table of the lower id's cell
+// alone, and the rows of lower ids (`both`) are searched through the transposed
+// table, the cells that have cell i for a neighbour.
+static int triclinic_neighbour_cells(SnbNl& L, const snb_ltmatrix3& cell, bool both)
 {
     const int nx = L.nx, ny = L.ny, nz = L.nz, ncell = L.ncell;
     const int txy = (int)(cell.a21 / L.grid_length), txz = (int)(cell.a31 / L.grid_length),
@@ -810,6 +817,21 @@ static int triclinic_neighbour_cells(SnbNl& L, const snb_ltmatrix3& cell)
     SNB_CHECK(hipMemcpy(L.nbr_cells, cells.data(), sizeof(int) * cells.size(),
                         hipMemcpyHostToDevice));
     SNB_CHECK(hipMemcpy(L.nbr_count, count.data(), sizeof(int) * ncell, hipMemcpyHostToDevice));
+    if (!both) return SNB_OK;
+    std::vector<int> of((size_t)ncell * SNB_NL_MAX_NBR), of_count(ncell, 0);
+    for (int ci = 0; ci < ncell; ci++)
+        for (int k = 0; k < count[ci]; k++)
+        {
+            const int cj = cells[(size_t)ci * SNB_NL_MAX_NBR + k];
+            if (of_count[cj] == SNB_NL_MAX_NBR) return SNB_OK;  // the half list alone
+            of[(size_t)cj * SNB_NL_MAX_NBR + of_count[cj]++] = ci;
+        }
+    rc = dalloc(&L.nbr_of_cells, of.size());
+    if (!rc) rc = dalloc(&L.nbr_of_count, (size_t)ncell);
+    if (rc) return rc;
+    SNB_CHECK(hipMemcpy(L.nbr_of_cells, of.data(), sizeof(int) * of.size(), hipMemcpyHostToDevice));
+    SNB_CHECK(hipMemcpy(L.nbr_of_count, of_count.data(), sizeof(int) * ncell,
+                        hipMemcpyHostToDevice));
     return SNB_OK;
 }
 
@@ -859,7 +881,7 @@ int snb_nl_initial(snb_context* c, float cutoff, float skin, snb_ltmatrix3 cell,
         free_nl(L);
         return rc;
     }
-    if (L.triclinic && (rc = triclinic_neighbour_cells(L, cell)))
+    if (L.triclinic && (rc = triclinic_neighbour_cells(L, cell, n <= SNB_FULL_MAX)))
     {
         free_nl(L);
         return rc;

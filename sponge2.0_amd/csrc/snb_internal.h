@@ -92,6 +92,10 @@ struct SnbNl
     bool triclinic = false;
     int* nbr_cells = nullptr;  // ncell * SNB_NL_MAX_NBR
     int* nbr_count = nullptr;  // ncell
+    // the transposed table (cells that have cell c for a neighbour), where the
+    // rows of lower ids are kept
+    int* nbr_of_cells = nullptr;
+    int* nbr_of_count = nullptr;
     // windowed pair path (every axis >= 5 cells)
     bool windowed = false;
     int export_mode = 1;  // reference-layout list at rebuild: 0 no, 1 yes, 2 yes with sorted rows

@@ -314,6 +314,7 @@ __device__ __forceinline__ void k_nl_search_body(
     const int* __restrict__ ex_num, int max_nb, int* __restrict__ serial,
     snb_atom_group* __restrict__ nl, int* __restrict__ status,
     const int* __restrict__ nbr_cells, const int* __restrict__ nbr_count,
+    const int* __restrict__ nbr_of_cells, const int* __restrict__ nbr_of_count,
     uint16_t* __restrict__ lo_rows, int* __restrict__ lo_count, int* __restrict__ cut,
     unsigned bid, unsigned nbid)
 {
@@ -358,10 +359,11 @@ __device__ __forceinline__ void k_nl_search_body(
     uint16_t* lo_row = lo_rows ? lo_rows + (size_t)i * n : nullptr;
     int count = 0, lo = 0;
     const uint64_t lower = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    // the candidates p0 .. p1 - 1 in cell order: the pairs of i among them.  A
-    // pair is decided as in the lower id's row: displacement from the higher
-    // to the lower id, the lower id's exclusions.
-    auto scan = [&](int p0, int p1) {
+    // the candidates p0 .. p1 - 1 in cell order: the pairs of i among them, with
+    // higher ids (up) and with lower ids (down).  A pair is decided as in the
+    // lower id's row: displacement from the higher to the lower id, the lower
+    // id's exclusions, and the table of the lower id's cell.
+    auto scan = [&](int p0, int p1, bool up, bool down) {
         for (int base = p0; base < p1; base += 64)
         {
             int p = base + lane;
@@ -371,7 +373,7 @@ __device__ __forceinline__ void k_nl_search_body(
             {
                 float4 q = sorted_crd[p];
                 j = __float_as_int(q.w);
-                if (j > i || (lo_row && j < i))
+                if ((up && j > i) || (down && j < i))
                 {
                     float dx = ri.x - q.x, dy = ri.y - q.y, dz = ri.z - q.z;
                     if (j < i)
@@ -418,7 +420,7 @@ __device__ __forceinline__ void k_nl_search_body(
                 if (slot < max_nb) row[slot] = j;
             }
             count += __popcll(mask);
-            if (lo_row)
+            if (down)
             {
                 mask = __ballot(ok && j < i);
                 if (ok && j < i) lo_row[lo + __popcll(mask & lower)] = (uint16_t)j;
@@ -428,10 +430,17 @@ __device__ __forceinline__ void k_nl_search_body(
     };
     if (nbr_cells)
     {
-        // triclinic cell: the cell's neighbour cells from the table
+        // triclinic cell: the cell's neighbour cells from the table, and for
+        // lower ids the cells that have this one for a neighbour
         const int* tab = nbr_cells + (size_t)c * SNB_NL_MAX_NBR;
         const int m = nbr_count[c];
-        for (int k = 0; k < m; k++) scan(start[tab[k]], start[tab[k] + 1]);
+        for (int k = 0; k < m; k++) scan(start[tab[k]], start[tab[k] + 1], true, false);
+        if (lo_row)
+        {
+            const int* of = nbr_of_cells + (size_t)c * SNB_NL_MAX_NBR;
+            const int mo = nbr_of_count[c];
+            for (int k = 0; k < mo; k++) scan(start[of[k]], start[of[k] + 1], false, true);
+        }
     }
     else
         for (int a = 0; a < nxs; a++)
@@ -439,7 +448,7 @@ __device__ __forceinline__ void k_nl_search_body(
             {
                 int col = (xs[a] * ny + ys[bq]) * nz;
                 for (int zr = 0; zr < nzr; zr++)
-                    scan(start[col + zr0[zr]], start[col + zr1[zr] + 1]);
+                    scan(start[col + zr0[zr]], start[col + zr1[zr] + 1], true, lo_row != nullptr);
             }
     if (lane == 0)
     {
@@ -462,12 +471,13 @@ __global__ void __launch_bounds__(256) k_nl_search(
     const int* __restrict__ ex_num, int max_nb, int* __restrict__ serial,
     snb_atom_group* __restrict__ nl, int* __restrict__ status,
     const int* __restrict__ nbr_cells, const int* __restrict__ nbr_count,
+    const int* __restrict__ nbr_of_cells, const int* __restrict__ nbr_of_count,
     uint16_t* __restrict__ lo_rows, int* __restrict__ lo_count, int* __restrict__ cut)
 {
     k_nl_search_body(
         need, n, crd, atom_cell, start, sorted_crd, box, cs2, nx, ny, nz, ex_start, ex_list, ex_num,
-        max_nb, serial, nl, status, nbr_cells, nbr_count, lo_rows, lo_count, cut,
-        blockIdx.x, gridDim.x);
+        max_nb, serial, nl, status, nbr_cells, nbr_count, nbr_of_cells, nbr_of_count, lo_rows, lo_count,
+        cut, blockIdx.x, gridDim.x);
 }
 
 struct NlSearchArgs
@@ -492,6 +502,8 @@ struct NlSearchArgs
     int* status;
     const int* nbr_cells;
     const int* nbr_count;
+    const int* nbr_of_cells;
+    const int* nbr_of_count;
     uint16_t* lo_rows;
     int* lo_count;
     int* cut;
@@ -504,7 +516,7 @@ __global__ void __launch_bounds__(256) k_nl_search_batch(SnbSegTab t)
     k_nl_search_body(
         a.need, a.n, a.crd, a.atom_cell, a.start, a.sorted_crd, a.box, a.cs2, a.nx, a.ny, a.nz,
         a.ex_start, a.ex_list, a.ex_num, a.max_nb, a.serial, a.nl, a.status, a.nbr_cells,
-        a.nbr_count, a.lo_rows, a.lo_count, a.cut, bid, nbid);
+        a.nbr_count, a.nbr_of_cells, a.nbr_of_count, a.lo_rows, a.lo_count, a.cut, bid, nbid);
 }
 
 int snb_launch_nl_update(snb_context* ctx, const snb_vector* crd, const SnbBox& box, int forced,
@@ -558,8 +570,8 @@ int snb_launch_nl_update(snb_context* ctx, const snb_vector* crd, const SnbBox& 
         SNB_LAUNCH_B(k_nl_search, k_nl_search_batch, NlSearchArgs, dim3((n + 3) / 4), dim3(256), 0,
                      s, L.need, n, crd, L.atom_cell, L.cell_start, L.sorted_crd, box, L.cs2, L.nx,
                      L.ny, L.nz, ex_start, ex_list, ex_num, L.max_nb, L.serial, L.dnl, ctx->status,
-                     L.nbr_cells, L.nbr_count, L.lo_rows, L.lo_count,
-                     L.cell_count + L.ncell);
+                     L.nbr_cells, L.nbr_count, L.nbr_of_cells, L.nbr_of_count, L.lo_rows,
+                     L.lo_count, L.cell_count + L.ncell);
     snb_prof_end(ctx, SNB_PROF_NL);
     SNB_CHECK(hipGetLastError());
     return SNB_OK;
