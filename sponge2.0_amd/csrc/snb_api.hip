@@ -418,6 +418,17 @@ int snb_join_pme(snb_context* c)
     return SNB_OK;
 }
 
+// Where the stream of the reciprocal pipeline may change (overlap switched, a
+// list of another path): what it has queued comes first,
+// and the next call that takes a stream of its own records its inputs anew.  An
+// event kept from before would let it start ahead of the work queued since.
+static int leave_pme_stream(snb_context* c)
+{
+    c->inputs_marked = false;
+    c->pme_waits_inputs = false;
+    return snb_join_pme(c);
+}
+
 // Force-only work of the fused mode (no float output) that the reciprocal
 // stream takes over: the exclusion correction, the 1-4 pairs and the bonds
 // read only coordinates, charges and module tables, so they may run beside
@@ -632,7 +643,7 @@ int snb_set_pme_overlap(snb_context* c, int enable)
 {
     if (!c) return SNB_ERR_ARGUMENT;
     DeviceGuard g(c->device);
-    int rc = snb_join_pme(c);
+    int rc = leave_pme_stream(c);
     if (rc) return rc;
     c->overlap = enable != 0;
     return SNB_OK;
@@ -845,6 +856,8 @@ int snb_nl_initial(snb_context* c, float cutoff, float skin, snb_ltmatrix3 cell,
         return SNB_ERR_ARGUMENT;
     DeviceGuard g(c->device);
     SnbNl& L = c->nl;
+    int rc = leave_pme_stream(c);  // the new list's path decides whether the pipeline takes its own
+    if (rc) return rc;
     free_nl(L);
     L.triclinic = !orthorhombic(cell);
     L.cutoff = cutoff;
@@ -863,7 +876,6 @@ int snb_nl_initial(snb_context* c, float cutoff, float skin, snb_ltmatrix3 cell,
     if (L.nx <= 2 || L.ny <= 2 || L.nz <= 2) return SNB_ERR_BOX_TOO_SMALL;
     L.ncell = L.nx * L.ny * L.nz;
     int n = c->n;
-    int rc = SNB_OK;
     if (!rc) rc = dalloc(&L.cell_count, L.ncell + 1);
     if (!rc) rc = dalloc(&L.cell_start, L.ncell + 1);
     if (!rc) rc = dalloc(&L.atom_cell, n);
@@ -1039,11 +1051,9 @@ int snb_nl_set_window_shape(snb_context* c, int a, int b, int s)
     if (plain ? !L.windowed : (L.windowed && L.win.a == W.a && L.win.b == W.b && L.win.s == W.s))
         return SNB_OK;
     DeviceGuard g(c->device);
-    int rc = snb_join_pme(c);
+    int rc = leave_pme_stream(c);  // the path decides whether the pipeline takes its own
     if (rc) return rc;
     SNB_CHECK(hipStreamSynchronize(c->stream));  // no launch in flight uses the old buffers
-    c->inputs_marked = false;  // the path decides whether the pipeline takes its own stream
-    c->pme_waits_inputs = false;
     free_window(L);
     L.built = false;  // the next snb_nl_update rebuilds for the new path
     if (plain) return setup_full_list(c);
