@@ -62,7 +62,7 @@ typedef struct snb_context snb_context;
 /* sticky device flags (snb_read_status); the reference keeps the first three
  * as device ints but never reads them (neighbor_list.cpp:887-965) */
 #define SNB_FLAG_NL_OVERFLOW 1      /* a row exceeded max_neighbor_numbers; row truncated */
-#define SNB_FLAG_CELL_OVERFLOW 2    /* a cell held more than max_atom_in_grid_numbers atoms */
+#define SNB_FLAG_CELL_OVERFLOW 2    /* a grid held more than max_atom_in_grid_numbers atoms (snb_nl_initial) */
 #define SNB_FLAG_NONFINITE_CRD 4    /* a coordinate was NaN/Inf (PME uses 0 for it, PM_force.cpp:710-714) */
 
 int snb_abi_version(void);
@@ -105,9 +105,10 @@ int snb_set_exclusions(snb_context* ctx, const int* h_excluded_list_start,
  * neighbor_list_max_atom_in_grid_numbers (150), neighbor_list_refresh_interval
  * (0 = displacement criterion), neighbor_list_skin_permit (0.5).  Cells are
  * (cutoff+skin)/2 wide or, in an orthorhombic box, the even share of its axis
- * above that (max_atom_in_grid_numbers then counts per (cutoff+skin)/2 cube);
- * boxes with < 3 cells on an axis return
- * SNB_ERR_BOX_TOO_SMALL.  The windowed pair path (below) is chosen only when
+ * above that; boxes with < 3 cells on an axis return SNB_ERR_BOX_TOO_SMALL.
+ * SNB_FLAG_CELL_OVERFLOW is the reference's report: one of its grids, which
+ * are (cutoff+skin)/2 wide with the remainder of an axis in the last, held more
+ * than max_atom_in_grid_numbers atoms (the list is whole all the same).  The windowed pair path (below) is chosen only when
  * max_atom_in_grid_numbers <= 256; a larger capacity keeps the plain path,
  * whose cells hold up to max_atom_in_grid_numbers atoms as the reference's.
  * A triclinic cell takes the plain path with the reference's neighbour-grid

@@ -101,6 +101,7 @@ void free_nl(SnbNl& L)
     L.triclinic = false;
     dfree(L.cell_count);
     dfree(L.cell_start);
+    dfree(L.grid_count);
     dfree(L.atom_cell);
     dfree(L.atom_slot);
     dfree(L.sorted_id);
@@ -878,6 +879,7 @@ int snb_nl_initial(snb_context* c, float cutoff, float skin, snb_ltmatrix3 cell,
     int n = c->n;
     if (!rc) rc = dalloc(&L.cell_count, L.ncell + 1);
     if (!rc) rc = dalloc(&L.cell_start, L.ncell + 1);
+    if (!rc && !L.triclinic) rc = dalloc(&L.grid_count, L.ncell);
     if (!rc) rc = dalloc(&L.atom_cell, n);
     if (!rc) rc = dalloc(&L.atom_slot, n);
     if (!rc) rc = dalloc(&L.sorted_id, n);

@@ -73,6 +73,7 @@ struct SnbNl
     int nx = 0, ny = 0, nz = 0, ncell = 0;
     int* cell_count = nullptr;   // ncell + 1; the last: set by a cut row of the plain path's list
     int* cell_start = nullptr;   // ncell + 1 (exclusive scan)
+    int* grid_count = nullptr;   // ncell: atoms of the reference's grids (orthorhombic boxes)
     int* atom_cell = nullptr;    // n
     int* atom_slot = nullptr;    // n
     int* sorted_id = nullptr;    // n (scatter order)

@@ -59,16 +59,19 @@ __global__ void k_nl_set_batch(SnbSegTab t)
 }
 
 __device__ __forceinline__ void k_nl_clear_counts_body(const int* __restrict__ need, int ncell, int* __restrict__ cnt,
+                                                       int* __restrict__ grid_count,
     unsigned bid, unsigned nbid)
 {
     if (need[0] == 0) return;
     int i = bid * blockDim.x + threadIdx.x;
     if (i <= ncell) cnt[i] = 0;
+    if (grid_count && i < ncell) grid_count[i] = 0;
 }
 
-__global__ void k_nl_clear_counts(const int* __restrict__ need, int ncell, int* __restrict__ cnt)
+__global__ void k_nl_clear_counts(const int* __restrict__ need, int ncell, int* __restrict__ cnt,
+                                  int* __restrict__ grid_count)
 {
-    k_nl_clear_counts_body(need, ncell, cnt, blockIdx.x, gridDim.x);
+    k_nl_clear_counts_body(need, ncell, cnt, grid_count, blockIdx.x, gridDim.x);
 }
 
 struct NlClearArgs
@@ -76,13 +79,14 @@ struct NlClearArgs
     const int* need;
     int ncell;
     int* cnt;
+    int* grid_count;
 };
 
 __global__ void k_nl_clear_counts_batch(SnbSegTab t)
 {
     unsigned bid, nbid;
     const NlClearArgs& a = snb_seg<NlClearArgs>(t, bid, nbid);
-    k_nl_clear_counts_body(a.need, a.ncell, a.cnt, bid, nbid);
+    k_nl_clear_counts_body(a.need, a.ncell, a.cnt, a.grid_count, bid, nbid);
 }
 
 // Put_Atom_In_Grids (neighbor_list.cpp:206-275): the wrap into the cell uses
@@ -94,12 +98,51 @@ __global__ void k_nl_clear_counts_batch(SnbSegTab t)
 // 262 us against 134, the list export 138 against 95; the pairs found are the
 // same).  A triclinic cell keeps the reference's widths, which its table of
 // neighbour cells is made for.  The slot inside the cell comes from an atomic
-// counter and is made deterministic later.
+// counter and is made deterministic later.  The overflow report is the
+// reference's, so its grids have a count of their own (grid_count; in a
+// triclinic cell they are the cells).
+__device__ __forceinline__ int cell_of(const snb_vector& r, float wx, float wy, float wz, int nx,
+                                       int ny, int nz)
+{
+    int ix = (int)(r.x / wx);
+    int iy = (int)(r.y / wy);
+    int iz = (int)(r.z / wz);
+    ix = ix < 0 ? 0 : (ix < nx ? ix : nx - 1);
+    iy = iy < 0 ? 0 : (iy < ny ? iy : ny - 1);
+    iz = iz < 0 ? 0 : (iz < nz ? iz : nz - 1);
+    return (ix * ny + iy) * nz + iz;
+}
+
+// Counts the lane's atom in cell c and returns its place there.  The atoms of
+// a wavefront that follow one another in one cell, those of a molecule, take one
+// add: the adds, hundreds to a line of counters, are what bounds k_nl_bin (an
+// add per atom 8.3 us for one count at 45,000 atoms of water and 11.5 for both,
+// an add per molecule and cell 4.9 for both).
+// The lanes at work are the wavefront's first ones.
+__device__ __forceinline__ int count_in_cell(int* __restrict__ cnt, int c)
+{
+    const int lane = threadIdx.x & 63;
+    const uint64_t upto = ~0ull >> (63 - lane);  // lanes 0 .. lane
+    const int before = __shfl_up(c, 1);
+    const bool head = lane == 0 || before != c;
+    const uint64_t heads = __ballot(head);
+    const int first = 63 - __builtin_clzll(heads & upto);
+    const int lanes = __popcll(__ballot(1));
+    int base = 0;
+    if (head)
+    {
+        const uint64_t later = heads & ~upto;
+        base = atomicAdd(&cnt[c], (later ? __builtin_ctzll(later) : lanes) - lane);
+    }
+    return __shfl(base, first) + lane - first;
+}
+
 __device__ __forceinline__ void k_nl_bin_body(const int* __restrict__ need, int n, const snb_vector* __restrict__ crd,
                          snb_vector* __restrict__ old, int copy_old, SnbBox box,
                          float wx, float wy, float wz, int nx, int ny, int nz,
                          int* __restrict__ atom_cell,
-                         int* __restrict__ atom_slot, int* __restrict__ cnt,
+                         int* __restrict__ atom_slot, int* __restrict__ cnt, float grid_length,
+                         int* __restrict__ grid_count,
     unsigned bid, unsigned nbid)
 {
     if (need[0] == 0) return;
@@ -114,26 +157,23 @@ __device__ __forceinline__ void k_nl_bin_body(const int* __restrict__ need, int 
     r.y -= k2 * box.c[2];
     r.x -= k3 * box.c[3] + k2 * box.c[1];
     r.x -= floorf(r.x / box.c[0]) * box.c[0];
-    int ix = (int)(r.x / wx);
-    int iy = (int)(r.y / wy);
-    int iz = (int)(r.z / wz);
-    ix = ix < 0 ? 0 : (ix < nx ? ix : nx - 1);
-    iy = iy < 0 ? 0 : (iy < ny ? iy : ny - 1);
-    iz = iz < 0 ? 0 : (iz < nz ? iz : nz - 1);
-    int c = (ix * ny + iy) * nz + iz;
+    const int c = cell_of(r, wx, wy, wz, nx, ny, nz);
     atom_cell[i] = c;
-    atom_slot[i] = atomicAdd(&cnt[c], 1);
+    if (grid_count)
+        count_in_cell(grid_count, cell_of(r, grid_length, grid_length, grid_length, nx, ny, nz));
+    atom_slot[i] = count_in_cell(cnt, c);
 }
 
 __global__ void k_nl_bin(const int* __restrict__ need, int n, const snb_vector* __restrict__ crd,
                          snb_vector* __restrict__ old, int copy_old, SnbBox box,
                          float wx, float wy, float wz, int nx, int ny, int nz,
                          int* __restrict__ atom_cell,
-                         int* __restrict__ atom_slot, int* __restrict__ cnt)
+                         int* __restrict__ atom_slot, int* __restrict__ cnt, float grid_length,
+                         int* __restrict__ grid_count)
 {
     k_nl_bin_body(
         need, n, crd, old, copy_old, box, wx, wy, wz, nx, ny, nz, atom_cell, atom_slot, cnt,
-        blockIdx.x, gridDim.x);
+        grid_length, grid_count, blockIdx.x, gridDim.x);
 }
 
 struct NlBinArgs
@@ -153,6 +193,8 @@ struct NlBinArgs
     int* atom_cell;
     int* atom_slot;
     int* cnt;
+    float grid_length;
+    int* grid_count;
 };
 
 __global__ void k_nl_bin_batch(SnbSegTab t)
@@ -161,7 +203,7 @@ __global__ void k_nl_bin_batch(SnbSegTab t)
     const NlBinArgs& a = snb_seg<NlBinArgs>(t, bid, nbid);
     k_nl_bin_body(
         a.need, a.n, a.crd, a.old, a.copy_old, a.box, a.wx, a.wy, a.wz, a.nx, a.ny, a.nz, a.atom_cell,
-        a.atom_slot, a.cnt, bid, nbid);
+        a.atom_slot, a.cnt, a.grid_length, a.grid_count, bid, nbid);
 }
 
 __device__ __forceinline__ void k_nl_scatter_body(const int* __restrict__ need, int n, const int* __restrict__ atom_cell,
@@ -200,9 +242,9 @@ __global__ void k_nl_scatter_batch(SnbSegTab t)
 }
 
 // One wave per cell: rank the cell's atoms by id (O(m^2) with m ~ 20-60) and
-// write ids, cell numbers and coordinates in id order.  Also flags cells above
-// the reference's per-cell capacity (max_atom_in_grid_numbers) for parity of
-// the overflow report; nothing is truncated here.
+// write ids, cell numbers and coordinates in id order.  Also flags grids of the
+// reference above its per-grid capacity (max_atom_in_grid_numbers) for parity
+// of the overflow report; nothing is truncated here.
 #define SNB_NL_SORT_MAX 1024
 __device__ __forceinline__ void k_nl_cell_sort_body(const int* __restrict__ need, int ncell,
                                                      const int* __restrict__ start,
@@ -211,7 +253,8 @@ __device__ __forceinline__ void k_nl_cell_sort_body(const int* __restrict__ need
                                                      float4* __restrict__ sorted_crd,
                                                      int* __restrict__ order,
                                                      int* __restrict__ sorted_cell,
-                                                     int max_in_cell, int* __restrict__ status,
+                                                     const int* __restrict__ grid_count,
+                                                     int max_in_grid, int* __restrict__ status,
     unsigned bid, unsigned nbid)
 {
     if (need[0] == 0) return;
@@ -220,7 +263,8 @@ __device__ __forceinline__ void k_nl_cell_sort_body(const int* __restrict__ need
     if (c >= ncell) return;
     int b = start[c], m = start[c + 1] - b;
     int lane = threadIdx.x;
-    if (m > max_in_cell && lane == 0) atomicOr(status, SNB_FLAG_CELL_OVERFLOW);
+    if (lane == 0 && (grid_count ? grid_count[c] : m) > max_in_grid)
+        atomicOr(status, SNB_FLAG_CELL_OVERFLOW);
     if (m > SNB_NL_SORT_MAX)
     {
         // keep scatter order (still a correct set)
@@ -255,11 +299,12 @@ __global__ void __launch_bounds__(64) k_nl_cell_sort(const int* __restrict__ nee
                                                      float4* __restrict__ sorted_crd,
                                                      int* __restrict__ order,
                                                      int* __restrict__ sorted_cell,
-                                                     int max_in_cell, int* __restrict__ status)
+                                                     const int* __restrict__ grid_count,
+                                                     int max_in_grid, int* __restrict__ status)
 {
     k_nl_cell_sort_body(
-        need, ncell, start, sorted_id, crd, sorted_crd, order, sorted_cell, max_in_cell, status,
-        blockIdx.x, gridDim.x);
+        need, ncell, start, sorted_id, crd, sorted_crd, order, sorted_cell, grid_count,
+        max_in_grid, status, blockIdx.x, gridDim.x);
 }
 
 struct NlCellSortArgs
@@ -272,7 +317,8 @@ struct NlCellSortArgs
     float4* sorted_crd;
     int* order;
     int* sorted_cell;
-    int max_in_cell;
+    const int* grid_count;
+    int max_in_grid;
     int* status;
 };
 
@@ -282,7 +328,7 @@ __global__ void __launch_bounds__(64) k_nl_cell_sort_batch(SnbSegTab t)
     const NlCellSortArgs& a = snb_seg<NlCellSortArgs>(t, bid, nbid);
     k_nl_cell_sort_body(
         a.need, a.ncell, a.start, a.sorted_id, a.crd, a.sorted_crd, a.order, a.sorted_cell,
-        a.max_in_cell, a.status, bid, nbid);
+        a.grid_count, a.max_in_grid, a.status, bid, nbid);
 }
 
 // The three axis offset sets of the +-2 stencil: five distinct cells when the
@@ -542,17 +588,13 @@ int snb_launch_nl_update(snb_context* ctx, const snb_vector* crd, const SnbBox& 
     SNB_CHECK(hipGetLastError());
     float w[3];
     snb_cell_widths(L, box, w);
-    // max_atom_in_grid_numbers is a count per reference cell of grid_length^3
-    const double wide = L.triclinic ? 1.0
-                                    : (double)w[0] * w[1] * w[2] /
-                                          ((double)L.grid_length * L.grid_length * L.grid_length);
-    const int max_in_cell = (int)(L.max_in_cell * (wide > 1.0 ? wide : 1.0));
     SNB_LAUNCH_B(k_nl_clear_counts, k_nl_clear_counts_batch, NlClearArgs,
-                 dim3((L.ncell + 256) / 256), dim3(256), 0, s, L.need, L.ncell, L.cell_count);
+                 dim3((L.ncell + 256) / 256), dim3(256), 0, s, L.need, L.ncell, L.cell_count,
+                 L.grid_count);
     SNB_LAUNCH_B(k_nl_bin, k_nl_bin_batch, NlBinArgs, dim3((n + 255) / 256), dim3(256), 0, s,
                  L.need, n, crd, L.old_crd,
                  L.refresh_interval <= 0 ? 1 : 0, box, w[0], w[1], w[2], L.nx, L.ny, L.nz, L.atom_cell,
-                 L.atom_slot, L.cell_count);
+                 L.atom_slot, L.cell_count, L.grid_length, L.grid_count);
     SNB_CHECK(hipGetLastError());
     int rc = snb_launch_exclusive_scan(s, L.cell_count, L.cell_start, L.ncell);
     if (rc) return rc;
@@ -560,7 +602,7 @@ int snb_launch_nl_update(snb_context* ctx, const snb_vector* crd, const SnbBox& 
                  0, s, L.need, n, L.atom_cell, L.atom_slot, L.cell_start, L.sorted_id);
     SNB_LAUNCH_B(k_nl_cell_sort, k_nl_cell_sort_batch, NlCellSortArgs, dim3(L.ncell), dim3(64), 0,
                  s, L.need, L.ncell, L.cell_start, L.sorted_id, crd, L.sorted_crd, L.order,
-                 L.sorted_cell, max_in_cell, ctx->status);
+                 L.sorted_cell, L.grid_count, L.max_in_cell, ctx->status);
     if (L.windowed)
     {
         rc = snb_launch_nl_window(ctx, box, ex_start, ex_list, ex_num);

@@ -70,8 +70,11 @@ class Segment:
         s = req.system()
         free0 = torch.cuda.mem_get_info()[0]
         self.stream = torch.cuda.Stream()
-        # the per-cell capacity key is raised from its default of 150 to the
-        # most that takes the windowed path
+        # the last of the reference's grids on each axis takes the remainder of
+        # box / grid width and can be nearly twice as wide, so a corner grid can
+        # hold ~8x the mean occupancy (~17 atoms here): the per-grid capacity
+        # key is raised from its default of 150 to the most that takes the
+        # windowed path
         nb = Nonbonded(s, cutoff=s["cutoff"], refresh_interval=chunk, stream=self.stream,
                        max_atom_in_grid_numbers=MAX_ATOMS_IN_CELL)
         nb.set_pme_overlap(overlap)

@@ -71,3 +71,76 @@ def test_windowed_list_matches_oracle(name, images):
     ic, _ = nb.internal_rows()
     assert ic.sum() == gc.sum()
     nb.close()
+
+
+def _clustered(box):
+    """One of seven particles around a corner of the reference's grids, which
+    are 6 A wide, well inside a cell that shares its axis evenly."""
+    s = _stretched(box)
+    rng = np.random.default_rng(2)
+    near = rng.random(s["n"]) < 0.15
+    s["crd"][near] = 6.0 + rng.normal(0, 0.6, (int(near.sum()), 3))
+    return s
+
+
+def _tilted():
+    from test_gpu_full_rows import _edges
+    return _edges(6000, (40.0, 44.0, 48.0), (85.0, 87.0, 84.0))
+
+
+def _most_in_a_grid(s, cutoff, even=False):
+    """Atoms of the fullest grid of the reference (grids of (cutoff + skin) / 2,
+    the last of an axis with the remainder; neighbor_list.cpp:206-275), or of
+    cells that share each axis evenly."""
+    f = np.float32
+    c = np.asarray(s["cell"], f)
+    gl = (f(cutoff) + f(2.0)) * f(0.5)
+    edge = c[[0, 2, 5]]
+    per = np.floor(edge / gl).astype(np.int64)
+    r = np.array(s["crd"], f)
+    k3 = np.floor(r[:, 2] / c[5])
+    r[:, 2] -= k3 * c[5]
+    r[:, 1] -= k3 * c[4]
+    k2 = np.floor(r[:, 1] / c[2])
+    r[:, 1] -= k2 * c[2]
+    r[:, 0] -= k3 * c[3] + k2 * c[1]
+    r[:, 0] -= np.floor(r[:, 0] / c[0]) * c[0]
+    width = edge / per.astype(f) if even else np.full(3, gl)
+    g = np.clip((r / width).astype(np.int64), 0, per - 1)
+    return int(np.bincount((g[:, 0] * per[1] + g[:, 1]) * per[2] + g[:, 2]).max())
+
+
+OVERFLOW = {
+    "exact_edges": dict(make=lambda: _stretched((30.0, 60.0, 36.0)), cutoff=10.0),
+    # the reference's corner grid holds several times the atoms of an even cell
+    "wide_cells": dict(make=lambda: _stretched((35.9, 47.9, 41.9)), cutoff=10.0),
+    # an even cell holds several times the atoms of the reference's fullest grid
+    "clustered": dict(make=lambda: _clustered((35.9, 47.9, 41.9)), cutoff=10.0, max_nb=2600),
+    "triclinic": dict(make=_tilted, cutoff=8.0, plain=True),
+}
+
+
+@pytest.mark.parametrize("plain", [False, True])
+@pytest.mark.parametrize("name", sorted(OVERFLOW))
+def test_grid_overflow_report(name, plain):
+    """The overflow flag counts the reference's grids, whatever the cells that
+    the list is built over: raised from the first atom above the limit."""
+    from sponge_amd.lib import FLAG_CELL_OVERFLOW, Nonbonded
+    c = OVERFLOW[name]
+    s = c["make"]()
+    most = _most_in_a_grid(s, c["cutoff"])
+    if name == "wide_cells":
+        assert 2 * _most_in_a_grid(s, c["cutoff"], even=True) < most
+    if name == "clustered":
+        assert _most_in_a_grid(s, c["cutoff"], even=True) > 3 * most
+    for limit in (most - 1, most):
+        nb = Nonbonded(s, cutoff=c["cutoff"], skin=2.0, max_neighbor_numbers=c.get("max_nb", 1200),
+                       max_atom_in_grid_numbers=limit)
+        if plain and nb.window_info()["windowed"]:
+            assert nb.set_window_shape(0, 0, 0)
+        elif not c.get("plain") and limit <= 256 and not plain:
+            assert nb.window_info()["windowed"]
+        for _ in range(2):
+            nb.nl_update(forced=True)
+            assert nb.status(clear=True) == (FLAG_CELL_OVERFLOW if limit < most else 0)
+        nb.close()
