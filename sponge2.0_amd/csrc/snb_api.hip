@@ -758,20 +758,19 @@ static int setup_window(snb_context* c)
 }
 
 // Rows of lower ids of a small system's plain-path list (filled at rebuilds).
-static int setup_full_list(snb_context* c)
+// The path does without them, so memory that is not there is no error.
+static void setup_full_list(snb_context* c)
 {
     SnbNl& L = c->nl;
     const int n = c->n;
-    if (n <= 0 || n > SNB_FULL_MAX || L.lo_rows) return SNB_OK;
-    if (L.triclinic && !L.nbr_of_cells) return SNB_OK;
-    int rc = dalloc(&L.lo_rows, (size_t)n * n);
-    if (!rc) rc = dalloc(&L.lo_count, n);
-    if (rc)
+    if (n <= 0 || n > SNB_FULL_MAX || L.lo_rows) return;
+    if (L.triclinic && !L.nbr_of_cells) return;
+    if (dalloc(&L.lo_rows, (size_t)n * n) || dalloc(&L.lo_count, n))
     {
         dfree(L.lo_rows);
         dfree(L.lo_count);
+        (void)hipGetLastError();
     }
-    return rc;
 }
 
 // Find_Neighor_Grids_Device (neighbor_list.cpp:5-48) for a triclinic cell:
@@ -838,9 +837,13 @@ static int triclinic_neighbour_cells(SnbNl& L, const snb_ltmatrix3& cell, bool b
             if (of_count[cj] == SNB_NL_MAX_NBR) return SNB_OK;  // the half list alone
             of[(size_t)cj * SNB_NL_MAX_NBR + of_count[cj]++] = ci;
         }
-    rc = dalloc(&L.nbr_of_cells, of.size());
-    if (!rc) rc = dalloc(&L.nbr_of_count, (size_t)ncell);
-    if (rc) return rc;
+    if (dalloc(&L.nbr_of_cells, of.size()) || dalloc(&L.nbr_of_count, (size_t)ncell))
+    {
+        dfree(L.nbr_of_cells);
+        dfree(L.nbr_of_count);
+        (void)hipGetLastError();
+        return SNB_OK;  // the half list alone
+    }
     SNB_CHECK(hipMemcpy(L.nbr_of_cells, of.data(), sizeof(int) * of.size(), hipMemcpyHostToDevice));
     SNB_CHECK(hipMemcpy(L.nbr_of_count, of_count.data(), sizeof(int) * ncell,
                         hipMemcpyHostToDevice));
@@ -912,11 +915,7 @@ int snb_nl_initial(snb_context* c, float cutoff, float skin, snb_ltmatrix3 cell,
         free_nl(L);
         return rc;
     }
-    if (!L.windowed && (rc = setup_full_list(c)))
-    {
-        free_nl(L);
-        return rc;
-    }
+    if (!L.windowed) setup_full_list(c);
     // ATOM_GROUP rows point into the padded table (neighbor_list.cpp:764-771)
     std::vector<snb_atom_group> h(n > 0 ? n : 1);
     for (int i = 0; i < n; i++)
@@ -1058,7 +1057,11 @@ int snb_nl_set_window_shape(snb_context* c, int a, int b, int s)
     SNB_CHECK(hipStreamSynchronize(c->stream));  // no launch in flight uses the old buffers
     free_window(L);
     L.built = false;  // the next snb_nl_update rebuilds for the new path
-    if (plain) return setup_full_list(c);
+    if (plain)
+    {
+        setup_full_list(c);
+        return SNB_OK;
+    }
     L.win = W;
     return setup_window(c);
 }
