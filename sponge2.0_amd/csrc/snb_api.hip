@@ -96,8 +96,8 @@ void free_nl(SnbNl& L)
 {
     dfree(L.nbr_cells);
     dfree(L.nbr_count);
-    dfree(L.nbr_of_cells);
-    dfree(L.nbr_of_count);
+    dfree(L.nbr_both);
+    dfree(L.nbr_both_count);
     L.triclinic = false;
     dfree(L.cell_count);
     dfree(L.cell_start);
@@ -764,7 +764,7 @@ static void setup_full_list(snb_context* c)
     SnbNl& L = c->nl;
     const int n = c->n;
     if (n <= 0 || n > SNB_FULL_MAX || L.lo_rows) return;
-    if (L.triclinic && !L.nbr_of_cells) return;
+    if (L.triclinic && !L.nbr_both) return;
     if (dalloc(&L.lo_rows, (size_t)n * n) || dalloc(&L.lo_count, n))
     {
         dfree(L.lo_rows);
@@ -782,8 +782,8 @@ static void setup_full_list(snb_context* c)
 // in ascending cell order, as the reference's search over all cells finds it.
 // [-3, 2] holds for an image and for its opposite, so j may be a neighbour of i
 // and i none of j: a pair is in the list by the table of the lower id's cell
-// alone, and the rows of lower ids (`both`) are searched through the transposed
-// table, the cells that have cell i for a neighbour.
+// alone, and the rows of lower ids (`both`) are searched in the cells that have
+// cell i for a neighbour.
 static int triclinic_neighbour_cells(SnbNl& L, const snb_ltmatrix3& cell, bool both)
 {
     const int nx = L.nx, ny = L.ny, nz = L.nz, ncell = L.ncell;
@@ -829,23 +829,38 @@ static int triclinic_neighbour_cells(SnbNl& L, const snb_ltmatrix3& cell, bool b
                         hipMemcpyHostToDevice));
     SNB_CHECK(hipMemcpy(L.nbr_count, count.data(), sizeof(int) * ncell, hipMemcpyHostToDevice));
     if (!both) return SNB_OK;
-    std::vector<int> of((size_t)ncell * SNB_NL_MAX_NBR), of_count(ncell, 0);
+    std::vector<std::vector<int>> of(ncell);  // ascending, as ci ascends
     for (int ci = 0; ci < ncell; ci++)
         for (int k = 0; k < count[ci]; k++)
-        {
-            const int cj = cells[(size_t)ci * SNB_NL_MAX_NBR + k];
-            if (of_count[cj] == SNB_NL_MAX_NBR) return SNB_OK;  // the half list alone
-            of[(size_t)cj * SNB_NL_MAX_NBR + of_count[cj]++] = ci;
-        }
-    if (dalloc(&L.nbr_of_cells, of.size()) || dalloc(&L.nbr_of_count, (size_t)ncell))
+            of[cells[(size_t)ci * SNB_NL_MAX_NBR + k]].push_back(ci);
+    const int most = 2 * SNB_NL_MAX_NBR;
+    std::vector<int> joined((size_t)ncell * most), joined_count(ncell, 0);
+    for (int ci = 0; ci < ncell; ci++)
     {
-        dfree(L.nbr_of_cells);
-        dfree(L.nbr_of_count);
+        const int* up = cells.data() + (size_t)ci * SNB_NL_MAX_NBR;
+        const int* up_end = up + count[ci];
+        auto down = of[ci].begin();
+        while (up < up_end || down != of[ci].end())
+        {
+            if (joined_count[ci] == most) return SNB_OK;  // the half list alone
+            const bool in_up = up < up_end && (down == of[ci].end() || *up <= *down);
+            const bool in_down = down != of[ci].end() && (!in_up || *down == *up);
+            joined[(size_t)ci * most + joined_count[ci]++] =
+                (in_up ? *up | SNB_NBR_UP : *down) | (in_down ? SNB_NBR_DOWN : 0);
+            up += in_up;
+            down += in_down;
+        }
+    }
+    if (ncell >= SNB_NBR_UP || dalloc(&L.nbr_both, joined.size()) ||
+        dalloc(&L.nbr_both_count, (size_t)ncell))
+    {
+        dfree(L.nbr_both);
+        dfree(L.nbr_both_count);
         (void)hipGetLastError();
         return SNB_OK;  // the half list alone
     }
-    SNB_CHECK(hipMemcpy(L.nbr_of_cells, of.data(), sizeof(int) * of.size(), hipMemcpyHostToDevice));
-    SNB_CHECK(hipMemcpy(L.nbr_of_count, of_count.data(), sizeof(int) * ncell,
+    SNB_CHECK(hipMemcpy(L.nbr_both, joined.data(), sizeof(int) * joined.size(), hipMemcpyHostToDevice));
+    SNB_CHECK(hipMemcpy(L.nbr_both_count, joined_count.data(), sizeof(int) * ncell,
                         hipMemcpyHostToDevice));
     return SNB_OK;
 }

@@ -46,6 +46,8 @@ enum SnbDoubleSlot
 #define SNB_NLC_MAXA 256
 // neighbour cells per cell of a triclinic grid (MAX_GRID_NEIGHBORS, neighbor_list.cpp:3)
 #define SNB_NL_MAX_NBR 192
+#define SNB_NBR_UP (1 << 29)    // an entry of the union: in the cell's own table
+#define SNB_NBR_DOWN (1 << 30)  // in the transposed one
 #define SNB_FFT_MAX_N 1024
 
 // A line transform: pass p (in order) takes the stage radices
@@ -93,10 +95,11 @@ struct SnbNl
     bool triclinic = false;
     int* nbr_cells = nullptr;  // ncell * SNB_NL_MAX_NBR
     int* nbr_count = nullptr;  // ncell
-    // the transposed table (cells that have cell c for a neighbour), where the
-    // rows of lower ids are kept
-    int* nbr_of_cells = nullptr;
-    int* nbr_of_count = nullptr;
+    // where the rows of lower ids are kept: the union of that table and the
+    // transposed one (cells that have cell c for a neighbour), each entry with
+    // the tables that it is in
+    int* nbr_both = nullptr;        // ncell * 2 * SNB_NL_MAX_NBR
+    int* nbr_both_count = nullptr;  // ncell
     // windowed pair path (every axis >= 5 cells)
     bool windowed = false;
     int export_mode = 1;  // reference-layout list at rebuild: 0 no, 1 yes, 2 yes with sorted rows

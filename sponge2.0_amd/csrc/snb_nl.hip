@@ -360,7 +360,7 @@ __device__ __forceinline__ void k_nl_search_body(
     const int* __restrict__ ex_num, int max_nb, int* __restrict__ serial,
     snb_atom_group* __restrict__ nl, int* __restrict__ status,
     const int* __restrict__ nbr_cells, const int* __restrict__ nbr_count,
-    const int* __restrict__ nbr_of_cells, const int* __restrict__ nbr_of_count,
+    const int* __restrict__ nbr_both, const int* __restrict__ nbr_both_count,
     uint16_t* __restrict__ lo_rows, int* __restrict__ lo_count, int* __restrict__ cut,
     unsigned bid, unsigned nbid)
 {
@@ -477,15 +477,23 @@ __device__ __forceinline__ void k_nl_search_body(
     if (nbr_cells)
     {
         // triclinic cell: the cell's neighbour cells from the table, and for
-        // lower ids the cells that have this one for a neighbour
-        const int* tab = nbr_cells + (size_t)c * SNB_NL_MAX_NBR;
-        const int m = nbr_count[c];
-        for (int k = 0; k < m; k++) scan(start[tab[k]], start[tab[k] + 1], true, false);
-        if (lo_row)
+        // lower ids the cells that have this one for a neighbour (most are both)
+        const int cu = __builtin_amdgcn_readfirstlane(c);
+        if (lo_rows)
         {
-            const int* of = nbr_of_cells + (size_t)c * SNB_NL_MAX_NBR;
-            const int mo = nbr_of_count[c];
-            for (int k = 0; k < mo; k++) scan(start[of[k]], start[of[k] + 1], false, true);
+            const int* tab = nbr_both + (size_t)cu * 2 * SNB_NL_MAX_NBR;
+            const int m = nbr_both_count[cu];
+            for (int k = 0; k < m; k++)
+            {
+                const int e = tab[k], cell = e & (SNB_NBR_UP - 1);
+                scan(start[cell], start[cell + 1], (e & SNB_NBR_UP) != 0, (e & SNB_NBR_DOWN) != 0);
+            }
+        }
+        else
+        {
+            const int* tab = nbr_cells + (size_t)cu * SNB_NL_MAX_NBR;
+            const int m = nbr_count[cu];
+            for (int k = 0; k < m; k++) scan(start[tab[k]], start[tab[k] + 1], true, false);
         }
     }
     else
@@ -517,12 +525,12 @@ __global__ void __launch_bounds__(256) k_nl_search(
     const int* __restrict__ ex_num, int max_nb, int* __restrict__ serial,
     snb_atom_group* __restrict__ nl, int* __restrict__ status,
     const int* __restrict__ nbr_cells, const int* __restrict__ nbr_count,
-    const int* __restrict__ nbr_of_cells, const int* __restrict__ nbr_of_count,
+    const int* __restrict__ nbr_both, const int* __restrict__ nbr_both_count,
     uint16_t* __restrict__ lo_rows, int* __restrict__ lo_count, int* __restrict__ cut)
 {
     k_nl_search_body(
         need, n, crd, atom_cell, start, sorted_crd, box, cs2, nx, ny, nz, ex_start, ex_list, ex_num,
-        max_nb, serial, nl, status, nbr_cells, nbr_count, nbr_of_cells, nbr_of_count, lo_rows, lo_count,
+        max_nb, serial, nl, status, nbr_cells, nbr_count, nbr_both, nbr_both_count, lo_rows, lo_count,
         cut, blockIdx.x, gridDim.x);
 }
 
@@ -548,8 +556,8 @@ struct NlSearchArgs
     int* status;
     const int* nbr_cells;
     const int* nbr_count;
-    const int* nbr_of_cells;
-    const int* nbr_of_count;
+    const int* nbr_both;
+    const int* nbr_both_count;
     uint16_t* lo_rows;
     int* lo_count;
     int* cut;
@@ -562,7 +570,7 @@ __global__ void __launch_bounds__(256) k_nl_search_batch(SnbSegTab t)
     k_nl_search_body(
         a.need, a.n, a.crd, a.atom_cell, a.start, a.sorted_crd, a.box, a.cs2, a.nx, a.ny, a.nz,
         a.ex_start, a.ex_list, a.ex_num, a.max_nb, a.serial, a.nl, a.status, a.nbr_cells,
-        a.nbr_count, a.nbr_of_cells, a.nbr_of_count, a.lo_rows, a.lo_count, a.cut, bid, nbid);
+        a.nbr_count, a.nbr_both, a.nbr_both_count, a.lo_rows, a.lo_count, a.cut, bid, nbid);
 }
 
 int snb_launch_nl_update(snb_context* ctx, const snb_vector* crd, const SnbBox& box, int forced,
@@ -612,7 +620,7 @@ int snb_launch_nl_update(snb_context* ctx, const snb_vector* crd, const SnbBox& 
         SNB_LAUNCH_B(k_nl_search, k_nl_search_batch, NlSearchArgs, dim3((n + 3) / 4), dim3(256), 0,
                      s, L.need, n, crd, L.atom_cell, L.cell_start, L.sorted_crd, box, L.cs2, L.nx,
                      L.ny, L.nz, ex_start, ex_list, ex_num, L.max_nb, L.serial, L.dnl, ctx->status,
-                     L.nbr_cells, L.nbr_count, L.nbr_of_cells, L.nbr_of_count, L.lo_rows,
+                     L.nbr_cells, L.nbr_count, L.nbr_both, L.nbr_both_count, L.lo_rows,
                      L.lo_count, L.cell_count + L.ncell);
     snb_prof_end(ctx, SNB_PROF_NL);
     SNB_CHECK(hipGetLastError());
