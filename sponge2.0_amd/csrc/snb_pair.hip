@@ -383,7 +383,8 @@ __global__ void __launch_bounds__(1024) k_lj_lds_batch(SnbSegTab t)
 // the device) for none of its three 64-bit global atomics per pair, whose
 // throughput (about 31 per ns) is what bounds k_lj_direct.  Reads the caller's coordinates and
 // charges and the square parameter table: no packing kernel precedes it.  At
-// 1,500 atoms 25.4 us and 2 for packing -> 5.3 us.
+// 1,500 atoms 25.4 us and 2 for packing -> 5.3 us, in a triclinic cell of 7,200
+// 60 with packing -> 16.
 // A list with rows cut at max_nb (*cut) is taken in one direction with the
 // atomics, as k_lj_direct takes it.
 __device__ __forceinline__ void k_lj_full_body(
@@ -1923,16 +1924,26 @@ int snb_launch_lj_window(snb_context* ctx, const snb_vector* crd, const float* c
                        box.rc[1] == 0.0f && box.rc[3] == 0.0f && box.rc[4] == 0.0f;
     // Force-only steps: the blocks add their window forces to the accumulators
     // by atomics, or write them to the stage (one slot per window atom) which
-    // k_stage_gather sums.  The stage pays only where its gather is wide enough
-    // and its slots are few: ten steps of 66,000 atoms at 10 A 1726 us through
-    // the stage and 1771 by atomics, 93,000 2030 and 2074; but 52,500 1620 and
-    // 1448, 81,000 with 27 slots per atom 2178 and 1905, 126,000 2995 and
-    // 2697, 200,000 3819 and 3667, 1,000,000 22340 and 19412.
+    // k_stage_gather sums.  What decides are the rounds of blocks over the
+    // compute units, one block on each at a time: in two rounds or less they
+    // all end together, and no block's arithmetic runs beside their adds; in
+    // more rounds it does, and the gather comes on top of the pair kernel.  Ten
+    // whole steps, stage / atomics in us, on 256 compute units:
+    //   490 to 512 blocks: 66,000 atoms 1729 / 1767, 81,000 1705 / 1758,
+    //     93,000 (8 A) 1924 / 1973, (10 A) 2237 / 2309, 108,000 2057 / 2136,
+    //     150,000 2656 / 2651;
+    //   612 and more: 87,000 (612) 1969 / 1825, (960) 2293 / 2062, 126,000
+    //     (700) 2510 / 2318, 150,000 (1000) 3527 / 3141, 1,000,000 22340 / 19412.
+    // The stage is kept to the sizes where two rounds are worth most of 2 to 4%
+    // of the step: a pair call by itself, with no other stream beside it, pays 4
+    // to 24% for the gather at any size (66,000 107 / 93 us, 93,000 123 / 117,
+    // at 8 A 105 / 84, 108,000 122 / 117); below, 24,000 to 61,500 atoms are within 3% either
+    // way, and from 135,000 on the step gains nothing any more.
     int jdirect = ctx->lj.j_direct;
     if (jdirect < 0)
     {
-        const bool few_slots = W.wu * W.wv * W.wz <= 22 * W.a * W.b * W.s;
-        jdirect = (n >= 65536 && n <= 98304 && few_slots) ? 0 : 1;
+        const bool two_rounds = W.nblock <= 2 * ctx->num_cu;
+        jdirect = (two_rounds && n >= 65536 && n <= 98304) ? 0 : 1;
     }
     if (need_energy || need_virial) jdirect = 0;
     const int ref_attr = ctx->lj.owner_attribution ? 0 : 1;

@@ -4,14 +4,15 @@ The pair kernel's workgroups own blocks of a x b x s neighbour-list cells and
 keep the force accumulators of the block's window in LDS.  Which shape is
 fastest depends on the box (cell counts), the density and the device: large
 blocks cut the window/stage overhead, small ones give more workgroups to fill
-the chip.  The library picks a shape from a fixed preference list; this tuner
+the chip.  The library picks the shape of the shortest modelled time; this tuner
 times every shape the library accepts for a context on that context's own
 workload (a full neighbour-list period of force steps at fixed coordinates)
 and keeps the fastest.  For each windowed shape it also times both ways the
 blocks hand their window forces to the accumulators on force-only steps
 (a staged per-atom gather, or atomic adds per block: the first is cheaper
-where the stage stays in the last-level cache and the gather's launch is
-hidden, the second removes a launch from small systems' dependent chain).
+where all blocks end together, in at most two rounds over the compute units,
+the second where later rounds run beside the adds, and it removes a launch
+from small systems' dependent chain).
 Every choice gives the same forces, energies and virials (integer
 fixed-point sums), so it affects time only.
 """
