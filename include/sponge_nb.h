@@ -178,10 +178,10 @@ int snb_lj_set_owner_attribution(snb_context* ctx, int enable);
  * compute unit (no counterpart in the reference). */
 int snb_nl_set_window_capacity(snb_context* ctx, int slots);
 /* Block shape of the windowed pair path: each workgroup owns a x b x s cells
- * (x, y, z); 0, 0, 0 selects the plain path (one row per thread group over
- * the public list, global integer atomics).  The default comes from a fixed
- * preference list; a tuner can time the shapes this call accepts and keep the
- * fastest.  SNB_ERR_ARGUMENT when the grid cannot take the shape or its
+ * (x, y, z); 0, 0, 0 selects the plain path (rows of the public list, see
+ * snb_lj_set_row_lds).  The default is the shape of the shortest modelled time
+ * among those whose window fits 60% of the LDS (75% where none does); a tuner
+ * can time the shapes this call accepts and keep the fastest.  SNB_ERR_ARGUMENT when the grid cannot take the shape or its
  * window does not fit the LDS.  Synchronises; the next snb_nl_update
  * rebuilds (setting the shape in use changes nothing).  Forces, energies and
  * virials are the same for every shape (no counterpart in the reference). */
@@ -189,9 +189,8 @@ int snb_nl_set_window_shape(snb_context* ctx, int a, int b, int s);
 /* How the windowed pair kernel hands its window forces to the accumulators
  * on force-only steps: 0 = through a per-block stage and a per-atom gather
  * kernel, 1 = atomic integer adds at the end of each block, -1 (default) =
- * by size (1 below 65,536 atoms and once the stage would exceed 128 MiB,
- * about 310k atoms; 0 between).  Energy
- * and virial steps always use the stage.  Results are the same either way
+ * 0 from 65,536 to 98,304 atoms where there are at most two blocks per compute
+ * unit, else 1.  Energy and virial steps always use the stage.  Results are the same either way
  * (integer sums); SNB_ERR_ARGUMENT for another mode (no counterpart in the
  * reference). */
 int snb_lj_set_direct_j(snb_context* ctx, int mode);
@@ -203,12 +202,14 @@ int snb_lj_set_row_stream(snb_context* ctx, int mode);
 /* Force-only steps of the row kernel (the plain path, used when the windowed
  * path is off): -1 (default) = up to 8,192 atoms each atom sums the pairs of
  * all its neighbours, of lower and of higher ids, without scattered adds
- * (those are what bounds the other two forms); 0 = every pair once, global
+ * (those are what bounds the other two forms; 2 n^2 bytes for the lower ids,
+ * form 0 where that memory is not there); 0 = every pair once, global
  * integer atomics for the higher id; 1 = every pair once, up to 2,560 atoms
  * with every atom's accumulators in LDS, one workgroup per 64 rows and one
  * global add per nonzero sum.  Larger systems and lists that are not the
- * library's own take form 0.  Results are the same either way (no counterpart
- * in the reference). */
+ * library's own take form 0 (by default form 1 up to 2,560 atoms in a recorded
+ * step batch).  Results are the same either way (no counterpart in the
+ * reference). */
 int snb_lj_set_row_lds(snb_context* ctx, int mode);
 /* Geometry of the windowed pair path (windowed = 0 when not used). */
 int snb_nl_window_info(snb_context* ctx, int* windowed, int* a, int* b, int* s, int* wcap,

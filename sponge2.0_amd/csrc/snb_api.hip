@@ -211,6 +211,7 @@ static double window_time(const SnbWin& W, double atoms_per_cell, double pairs_p
         total += kinds.back().first * count;
     }
     std::sort(kinds.rbegin(), kinds.rend());
+    // many rounds of blocks: an even share, in whatever order they start
     if (W.nblock > 16 * num_cu) return total / num_cu + 0.5 * kinds[0].first;
     std::priority_queue<double, std::vector<double>, std::greater<double>> cu;
     for (int i = 0; i < num_cu; i++) cu.push(0.0);

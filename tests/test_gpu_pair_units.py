@@ -102,3 +102,15 @@ def test_new_lj_tables_under_a_built_list():
                                   nb.cutoff), "snb_lj_initial")
     _check(nb, s, s["crd"], lj_a=a, lj_b=b)
     nb.close()
+
+
+def test_row_stream_modes_accepted_and_refused():
+    """snb_lj_set_row_stream takes the modes that it documents and no other."""
+    from sponge_amd.lib import Nonbonded
+    nb = Nonbonded(_gas(150, 64.0), skin=2.0, max_neighbor_numbers=60)
+    for mode in (-1, 0, 1):
+        nb.set_row_stream(mode)
+    for mode in (-2, 2):
+        with pytest.raises(RuntimeError):
+            nb.set_row_stream(mode)
+    nb.close()

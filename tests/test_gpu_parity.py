@@ -66,8 +66,8 @@ def test_neighbor_list_sets_equal_oracle(request, name):
 def test_pair_kernel_bit_exact_with_twin(request, name, energy, virial, owner, stream):
     """Default: per-atom terms on the lower id, as the reference's rows hold
     them (twin over the public list).  owner=True: per-atom terms on the row
-    owner of the internal list (twin over the internal rows).  stream: the
-    force-only loop pipelined within rows (0) or across row ends (1)."""
+    owner of the internal list (twin over the internal rows).  stream: a mode
+    of snb_lj_set_row_stream, all of which run the one force-only loop."""
     import oracle
     s = _get(request, name)
     nb = _nb(s)
@@ -625,8 +625,9 @@ def test_window_overflow_path_bit_exact(water_9k, slots):
 @pytest.mark.parametrize("stream", [0, 1])
 def test_window_direct_j_adds_bit_exact(water_9k, slots, stream):
     """Force-only steps with the window forces added atomically per block
-    (mode 1) match the twin bit for bit, as the staged gather (mode 0) does,
-    with either pair loop; 64 slots puts most blocks on the overflow path."""
+    (mode 1) match the twin bit for bit, as the staged gather (mode 0) does;
+    64 slots puts most blocks on the overflow path.  stream: a mode of
+    snb_lj_set_row_stream, all of which run the one force-only loop."""
     import oracle
     s = water_9k
     t_f = None
