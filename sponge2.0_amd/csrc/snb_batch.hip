@@ -12,6 +12,7 @@
 // bit-identical to running it alone.
 #include <algorithm>
 #include <map>
+#include <tuple>
 
 #include "snb_internal.h"
 
@@ -30,6 +31,13 @@ struct PlanOp
     int lane = 0;
     bool join = false, writes_inputs = false;
 };
+
+// what the members' launches of one dispatch have in common
+typedef std::tuple<const void*, unsigned, int> PlanKey;
+PlanKey key_of(const SnbRecOp& o) { return std::make_tuple(o.bfn, o.block, o.lane); }
+// Launches that the planner looks ahead: a list rebuild and the step around it
+// (about 14 and 14), short of the next but one step.
+#define PLAN_AHEAD 28
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 }  // namespace
@@ -136,6 +144,7 @@ static int batch_plan(snb_batch* b)
 {
     const int M = (int)b->member.size();
     std::vector<size_t> cur(M, 0);
+    std::vector<std::map<PlanKey, int>> done(M);  // batched launches of each kernel so far
     std::vector<char> host;
     auto place = [&](const void* p, size_t bytes, size_t align) {
         size_t off = align_up(host.size(), align);
@@ -165,40 +174,68 @@ static int batch_plan(snb_batch* b)
                 cur[m]++;
             }
         }
-        // Next dispatch: among the heads of the members that have issued the
-        // fewest launches so far, the batched kernel (with its block size and
-        // lane) at the head of most members.  Members whose sequences differ for a while
-        // (plain and windowed pair path, grids with and without the fused
-        // plane transform) so fall back into step with the others.
-        size_t lag = (size_t)-1;
-        for (int m = 0; m < M; m++)
-            if (cur[m] < b->rec[m].ops.size()) lag = std::min(lag, cur[m]);
-        if (lag == (size_t)-1) break;
-        std::vector<std::tuple<const void*, unsigned, int>> keys;
-        std::vector<int> votes;
+        // Next dispatch: among the batched kernels (with block size and lane) at
+        // the members' heads, the one that the fewest members are still to
+        // reach, then the one at most heads, then the head of the member that
+        // has issued the fewest launches.  A member is still to reach a kernel
+        // when one of its next launches is that kernel's counterpart, i.e. it
+        // has launched it no more often than the members that have it at their
+        // head.  So members whose sequences differ for a while (plain and
+        // windowed pair path, grids with and without the fused plane transform)
+        // meet again at the next kernel that they share, whatever the number
+        // of launches in between.
+        // (Taken by the fewest launches issued so far, a member with one launch
+        // less in a step ran ahead for good: 256 dispatches a period of eight
+        // segments of 1,500 to 40,000 atoms, 2900 us, in place of 152, 2379.)
+        bool left = false;
+        std::vector<PlanKey> keys;
+        std::vector<int> votes, often;
+        std::vector<size_t> least;
         for (int m = 0; m < M; m++)
         {
             if (cur[m] >= b->rec[m].ops.size()) continue;
-            const SnbRecOp& o = b->rec[m].ops[cur[m]];
-            auto key = std::make_tuple(o.bfn, o.block, o.lane);
+            left = true;
+            const PlanKey key = key_of(b->rec[m].ops[cur[m]]);
             auto it = std::find(keys.begin(), keys.end(), key);
             if (it == keys.end())
             {
                 keys.push_back(key);
                 votes.push_back(0);
+                often.push_back(0);
+                least.push_back(cur[m]);
                 it = keys.end() - 1;
             }
-            votes[it - keys.begin()] += 1;
+            const size_t k = it - keys.begin();
+            votes[k] += 1;
+            often[k] = std::max(often[k], done[m][key]);
+            least[k] = std::min(least[k], cur[m]);
         }
-        int best = -1;
-        for (int m = 0; m < M; m++)
+        if (!left) break;
+        int best = -1, best_awaited = 0;
+        for (int k = 0; k < (int)keys.size(); k++)
         {
-            if (cur[m] != lag || cur[m] >= b->rec[m].ops.size()) continue;
-            const SnbRecOp& o = b->rec[m].ops[cur[m]];
-            const int k = (int)(std::find(keys.begin(), keys.end(),
-                                          std::make_tuple(o.bfn, o.block, o.lane)) -
-                                keys.begin());
-            if (best < 0 || votes[k] > votes[best]) best = k;
+            int awaited = 0;
+            for (int m = 0; m < M; m++)
+            {
+                const std::vector<SnbRecOp>& ops = b->rec[m].ops;
+                if (cur[m] >= ops.size() || key_of(ops[cur[m]]) == keys[k] ||
+                    done[m][keys[k]] > often[k])
+                    continue;
+                const size_t end = std::min(ops.size(), cur[m] + PLAN_AHEAD);
+                for (size_t i = cur[m] + 1; i < end; i++)
+                    if (key_of(ops[i]) == keys[k])
+                    {
+                        awaited++;
+                        break;
+                    }
+            }
+            if (best < 0 || awaited < best_awaited ||
+                (awaited == best_awaited &&
+                 (votes[k] > votes[best] || (votes[k] == votes[best] && least[k] < least[best]))))
+            {
+                best = k;
+                best_awaited = awaited;
+            }
         }
         const auto key = keys[best];
         PlanOp p;
@@ -214,7 +251,7 @@ static int batch_plan(snb_batch* b)
         {
             if (cur[m] >= b->rec[m].ops.size()) continue;
             const SnbRecOp& o = b->rec[m].ops[cur[m]];
-            if (std::make_tuple(o.bfn, o.block, o.lane) != key) continue;
+            if (key_of(o) != key) continue;
             take.push_back(m);
         }
         std::stable_sort(take.begin(), take.end(), [&](int x, int y) {
@@ -224,6 +261,7 @@ static int batch_plan(snb_batch* b)
         {
             const SnbRecOp& o = b->rec[m].ops[cur[m]];
             cur[m]++;
+            done[m][key]++;
             if (o.grid == 0) continue;
             if (p.nseg == 0)
                 p.stride = (int)o.args.size();

@@ -78,6 +78,30 @@ def test_step_batch_matches_each_system_alone():
         nb.close()
 
 
+def test_members_of_both_pair_paths_share_dispatches():
+    """Members whose sequences differ by the pair kernels (one launch without
+    windows, two with) keep one dispatch for every other kernel: the launches
+    of the windowed member and the other's own pair and list kernels."""
+    from sponge_amd.lib import StepBatch
+    plain, windowed = _member(1600, 21), _member(5200, 22)
+    assert plain[0].set_window_shape(0, 0, 0) and windowed[0].set_window_shape(2, 2, 2)
+    for nb, st in (plain, windowed):
+        nb.nl_update(forced=True)         # a new path starts with a rebuild of its own
+        nb.sync()
+    launches = []
+    for members in ([plain], [windowed], [plain, windowed], [windowed, plain]):
+        b = StepBatch()
+        for nb, st in members:
+            b.record(nb, CHUNK, CHUNK)
+        launches.append(b.plan()[0])
+        b.close()
+    print("launches", launches, flush=True)
+    # one k_lj_full a step, one k_nl_search a rebuild
+    assert launches[2] == launches[3] == launches[1] + CHUNK + 1
+    for nb, st in (plain, windowed):
+        nb.close()
+
+
 def test_step_batch_rejects_second_stream_and_double_record():
     from sponge_amd.lib import SnbError, StepBatch
     nb, st = _member(1600, 11, overlap=True)
