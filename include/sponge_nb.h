@@ -75,7 +75,7 @@ int snb_context_destroy(snb_context* ctx);
 int snb_set_stream(snb_context* ctx, void* hip_stream);
 /* Runs the PME reciprocal pipeline on a second, library-owned stream beside
  * the direct-space work (default 1; systems of up to 8,192 atoms without
- * windows keep to one stream).  It starts once the step's coordinates
+ * windows keep to one stream with the default snb_lj_set_row_lds).  It starts once the step's coordinates
  * are final -- at the last snb_nl_update, or at the reciprocal call when no
  * update came since the previous one -- and every later call that reads its
  * results (force flush, copies, energies, status) waits for it on the

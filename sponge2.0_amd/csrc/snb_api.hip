@@ -421,7 +421,7 @@ int snb_join_pme(snb_context* c)
 }
 
 // Where the stream of the reciprocal pipeline may change (overlap switched, a
-// list of another path): what it has queued comes first,
+// list of another path, another row kernel): what it has queued comes first,
 // and the next call that takes a stream of its own records its inputs anew.  An
 // event kept from before would let it start ahead of the work queued since.
 static int leave_pme_stream(snb_context* c)
@@ -1102,6 +1102,10 @@ int snb_lj_set_row_lds(snb_context* c, int mode)
 {
     if (!c) return SNB_ERR_ARGUMENT;
     if (mode < -1 || mode > 1) return SNB_ERR_ARGUMENT;
+    if (mode == c->lj.row_lds) return SNB_OK;
+    DeviceGuard g(c->device);
+    const int rc = leave_pme_stream(c);
+    if (rc) return rc;
     c->lj.row_lds = mode;
     return SNB_OK;
 }

@@ -462,10 +462,12 @@ inline void snb_cell_widths(const SnbNl& L, const SnbBox& box, float w[3])
 // than the fork and join of the second stream cost the step's launches (25
 // steps of 1,500 atoms in a graph 1431 us on one stream and 1570 on two, 2,400
 // atoms at 10 A 1501 and 1613); with windows the pair kernel is long enough
-// (9,000 atoms: 1949 and 1601).
+// (9,000 atoms: 1949 and 1601).  The other forms of the row kernel, on
+// request, are long enough too (a step of 1,500 atoms with LDS accumulators
+// 77.8 us on one stream and 60.4 on two, of 6,000 with global atomics 113 and 104).
 inline bool snb_pme_side(const snb_context* c)
 {
-    return c->overlap && (c->nl.windowed || !c->nl.lo_rows);
+    return c->overlap && (c->nl.windowed || !c->nl.lo_rows || c->lj.row_lds >= 0);
 }
 
 // A launch of a kernel without a batched form.

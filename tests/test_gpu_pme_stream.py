@@ -53,8 +53,17 @@ def _overlap(nb):
     nb.set_pme_overlap(True)
 
 
+def _row_kernel(nb):
+    _initial(nb, PLAIN)
+    nb.set_row_lds(1)
+    nb.nl_update(forced=True)
+    nb.set_row_lds(-1)
+    nb.reciprocal(step=0, frc=False)
+    nb.set_row_lds(1)
+
+
 CHANGES = {"reinitialise": _reinitialise, "reinitialise_pending": _reinitialise_pending,
-           "window_shape": _window_shape, "overlap": _overlap}
+           "window_shape": _window_shape, "overlap": _overlap, "row_kernel": _row_kernel}
 
 
 @pytest.mark.parametrize("name", sorted(CHANGES))
